@@ -349,6 +349,7 @@ struct Runtime {
     {
         V.xcd_remap = tuning[1];
         V.tiles_per_xcd = (V.node_tiles + 7) / 8;
+        V.patch_blocks_per_xcd = (V.patch_blocks + 7) / 8;
         drop_graph();
     }
     void drop_graph()
@@ -905,6 +906,93 @@ struct TileScratch {
     }
 };
 
+// One-step layouts: runs of kPatchNodes nodes that form a patch (PatchT), as
+// start nodes in ascending order, with the ring of each.  A run is a patch
+// where its nodes are an aligned cell of the Morton order of a uniform part
+// of the mesh: every node is updated by the plain formula, has four elements
+// without hanging corners, and its eight neighbours are the nodes that its
+// place in the patch says.  `taken` marks nodes that tiles need (the corners
+// by which receivers are given to tiles).
+struct PatchRuns {
+    std::vector<int> start;
+    std::vector<int> ring;      // kPatchRing per start
+};
+
+PatchRuns find_patches(const PackedHost& H, int NA, const std::vector<char>& taken)
+{
+    constexpr int N = kPatch, W = N + 2;
+    // node n's neighbour at (x, z) offset d, from its four elements; -1 where
+    // n is not plain or the elements do not agree
+    std::vector<char> plain(NA, 0);
+    auto corners = [&](int e) { return H.elem_corners[e]; };
+    const int nblk = std::max(1, std::min(256, NA / 4096 + 1)), nth = setup_threads();
+    parallel_items(nblk, nth, [&](int b) {
+        for (int n = (int)((long)NA * b / nblk); n < (int)((long)NA * (b + 1) / nblk); ++n) {
+            const int4 q = H.node_elems[n];
+            if (taken[n] || H.node_side[n] >= 0 || q.x < 0 || q.y < 0 || q.z < 0 || q.w < 0) continue;
+            const int4 a = corners(q.x), c = corners(q.y), d = corners(q.z), e = corners(q.w);
+            bool ok = c.x == d.w && a.y == e.z && a.w == c.z && d.y == e.x;
+            for (const int4& k : {a, c, d, e}) ok = ok && std::max(std::max(k.x, k.y), std::max(k.z, k.w)) < NA;
+            plain[n] = ok;
+        }
+    });
+    int xof[kPatchNodes], zof[kPatchNodes];
+    for (int m = 0; m < kPatchNodes; ++m) {
+        xof[m] = zof[m] = 0;
+        for (int b = 0; (1 << (2 * b)) < kPatchNodes; ++b) {
+            zof[m] |= ((m >> (2 * b)) & 1) << b;
+            xof[m] |= ((m >> (2 * b + 1)) & 1) << b;
+        }
+    }
+    // fills the (N + 2)^2 image of the patch at s; false where it is none
+    auto image = [&](int s, int* img) {
+        std::fill(img, img + W * W, -1);
+        for (int m = 0; m < kPatchNodes; ++m) img[(xof[m] + 1) * W + zof[m] + 1] = s + m;
+        for (int m = 0; m < kPatchNodes; ++m) {
+            const int n = s + m;
+            if (!plain[n]) return false;
+            const int4 q = H.node_elems[n];
+            const int4 a = corners(q.x), c = corners(q.y), d = corners(q.z), e = corners(q.w);
+            const int nb[8][3] = {{1, 0, a.y}, {1, 1, a.z}, {0, 1, a.w}, {-1, 0, c.x},
+                                  {-1, 1, c.w}, {-1, -1, d.x}, {0, -1, d.y}, {1, -1, e.y}};
+            for (const auto& k : nb) {
+                int& at = img[(xof[m] + 1 + k[0]) * W + zof[m] + 1 + k[1]];
+                if (at < 0) at = k[2];
+                if (at != k[2]) return false;
+            }
+        }
+        return true;
+    };
+    std::vector<char> is(NA, 0);
+    parallel_items(nblk, nth, [&](int b) {
+        int img[W * W];
+        const int lo = (int)((long)NA * b / nblk), hi = (int)((long)NA * (b + 1) / nblk);
+        for (int s = lo; s < hi; ++s)
+            if (s + kPatchNodes <= NA && plain[s] && plain[s + kPatchNodes - 1]) is[s] = image(s, img);
+    });
+    PatchRuns out;
+    for (int s = 0; s < NA; ++s)
+        if (is[s]) {
+            out.start.push_back(s);
+            s += kPatchNodes - 1;
+        }
+    const int np = (int)out.start.size();
+    out.ring.resize((size_t)np * kPatchRing);
+    parallel_items(std::max(1, std::min(np, nblk)), nth, [&](int b) {
+        const int nb = std::max(1, std::min(np, nblk));
+        int img[W * W];
+        for (int i = (int)((long)np * b / nb); i < (int)((long)np * (b + 1) / nb); ++i) {
+            image(out.start[i], img);
+            int* r = &out.ring[(size_t)i * kPatchRing];
+            for (int z = 0; z <= N; ++z) *r++ = img[z];                       // x = -1
+            for (int x = 1; x <= N; ++x) *r++ = img[x * W];                   // z = -1
+            for (int x = 0; x <= N; ++x) *r++ = img[x * W + N + 1];           // z = N
+            for (int z = 0; z <= N + 1; ++z) *r++ = img[(N + 1) * W + z];     // x = N
+        }
+    });
+    return out;
+}
+
 void build_tiles(Runtime& R)
 {
     PhaseTimer pt("tiles");
@@ -916,7 +1004,7 @@ void build_tiles(Runtime& R)
     R.tiles_depth = 0;
     const int NA = V.na, NV = V.nv;
     const int B = R.tuning[0], K = R.tuning[3];
-    const int ntiles = (NA + B - 1) / B;
+    int ntiles = (NA + B - 1) / B;
     const int NR = (int)H.recv.size();
     const int NFF = (int)H.ff.size();
     const int NM = (int)(H.lm.size() / 2);
@@ -933,8 +1021,28 @@ void build_tiles(Runtime& R)
     int ncu = 0;
     if (hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, R.device) != hipSuccess || ncu < 1)
         ncu = 256;
-    std::vector<int> tstart(ntiles + 1, 0);
-    if (K == 1 || ntiles > 2 * ncu) {
+    std::vector<int> tstart(ntiles + 1, 0), tend;
+    // one step per launch: uniform parts of the mesh as patches, the runs of
+    // nodes between them as tiles of at most B nodes
+    PatchRuns patches;
+    if (K == 1) {
+        std::vector<char> taken(NA, 0);
+        for (const RecvRec& x : H.recv) {
+            const int c = x.c[0];
+            if (c >= 0) taken[c < NA ? c : H.vanch[c - NA].x] = 1;
+        }
+        patches = find_patches(H, NA, taken);
+        const int np = (int)patches.start.size();
+        tstart.clear();
+        for (int i = 0; i <= np; ++i) {
+            const int lo = i ? patches.start[i - 1] + kPatchNodes : 0, hi = i < np ? patches.start[i] : NA;
+            for (int n = lo; n < hi; n += B) {
+                tstart.push_back(n);
+                tend.push_back(std::min(n + B, hi));
+            }
+        }
+        ntiles = (int)tstart.size();
+    } else if (ntiles > 2 * ncu) {
         for (int t = 1; t <= ntiles; ++t) tstart[t] = std::min(t * B, NA);
     } else {
         std::vector<double> cum(NA + 1, 0.0);
@@ -952,6 +1060,8 @@ void build_tiles(Runtime& R)
         }
         tstart[ntiles] = NA;
     }
+    if (K > 1) tend.assign(tstart.begin() + 1, tstart.end());
+    tstart.resize(ntiles);
     auto tile_of = [&](int node) {
         return (int)(std::upper_bound(tstart.begin(), tstart.end(), node) - tstart.begin()) - 1;
     };
@@ -969,7 +1079,7 @@ void build_tiles(Runtime& R)
 
     // one tile into part P (offsets local to P)
     auto build_one = [&](int t, TileScratch& S, TilePart& P) {
-        const int n0 = tstart[t], cnt = tstart[t + 1] - tstart[t];
+        const int n0 = tstart[t], cnt = tend[t] - tstart[t];
         std::vector<int>& ent = S.ent;
         std::vector<int>& vl = S.vl;
         std::vector<int>& vlist = S.vlist;
@@ -1411,7 +1521,6 @@ void build_tiles(Runtime& R)
         }
     }
     V.has_elem = has_elem ? 1 : 0;
-    V.block = B;
     V.threads = std::max(64, (max_ent + 63) / 64 * 64);
     V.depth = K;
     V.node_tiles = ntiles;
@@ -1434,10 +1543,8 @@ void build_tiles(Runtime& R)
         auto check_tile = [&](int t) {
             const TileInfo& T = tiles[t];
             const int cnt = T.cnt;
-            if (T.n0 != tstart[t] || cnt < 1 || T.n0 + cnt != tstart[t + 1]) throw bad(t, "core range");
-            // the one-step kernel derives the core range from the tile index
-            if (K == 1 && (T.n0 != t * B || cnt != std::min(B, NA - t * B) || cnt > V.threads))
-                throw bad(t, "one-step core range");
+            if (T.n0 != tstart[t] || cnt < 1 || T.n0 + cnt != tend[t] || tend[t] > NA || cnt > V.threads)
+                throw bad(t, "core range");
             const int nslots = T.n_ent + T.n_virt;
             if (T.n_ent < cnt || T.lev_end[K - 1] > V.threads || nslots > V.lds_slots || nslots > kMaxSlots)
                 throw bad(t, "entries");
@@ -1531,6 +1638,40 @@ void build_tiles(Runtime& R)
             for (int t = t0; t < t1; ++t) check_tile(t);
         });
     }
+    // patches: uniform moduli and mass term in the record where they are
+    // uniform, else read per node
+    V.patches = (int)patches.start.size();
+    V.patch_hetero = 0;
+    V.patch_blocks = (V.patches + V.threads / 64 - 1) / (V.threads / 64);
+    std::vector<PatchT> patch(V.patches);
+    {
+        const int nblk = std::max(1, std::min(V.patches, 16 * setup_threads()));
+        parallel_items(nblk, setup_threads(), [&](int b) {
+            for (int i = (int)((long)V.patches * b / nblk); i < (int)((long)V.patches * (b + 1) / nblk); ++i) {
+                PatchT& P = patch[i];
+                P = PatchT{};
+                P.n0 = patches.start[i];
+                if (P.n0 < 0 || P.n0 + kPatchNodes > NA) throw fail(DMP_EINVAL, "internal: patch %d out of range", i);
+                const int* ring = &patches.ring[(size_t)i * kPatchRing];
+                P.lam = H.node_em[2 * (size_t)P.n0];
+                P.mu = H.node_em[2 * (size_t)P.n0 + 1];
+                P.invm = H.invm[P.n0];
+                auto same = [&](int n) {
+                    if (H.node_em[2 * (size_t)n] != P.lam || H.node_em[2 * (size_t)n + 1] != P.mu) P.hetero = 1;
+                };
+                for (int m = 0; m < kPatchNodes; ++m) {
+                    same(P.n0 + m);
+                    if (H.invm[P.n0 + m] != P.invm) P.coefs = 1;
+                    core_coef[P.n0 + m] = H.invm[P.n0 + m];
+                }
+                for (int r = 0; r < kPatchRing; ++r) {
+                    if (ring[r] < 0 || ring[r] >= NA) throw fail(DMP_EINVAL, "internal: patch %d: ring node out of range", i);
+                    if (r < kPatchLow) same(ring[r]);
+                }
+            }
+        });
+        for (const PatchT& P : patch) V.patch_hetero |= P.hetero;
+    }
     const size_t lds = step_lds_bytes(V, R.precision);
     if (std::getenv("DMP_LAYOUT_STATS")) {
         double ent = 0, ring = 0;
@@ -1550,12 +1691,14 @@ void build_tiles(Runtime& R)
         for (int h : hist) std::fprintf(stderr, "%d,", h);
         int with_vrow = 0;
         for (const TileInfo& T : tiles) with_vrow += T.n_vrow > 0;
-        std::fprintf(stderr, " tiles with hanging-node rows %d\n", with_vrow);
+        std::fprintf(stderr, " tiles with hanging-node rows %d, patches %d\n", with_vrow, V.patches);
     }
     if (lds > R.lds_limit)
         throw fail(DMP_EUNSUPPORTED, "tiles of %d nodes for %d steps per launch need %zu B of LDS "
                    "(limit %zu)", B, K, lds, R.lds_limit);
     V.tiles = R.upload_tile(tiles);
+    V.patch = R.upload_tile(patch);
+    V.patch_ring = R.upload_tile(patches.ring);
     V.core_desc = R.upload_tile(core_desc);
     V.ring_gid = R.upload_tile(ring_gid);
     V.elist = nullptr;

@@ -110,6 +110,35 @@ struct TileInfo {
     int pad[3];
 };
 
+// One-step layouts: a patch of kPatch x kPatch nodes of a uniform part of the
+// mesh, one wavefront's work.  Its nodes are an aligned cell of the Morton
+// order, n0 + m for the node whose x and z bits interleave to m (z in the even
+// bits); each has four elements, none with a hanging corner, and needs the
+// plain update only (no side record), and the tile samples no receiver.  The
+// neighbours of a node then sit at fixed distances from it in the patch and no
+// descriptor is needed.
+constexpr int kPatch = 8;
+constexpr int kPatchNodes = kPatch * kPatch;
+constexpr int kPatchRing = 4 * kPatch + 4;
+// LDS image of a patch and its ring: x (the slow index) and z from -1 to
+// kPatch.  Eight lanes of a 16-byte access cover two x and four z, so a pitch
+// of 4 mod 8 puts them on different banks.
+constexpr int kPatchPitch = 12;
+constexpr int kPatchSlots = (kPatch + 2) * kPatchPitch;
+// Ring order: x = -1 and then z = -1 (the corners 0 of the elements at the
+// patch's lower x and z sides, whose moduli are read), then the rest.
+constexpr int kPatchLow = 2 * kPatch + 1;
+
+struct PatchT {
+    int n0;
+    int hetero;          // 1: (lambda, mu) per element from node_em, 0: lam, mu
+    int coefs;           // 1: 1 / e_mfull per node from core_coef, 0: invm
+    int pad;
+    double lam, mu, invm;
+    double pad2;
+};
+static_assert(sizeof(PatchT) == 48, "patch records are read as whole 16-byte words");
+
 // Node whose update needs more than the plain interior formula: absorbing
 // dashpots, hanging-node anchors, plane-wave forces or a point source.
 // word: bits 0-2 transfer count, 3-4 point kind (1 force, 2 prescribed z),
@@ -186,10 +215,9 @@ struct Ctrl {
 struct DevView {
     int na, nv, ne;
     int nrecv;
-    int block;           // core nodes per tile on average (tiles are cut at equal work)
     int threads;         // threads per workgroup (one LDS entry each)
     int depth;           // rings per tile = most steps one launch may take
-    int node_tiles;      // ceil(na / block)
+    int node_tiles;
     int xcd_remap;       // 1: consecutive tiles stay on one XCD
     int tiles_per_xcd;
     int has_elem;        // some tile reads (lambda, mu) per slot (mat_mode 1)
@@ -231,6 +259,13 @@ struct DevView {
     const RecvG* rg;          // receivers in global node ids
     void* U[kStateSlots];     // u_j in U[j mod kStateSlots], 16 B per active node
     Ctrl* ctrl;
+    // one-step layouts: patches, beside the tiles
+    int patches;
+    int patch_hetero;    // some patch reads (lambda, mu) per element
+    int patch_blocks;    // workgroups of threads / 64 patches
+    int patch_blocks_per_xcd;
+    const PatchT* patch;
+    const int* patch_ring;    // [patches][kPatchRing] nodes around each
 };
 
 } // namespace dmp

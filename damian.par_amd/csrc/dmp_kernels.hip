@@ -129,7 +129,7 @@ struct PF64 {
     // u_{i} = 2 u_{i-1} - u_{i-2} + corr
     __device__ static node_t advance(node_t u, node_t up, V2<real> c)
     {
-        return make_double2((2.0 * u.x - up.x) + c.x, (2.0 * u.y - up.y) + c.y);
+        return make_double2(fma(2.0, u.x, -up.x) + c.x, fma(2.0, u.y, -up.y) + c.y);
     }
 };
 
@@ -163,9 +163,10 @@ struct PF32C {
     }
     __device__ static void adv1(float uh, float ul, float ph, float pl, float c, float& rh, float& rl)
     {
-        float s, e;
-        two_sum(2.0f * uh, -ph, s, e);             // 2*uh exact
-        const float lo = ((2.0f * ul - pl) + e) + c;
+        // two_sum(2 uh, -ph); 2 uh is exact, so its products are fused
+        const float s = fma(2.0f, uh, -ph), bb = fma(-2.0f, uh, s);
+        const float e = fma(2.0f, uh, -(s - bb)) + (-ph - bb);
+        const float lo = (fma(2.0f, ul, -pl) + e) + c;
         two_sum(s, lo, rh, rl);
     }
     __device__ static node_t advance(node_t u, node_t up, V2<real> c)
@@ -197,6 +198,27 @@ __device__ __forceinline__ float4 avg2(float4 a, float4 b)
     return r;
 }
 
+// The increment: forces over mass, rounded before it is added to the state (in
+// every kernel, so that they give the same bits).
+template <class R>
+__device__ __forceinline__ V2<R> over_mass(V2<R> f, R inv0, R inv1)
+{
+#pragma clang fp contract(off)
+    return {f.x * inv0, f.y * inv1};
+}
+
+// f -= m a + n b, the product m a rounded and n b fused, written out so that
+// every kernel gives the same bits (left to the compiler, the choice depends
+// on the code around it).
+template <class R>
+__device__ __forceinline__ void sub_rows(R m, V2<R> a, R n, V2<R> b, V2<R>& f)
+{
+#pragma clang fp contract(off)
+    const R x = m * a.x, z = m * a.y;
+    f.x -= fma(n, b.x, x);
+    f.y -= fma(n, b.y, z);
+}
+
 // f -= rows (2K, 2K+1) of K_e (lam, mu) applied to u_j - uref over the three
 // other corners of the element, whose LDS slots are packed in w.
 template <class P, int K>
@@ -219,8 +241,7 @@ __device__ __forceinline__ void slot_rows(const typename P::node_t* val, uint32_
         zl = fma(R(KL(2 * K + 1, 2 * j + 1)), d.y, fma(R(KL(2 * K + 1, 2 * j)), d.x, zl));
         zm = fma(R(KM(2 * K + 1, 2 * j + 1)), d.y, fma(R(KM(2 * K + 1, 2 * j)), d.x, zm));
     }
-    f.x -= lm.x * xl + lm.y * xm;
-    f.y -= lm.x * zl + lm.y * zm;
+    sub_rows<R>(lm.x, {xl, zl}, lm.y, {xm, zm}, f);
 }
 
 // slot_rows on corner values already in registers (c[q] = value of the q-th
@@ -243,8 +264,7 @@ __device__ __forceinline__ void slot_rows_v(const typename P::node_t (&c)[3], V2
         zl = fma(R(KL(2 * K + 1, 2 * j + 1)), d.y, fma(R(KL(2 * K + 1, 2 * j)), d.x, zl));
         zm = fma(R(KM(2 * K + 1, 2 * j + 1)), d.y, fma(R(KM(2 * K + 1, 2 * j)), d.x, zm));
     }
-    f.x -= lm.x * xl + lm.y * xm;
-    f.y -= lm.x * zl + lm.y * zm;
+    sub_rows<R>(lm.x, {xl, zl}, lm.y, {xm, zm}, f);
 }
 
 // Element rows of one node (or hanging node) from its descriptor: per
@@ -353,8 +373,7 @@ struct Rows {
         const V2<R> lm = elem ? em[ms] : lmt[(wk >> 30) & 3];
         const R xl = row<0, 0>(q, dx, dz, dd), xm = row<1, 0>(q, dx, dz, dd);
         const R zl = row<0, 1>(q, dx, dz, dd), zm = row<1, 1>(q, dx, dz, dd);
-        f.x -= lm.x * xl + lm.y * xm;
-        f.y -= lm.x * zl + lm.y * zm;
+        sub_rows<R>(lm.y, {xm, zm}, lm.x, {xl, zl}, f);
     }
     // A hanging node's row, one half per lane of a pair: side 0 takes
     // quadrants 0 and 2, side 1 quadrants 1 and 3, so that the node's two
@@ -611,6 +630,108 @@ __device__ __forceinline__ void load_entries(const DevView& V, int tile, const v
     }
 }
 
+// LDS of one patch: values, and moduli per element where a patch needs them.
+__host__ __device__ inline int patch_lds_bytes(const DevView& V, int real_bytes)
+{
+    return kPatchSlots * (16 + (V.patch_hetero ? 2 * real_bytes : 0));
+}
+
+// ---------------------------------------------------------------------------
+// One step of a patch (PatchT) by one wavefront.
+//
+// Bound by memory: 48 B per node and step have to move (two levels read, one
+// written), and the vector instructions (about 200 per node in FP32C, 145 in
+// FP64) take two thirds of that time, overlapped between the wavefronts of a
+// SIMD.  A tile reads 20 to 24 B more per node (descriptor, mass term) and
+// spends some 100 more instructions on decoding descriptors and on the 12
+// corner reads that are 8 here, all at fixed offsets from one LDS address; and
+// a wavefront on its own needs no barrier.  The uniform 944,492-element canyon
+// takes 10.9 us a step in FP32C (4.2 TB/s of those 48 B) against 16.0 with
+// tiles only, and 12.0 against 17.2 in FP64.
+// ---------------------------------------------------------------------------
+// Ring position r (kPatchRing of them) in the patch's LDS image.
+__device__ __forceinline__ int patch_ring_slot(int r)
+{
+    constexpr int N = kPatch, W = kPatchPitch;
+    if (r <= N) return r;                                    // x = -1, z = -1 .. N-1
+    if (r < kPatchLow) return (r - N) * W;                   // z = -1, x = 0 .. N-1
+    if (r < kPatchLow + N + 1) return (r - kPatchLow) * W + N + 1;   // z = N, x = -1 .. N-1
+    return (N + 1) * W + (r - kPatchLow - N - 1);            // x = N, z = -1 .. N
+}
+
+template <class P>
+__device__ __forceinline__ void patch_step(const DevView& V, int t, const void* U0, const void* Um, void* Uk,
+                                           unsigned char* lds)
+{
+    using R = typename P::real;
+    using node_t = typename P::node_t;
+    constexpr int Q = kPatchNodes / 64, W = kPatchPitch;
+    const int lane = (int)threadIdx.x & 63;
+    node_t* val = reinterpret_cast<node_t*>(lds);
+    V2<R>* em = reinterpret_cast<V2<R>*>(val + kPatchSlots);
+    const PatchT T = V.patch[t];
+    const int* ring = V.patch_ring + (size_t)t * kPatchRing;
+    const int g0 = lane < kPatchRing ? ring[lane] : T.n0;
+    int g1 = 0;
+    if (lane < kPatchRing - 64) g1 = ring[64 + lane];
+    // node m = 64 q + lane: the lane's six bits are its place in an 8 x 8
+    // block, q the block (bit 0: z, bit 1: x)
+    const int x = ((lane >> 1) & 1) | ((lane >> 2) & 2) | ((lane >> 3) & 4);
+    const int z = (lane & 1) | ((lane >> 1) & 2) | ((lane >> 2) & 4);
+    const int at = (x + 1) * W + z + 1;
+    node_t u[Q], p[Q];
+#pragma unroll
+    for (int q = 0; q < Q; ++q) u[q] = P::ld(U0, T.n0 + 64 * q + lane);
+#pragma unroll
+    for (int q = 0; q < Q; ++q) p[q] = P::ld(Um, T.n0 + 64 * q + lane);
+    const node_t r0 = P::ld(U0, g0);
+    node_t r1{};
+    if (lane < kPatchRing - 64) r1 = P::ld(U0, g1);
+    if (T.hetero) {
+        V2<R> e[Q];
+#pragma unroll
+        for (int q = 0; q < Q; ++q) e[q] = P::lm(V.node_em, T.n0 + 64 * q + lane);
+        V2<R> er{0, 0};
+        if (lane < kPatchLow) er = P::lm(V.node_em, g0);
+#pragma unroll
+        for (int q = 0; q < Q; ++q) em[at + (q >> 1) * 8 * W + (q & 1) * 8] = e[q];
+        if (lane < kPatchLow) em[patch_ring_slot(lane)] = er;
+    }
+#pragma unroll
+    for (int q = 0; q < Q; ++q) val[at + (q >> 1) * 8 * W + (q & 1) * 8] = u[q];
+    if (lane < kPatchRing) val[patch_ring_slot(lane)] = r0;
+    if (lane < kPatchRing - 64) val[patch_ring_slot(64 + lane)] = r1;
+    // the wavefront reads what its own lanes wrote: LDS operations of a
+    // wavefront complete in order, so only the compiler has to keep them so
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+#pragma unroll
+    for (int q = 0; q < Q; ++q) {
+        const node_t* c = val + at + (q >> 1) * 8 * W + (q & 1) * 8;
+        const V2<R>* m = em + at + (q >> 1) * 8 * W + (q & 1) * 8;
+        const node_t un = c[0];
+        const node_t xm = c[-W], xp = c[W], zm = c[-1], zp = c[1];
+        const node_t mm = c[-W - 1], mp = c[-W + 1], pm = c[W - 1], pp = c[W + 1];
+        V2<R> l0{R(T.lam), R(T.mu)}, l1 = l0, l2 = l0, l3 = l0;
+        if (T.hetero) {
+            l0 = m[0];
+            l1 = m[-W];
+            l2 = m[-W - 1];
+            l3 = m[-1];
+        }
+        // the element of which the node is corner 0, 1, 2, 3, as Rows::apply
+        V2<R> f{0, 0};
+        const node_t c0[3] = {xp, pp, zp}, c1[3] = {xm, zp, mp}, c2[3] = {mm, zm, xm}, c3[3] = {zm, pm, xp};
+        slot_rows_v<P, 0>(c0, l0, un, f);
+        slot_rows_v<P, 1>(c1, l1, un, f);
+        slot_rows_v<P, 2>(c2, l2, un, f);
+        slot_rows_v<P, 3>(c3, l3, un, f);
+        const R cf = T.coefs ? P::coef(V.core_coef, T.n0 + 64 * q + lane) : R(T.invm);
+        P::st(Uk, T.n0 + 64 * q + lane, P::advance(un, p[q], over_mass(f, cf, cf)));
+    }
+}
+
 // ONE: the layout has depth 1 (one step per launch): two LDS buffers, no
 // rotation, side records read straight into registers.
 template <class P, bool ONE>
@@ -623,11 +744,7 @@ __device__ void tile_steps(const DevView& V, int tile, int t0, int k, int end)
     const int NT = blockDim.x;
     const int tid = threadIdx.x;
     const TileInfo T = V.tiles[tile];
-    // one-step layouts cut tiles of exactly `block` nodes (the last one
-    // shorter): the core range follows from the tile index, so the core loads
-    // need not wait for the tile record
-    const int n0 = ONE ? tile * V.block : T.n0;
-    const int cnt = ONE ? min(V.block, V.na - n0) : T.cnt;
+    const int n0 = T.n0, cnt = T.cnt;
     const int S = V.lds_slots;
     const int D = ONE ? 1 : V.depth;
 
@@ -871,7 +988,7 @@ __device__ void tile_steps(const DevView& V, int tile, int t0, int k, int end)
             int point = 0;
             double pz = 0.0;
             if (!side) {
-                corr = {f.x * cf, f.y * cf};                                   // interior node
+                corr = over_mass(f, cf, cf);                                   // interior node
             } else {
                 // the record as scalars (a dynamic index into it would put it
                 // on the scratch stack)
@@ -923,7 +1040,7 @@ __device__ void tile_steps(const DevView& V, int tile, int t0, int k, int end)
                     f.x += h.x;
                     f.y += h.y;
                 }
-                corr = {f.x * R(invm0), f.y * R(invm1)};
+                corr = over_mass(f, R(invm0), R(invm1));
             }
             node_t unew = P::advance(un, upn, corr);
             if (point == 2) unew = set_z(unew, pz);
@@ -965,7 +1082,22 @@ __global__ __launch_bounds__(kMaxThreads) __attribute__((amdgpu_waves_per_eu(ONE
 void step_kernel(DevView V, int t0_arg, int use_base, int k, int end)
 {
     const int t0 = t0_arg + (use_base ? V.ctrl->base : 0);
-    const int b = blockIdx.x;
+    int b = blockIdx.x;
+    if (ONE) {
+        // tiles first (the longer work), then the patches
+        const int nb = V.xcd_remap ? 8 * V.tiles_per_xcd : V.node_tiles;
+        if (b >= nb) {
+            b -= nb;
+            const int blk = V.xcd_remap ? (b & 7) * V.patch_blocks_per_xcd + (b >> 3) : b;
+            const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+            const int t = blk * ((int)blockDim.x >> 6) + wave;
+            if (blk >= V.patch_blocks || t >= V.patches || k < 1) return;
+            extern __shared__ __align__(16) unsigned char smem[];
+            patch_step<P>(V, t, V.U[t0 % kStateSlots], V.U[(t0 + kStateSlots - 1) % kStateSlots],
+                          V.U[(t0 + k) % kStateSlots], smem + wave * patch_lds_bytes(V, sizeof(typename P::real)));
+            return;
+        }
+    }
     const int tile = V.xcd_remap ? (b & 7) * V.tiles_per_xcd + (b >> 3) : b;
     if (tile >= V.node_tiles) return;   // whole block exits together
     tile_steps<P, ONE>(V, tile, t0, k, end);
@@ -1086,18 +1218,19 @@ hipError_t scratch_address(int device, double** out)
 static int node_grid(const DevView& V)
 {
     if (V.na == 0) return 0;
-    return V.xcd_remap ? 8 * V.tiles_per_xcd : V.node_tiles;
+    return V.xcd_remap ? 8 * (V.tiles_per_xcd + V.patch_blocks_per_xcd) : V.node_tiles + V.patch_blocks;
 }
 
 size_t step_lds_bytes(const DevView& V, int precision)
 {
     const size_t rb = precision == 0 ? sizeof(double) : sizeof(float);
-    return (size_t)(V.depth > 1 ? 3 : 2) * V.lds_slots * 16 +
+    const size_t patches = V.patches ? (size_t)(V.threads / 64) * patch_lds_bytes(V, (int)rb) : 0;
+    return std::max(patches, (size_t)(V.depth > 1 ? 3 : 2) * V.lds_slots * 16 +
            (size_t)V.depth * V.lds_force * sizeof(double2) +
            (size_t)V.depth * V.lds_recv * sizeof(double2) +
            (size_t)V.lds_side * sizeof(SideT) + (size_t)V.lds_recv * sizeof(RecvT) +
            (size_t)V.lds_mat * 2 * rb + (size_t)V.lds_vrows * 4 * rb +
-           (size_t)V.lds_virt * sizeof(int2) + (V.has_elem ? (size_t)V.lds_slots * 2 * rb : 0);
+           (size_t)V.lds_virt * sizeof(int2) + (V.has_elem ? (size_t)V.lds_slots * 2 * rb : 0));
 }
 
 template <class P>

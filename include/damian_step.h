@@ -161,7 +161,8 @@ int dmp_export_mesh(void *h, int *eptr, int *eind, bool *ediv, int *hanging, int
 /* Launch parameters (4 ints).  tuning[0] = nodes per tile on average (32..1024;
  * each workgroup owns one of ceil(nodes / tuning[0]) tiles; with several steps
  * per launch and at most two tiles per compute unit the tiles are cut at equal
- * work, so tiles holding hanging-node anchors are smaller), tuning[1] = XCD-aware tile remap (0/1), tuning[2] = steps
+ * work, so tiles holding hanging-node anchors are smaller; with one step per
+ * launch 8 x 8 patches of uniform parts of the mesh are cut out first), tuning[1] = XCD-aware tile remap (0/1), tuning[2] = steps
  * per captured hipGraph (0 = eager launches), tuning[3] = time steps one
  * launch advances (1..8; each tile then carries that many rings of
  * neighbours in LDS).  dmp_init starts from {256, 1, 60, 3} ({256, 1, 60, 1}
