@@ -479,6 +479,19 @@ __device__ void drm_rows(const DrmElem& E, const double4 f[4], double& fx, doubl
 // ---------------------------------------------------------------------------
 // The step kernel.
 // ---------------------------------------------------------------------------
+// A workgroup's (or wavefront's) record at a uniform address, which nothing
+// writes during the launch, by scalar loads.
+template <class T>
+__device__ __forceinline__ T uniform_record(const T* p)
+{
+    static_assert(sizeof(T) % 4 == 0, "copied as words");
+    using Words = const __attribute__((address_space(4))) uint32_t*;
+    struct { uint32_t w[sizeof(T) / 4]; } r;
+#pragma unroll
+    for (unsigned i = 0; i < sizeof(T) / 4; ++i) r.w[i] = ((Words)(uintptr_t)p)[i];
+    return __builtin_bit_cast(T, r);
+}
+
 // Receiver samples of step j = t0 + s (visu_field, visualization.f90:156-181)
 // from the tile's values at that step; the free field is added in the
 // exterior region.
@@ -669,7 +682,7 @@ __device__ __forceinline__ void patch_step(const DevView& V, int t, const void* 
     const int lane = (int)threadIdx.x & 63;
     node_t* val = reinterpret_cast<node_t*>(lds);
     V2<R>* em = reinterpret_cast<V2<R>*>(val + kPatchSlots);
-    const PatchT T = V.patch[t];
+    const PatchT T = uniform_record(V.patch + t);
     const int* ring = V.patch_ring + (size_t)t * kPatchRing;
     const int g0 = lane < kPatchRing ? ring[lane] : T.n0;
     int g1 = 0;
@@ -713,20 +726,21 @@ __device__ __forceinline__ void patch_step(const DevView& V, int t, const void* 
         const node_t un = c[0];
         const node_t xm = c[-W], xp = c[W], zm = c[-1], zp = c[1];
         const node_t mm = c[-W - 1], mp = c[-W + 1], pm = c[W - 1], pp = c[W + 1];
-        V2<R> l0{R(T.lam), R(T.mu)}, l1 = l0, l2 = l0, l3 = l0;
-        if (T.hetero) {
-            l0 = m[0];
-            l1 = m[-W];
-            l2 = m[-W - 1];
-            l3 = m[-1];
-        }
         // the element of which the node is corner 0, 1, 2, 3, as Rows::apply
-        V2<R> f{0, 0};
         const node_t c0[3] = {xp, pp, zp}, c1[3] = {xm, zp, mp}, c2[3] = {mm, zm, xm}, c3[3] = {zm, pm, xp};
-        slot_rows_v<P, 0>(c0, l0, un, f);
-        slot_rows_v<P, 1>(c1, l1, un, f);
-        slot_rows_v<P, 2>(c2, l2, un, f);
-        slot_rows_v<P, 3>(c3, l3, un, f);
+        V2<R> f{0, 0};
+        if (T.hetero) {
+            slot_rows_v<P, 0>(c0, m[0], un, f);
+            slot_rows_v<P, 1>(c1, m[-W], un, f);
+            slot_rows_v<P, 2>(c2, m[-W - 1], un, f);
+            slot_rows_v<P, 3>(c3, m[-1], un, f);
+        } else {
+            const V2<R> lm{R(T.lam), R(T.mu)};
+            slot_rows_v<P, 0>(c0, lm, un, f);
+            slot_rows_v<P, 1>(c1, lm, un, f);
+            slot_rows_v<P, 2>(c2, lm, un, f);
+            slot_rows_v<P, 3>(c3, lm, un, f);
+        }
         const R cf = T.coefs ? P::coef(V.core_coef, T.n0 + 64 * q + lane) : R(T.invm);
         P::st(Uk, T.n0 + 64 * q + lane, P::advance(un, p[q], over_mass(f, cf, cf)));
     }
@@ -743,7 +757,7 @@ __device__ void tile_steps(const DevView& V, int tile, int t0, int k, int end)
     extern __shared__ __align__(16) unsigned char smem[];
     const int NT = blockDim.x;
     const int tid = threadIdx.x;
-    const TileInfo T = V.tiles[tile];
+    const TileInfo T = uniform_record(V.tiles + tile);
     const int n0 = T.n0, cnt = T.cnt;
     const int S = V.lds_slots;
     const int D = ONE ? 1 : V.depth;
@@ -980,7 +994,7 @@ __device__ void tile_steps(const DevView& V, int tile, int t0, int k, int end)
             if (recv_in_rows) sample_receivers<P>(V, cur, rff, rcv, n_recv, t0, s - 1, rlane);
             __syncthreads();
         }
-        if (e < lev_end(D - s)) {
+        if (e < (ONE ? cnt : lev_end(D - s))) {
             const node_t un = cur[e], upn = prv[e];
             V2<R> f = ONE ? rows.apply(cur, un, e, lmt, em, elem)
                           : rows.apply_pairs(cur, un, e, lmt, em, elem);   // -K u
