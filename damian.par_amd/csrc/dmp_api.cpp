@@ -270,6 +270,7 @@ struct Runtime {
     std::vector<int> inst_na, inst_nrecv;
     PackedHost host;
     int tiles_block = 0, tiles_depth = 0;   // shape the tile arrays were built for
+    int state_depth = kMaxDepth;   // depth whose state_slot() the state buffers are in
     std::vector<void*> tile_allocs;
     hipEvent_t ev0 = nullptr, ev1 = nullptr;
     float last_ms = 0.0f;          // device time of the last run (events on `stream`)
@@ -1757,6 +1758,27 @@ void build_tiles(Runtime& R)
     }
     V.force_slots = R.upload_tile(force_slots);
     V.recvs = R.upload_tile(recvs);
+    // the two live state levels to where launches of this depth look for them
+    // (buffers change places, nothing is copied)
+    if (state_slots(K) != state_slots(R.state_depth)) {
+        void* U[kStateSlots];
+        int from[2], to[2];
+        for (int q = 0; q < 2; ++q) {
+            from[q] = state_slot(R.step - q, R.state_depth);
+            to[q] = state_slot(R.step - q, K);
+        }
+        int next = 0;
+        for (int k = 0; k < kStateSlots; ++k) {
+            if (k == to[0] || k == to[1]) {
+                U[k] = V.U[from[k == to[0] ? 0 : 1]];
+                continue;
+            }
+            while (next == from[0] || next == from[1]) ++next;
+            U[k] = V.U[next++];
+        }
+        std::copy(U, U + kStateSlots, V.U);
+    }
+    R.state_depth = K;
     R.tiles_block = B;
     R.tiles_depth = K;
 }
@@ -2121,9 +2143,9 @@ void build_runtime(Runtime& R, const std::vector<Instance*>& insts)
         const double z0 = rk(0.0), zm = rk(-I.dt);
         for (int nd1 : I.point_nodes) {
             const int g = R.inst_node_base[q] + L.node_int[nd1 - 1];
-            for (int k : {0, kStateSlots - 1}) {
-                const double z = k == 0 ? z0 : zm;
-                char* base = static_cast<char*>(V.U[k]) + (size_t)g * 16;
+            for (int j : {0, -1}) {
+                const double z = j == 0 ? z0 : zm;
+                char* base = static_cast<char*>(V.U[state_slot(j, R.state_depth)]) + (size_t)g * 16;
                 if (R.precision == DMP_FP64) {
                     HIPCHECK(hipMemcpy(base + 8, &z, 8, hipMemcpyHostToDevice));
                 } else {
@@ -2505,7 +2527,7 @@ int run_steps_noalloc(Runtime& R, int n, double* out)
 void fetch_state(Runtime& R, int q, int nnodes, int j, double* u)
 {
     const int na = R.inst_na[q], nb = R.inst_node_base[q];
-    const void* U = R.V.U[((j % kStateSlots) + kStateSlots) % kStateSlots];
+    const void* U = R.V.U[state_slot(j, R.state_depth)];
     std::vector<double2> all(na);
     if (R.precision == DMP_FP64) {
         HIPCHECK(hipMemcpy(all.data(), static_cast<const double2*>(U) + nb, sizeof(double2) * na,
@@ -2569,7 +2591,7 @@ void check_tuning(const int* t)
 
 // Runs every candidate shape for nsteps steps from a saved state, once to
 // warm up and twice timed; keeps the shape with the shortest timed run.  The
-// state (the six state buffers, step) is restored.
+// state (both levels, step) is restored.
 void autotune(Runtime& R, int nsteps, int* out)
 {
     if (nsteps <= 0) throw fail(DMP_EINVAL, "autotune needs a positive step count");
@@ -2585,16 +2607,18 @@ void autotune(Runtime& R, int nsteps, int* out)
         }
     } scratch;
     const size_t ub = (size_t)std::max(R.V.na, 1) * 16;
-    void* save[kStateSlots];
-    for (int k = 0; k < kStateSlots; ++k) {
-        save[k] = scratch.get(ub);
-        HIPCHECK(hipMemcpyAsync(save[k], R.V.U[k], ub, hipMemcpyDeviceToDevice, R.stream));
-    }
     const int step0 = R.step;
+    void* save[2];   // u and u_prev
+    for (int q = 0; q < 2; ++q) {
+        save[q] = scratch.get(ub);
+        HIPCHECK(hipMemcpyAsync(save[q], R.V.U[state_slot(step0 - q, R.state_depth)], ub, hipMemcpyDeviceToDevice,
+                                R.stream));
+    }
     const bool fr0 = R.first_run;
     auto restore = [&]() {
-        for (int k = 0; k < kStateSlots; ++k)
-            HIPCHECK(hipMemcpyAsync(R.V.U[k], save[k], ub, hipMemcpyDeviceToDevice, R.stream));
+        for (int q = 0; q < 2; ++q)
+            HIPCHECK(hipMemcpyAsync(R.V.U[state_slot(step0 - q, R.state_depth)], save[q], ub,
+                                    hipMemcpyDeviceToDevice, R.stream));
         HIPCHECK(hipStreamSynchronize(R.stream));
         R.step = step0;
     };

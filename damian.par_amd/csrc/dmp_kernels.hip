@@ -11,7 +11,7 @@
 // P2), plane-wave forces (wave_reactions, model.f90:745-800, FP64 phase and
 // time, evaluated in the workgroup for its k steps), point sources, division
 // by e_mfull (:148); receivers are sampled every step from LDS
-// (visu_field, visualization.f90:156-181).  u_j lives in U[j mod 10]; hanging
+// (visu_field, visualization.f90:156-181).  u_j lives in U[state_slot(j)]; hanging
 // nodes are never stored, their value is the mean of their anchors
 // (model.f90:612-624).
 //
@@ -779,8 +779,8 @@ __device__ void tile_steps(const DevView& V, int tile, int t0, int k, int end)
     node_t* cur = buf;           // u_{t0+s-1}
     node_t* prv = buf + S;       // u_{t0+s-2}
     node_t* nxt = buf + 2 * S;   // u_{t0+s} (a third buffer only when D > 1)
-    const void* U0 = V.U[t0 % kStateSlots];
-    const void* Um = V.U[(t0 + kStateSlots - 1) % kStateSlots];
+    const void* U0 = V.U[state_slot(t0, ONE ? 1 : kMaxDepth)];
+    const void* Um = V.U[state_slot(t0 - 1, ONE ? 1 : kMaxDepth)];
 
     // ---- phase 0: every global load of the launch
     // material table: 4 per tile at a fixed stride (no dependence on the
@@ -923,8 +923,8 @@ __device__ void tile_steps(const DevView& V, int tile, int t0, int k, int end)
     // means (a sample takes longer than the means phase)
     const bool recv_in_rows = !ONE && T.n_vrow > 0;
 
-    void* Uk = V.U[(t0 + k) % kStateSlots];
-    void* Uk1 = V.U[(t0 + k - 1 + kStateSlots) % kStateSlots];
+    void* Uk = V.U[state_slot(t0 + k, ONE ? 1 : kMaxDepth)];
+    void* Uk1 = V.U[state_slot(t0 + k - 1, ONE ? 1 : kMaxDepth)];
     // several steps per launch: the record's words (force index, transfers) in
     // registers, so that the force and transfer reads of a sub-step do not
     // wait for the record
@@ -1107,8 +1107,7 @@ void step_kernel(DevView V, int t0_arg, int use_base, int k, int end)
             const int t = blk * ((int)blockDim.x >> 6) + wave;
             if (blk >= V.patch_blocks || t >= V.patches || k < 1) return;
             extern __shared__ __align__(16) unsigned char smem[];
-            patch_step<P>(V, t, V.U[t0 % kStateSlots], V.U[(t0 + kStateSlots - 1) % kStateSlots],
-                          V.U[(t0 + k) % kStateSlots], smem + wave * patch_lds_bytes(V, sizeof(typename P::real)));
+            patch_step<P>(V, t, V.U[state_slot(t0, 1)], V.U[state_slot(t0 - 1, 1)], V.U[state_slot(t0 + k, 1)], smem + wave * patch_lds_bytes(V, sizeof(typename P::real)));
             return;
         }
     }
@@ -1126,7 +1125,7 @@ __global__ void recv_kernel(DevView V, int j)
     const int r = (int)(blockIdx.x * blockDim.x + threadIdx.x);
     if (r >= V.nrecv) return;
     const RecvG g = V.rg[r];
-    const void* U = V.U[j % kStateSlots];
+    const void* U = V.U[state_slot(j, V.depth)];
     double fx = 0.0, fz = 0.0;
     if (g.found) {
 #pragma unroll

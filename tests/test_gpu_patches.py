@@ -47,3 +47,31 @@ def test_patches(nx, nz, het, prec):
                 assert rel_l2(got, want) <= TOL[prec]
         for got, want in zip((rec, u, up), ref):
             assert np.array_equal(got, want)
+
+
+@pytest.mark.parametrize("prec", [0, 1])
+def test_state_across_layouts(prec):
+    """Layouts of one and of several steps per launch keep the state levels in
+    rings of different length: changing the shape between calls, at every
+    residue of the step, keeps the trajectory."""
+    from damian_hip import cases, lib
+    case = cases.f2()
+    ref = lib.Solver(case, precision=prec)
+    r0 = ref.run(120)
+    u0, up0, _ = ref.state()
+    ref.close()
+    s = lib.Solver(case, precision=prec)
+    parts, n, k = [], 0, 0
+    while n < 120:
+        s.set_tuning(*((64, 0, 0, 1), (128, 1, 0, 3), (256, 1, 12, 1), (64, 1, 0, 2))[k % 4])
+        m = min(120 - n, 1 + k % 7)
+        parts.append(s.run(m))
+        n, k = n + m, k + 1
+    u, up, _ = s.state()
+    t = s.autotune(5)   # leaves the state where it was
+    assert len(t) == 4
+    u1, up1, _ = s.state()
+    s.close()
+    assert np.array_equal(np.concatenate(parts), r0)
+    for a, b in ((u, u0), (up, up0), (u1, u0), (up1, up0)):
+        assert np.array_equal(a, b)
