@@ -33,6 +33,8 @@ hipError_t launch_step(const DevView& V, int precision, int t0, int use_base, in
                        int end = 0);
 hipError_t launch_recv(const DevView& V, int precision, int j, hipStream_t st);
 size_t step_lds_bytes(const DevView& V, int precision);
+hipError_t launch_state(int precision, const void* U, const int* node_int, const int2* vanch, int first, int n,
+                        int base, int vbase, double2* out, hipStream_t st);
 hipError_t launch_tables(const DevView& V, int j0, int n, hipStream_t st);
 hipError_t configure_kernels(size_t* max_lds);
 hipError_t launch_advance(Ctrl* c, int g, hipStream_t st);
@@ -56,6 +58,13 @@ constexpr double kAnchorWeight = 5.0;
 // two and kTuneMinSeconds of them, at most kTuneMaxRuns.
 constexpr int kTuneMaxRuns = 15;
 constexpr double kTuneMinSeconds = 2e-3;
+
+// State downloads: nodes per chunk (2 MiB) and chunks of pinned staging, and
+// the bytes to write that are worth one more host thread (starting one takes
+// about 20 us, copying 2 MiB into pages not yet mapped about 500).
+constexpr int kStateChunk = 1 << 17;
+constexpr int kStateChunks = 4;
+constexpr size_t kStateThreadBytes = size_t(2) << 20;
 
 const double kAngZero = (double)0.0001f;   // f_wangzero is a default-real literal (pwaves.f90:8)
 
@@ -281,9 +290,15 @@ struct Runtime {
     std::vector<hipEvent_t> free_ev;    // events not marking a pending chunk
     double* hstage = nullptr;           // pinned, hstage_cap doubles
     size_t hstage_cap = 0;
-    // node numbering of the caller (host copies, for state downloads)
-    std::vector<int> h_act_orig, h_virt_orig;
     std::vector<int> recv_missing;   // receivers in no element: sampled as zero
+    // state downloads: place of each node of the caller (instances end to
+    // end), and a ring of chunks of mapped pinned host memory
+    int* d_node_int = nullptr;
+    std::vector<size_t> inst_nodes_base;
+    double2* sstage = nullptr;
+    double2* sstage_dev = nullptr;
+    int schunk = 0;                  // nodes per chunk
+    hipEvent_t sev[kStateChunks] = {};
     int* d_act_orig = nullptr;
     int* d_virt_orig = nullptr;
     int* d_elem_orig = nullptr;
@@ -316,6 +331,12 @@ struct Runtime {
         if (hstage) (void)hipHostFree(hstage);
         hstage = nullptr;
         hstage_cap = 0;
+        if (sstage) (void)hipHostFree(sstage);
+        sstage = nullptr;
+        for (hipEvent_t& e : sev) {
+            if (e) (void)hipEventDestroy(e);
+            e = nullptr;
+        }
         if (stream) (void)hipStreamDestroy(stream);
         stream = nullptr;
     }
@@ -2190,8 +2211,25 @@ void build_runtime(Runtime& R, const std::vector<Instance*>& insts)
         }
         V.rg = R.upload(rg);
     }
-    R.h_act_orig = act_orig;
-    R.h_virt_orig = virt_orig;
+    {
+        std::vector<int> node_int;
+        size_t most = 1;
+        for (Instance* I : insts) {
+            R.inst_nodes_base.push_back(node_int.size());
+            node_int.insert(node_int.end(), I->L->node_int.begin(), I->L->node_int.end());
+            most = std::max(most, I->L->node_int.size());
+        }
+        R.d_node_int = R.upload(node_int);
+        R.schunk = (int)std::min<size_t>(kStateChunk, most);
+        void* p = nullptr;
+        const size_t bytes = (size_t)kStateChunks * R.schunk * sizeof(double2);
+        const hipError_t e = hipHostMalloc(&p, bytes, hipHostMallocMapped);
+        if (e != hipSuccess) throw fail(DMP_ENOMEM, "hipHostMalloc(%zu bytes) failed: %s", bytes, hipGetErrorString(e));
+        R.sstage = static_cast<double2*>(p);
+        HIPCHECK(hipHostGetDevicePointer(&p, R.sstage, 0));
+        R.sstage_dev = static_cast<double2*>(p);
+        for (hipEvent_t& ev : R.sev) HIPCHECK(hipEventCreateWithFlags(&ev, hipEventDisableTiming));
+    }
     R.d_act_orig = R.upload(act_orig);
     R.d_virt_orig = R.upload(virt_orig);
     R.d_elem_orig = R.upload(elem_orig);
@@ -2521,39 +2559,89 @@ int run_steps_noalloc(Runtime& R, int n, double* out)
     return (int)nsamp;
 }
 
-// Active-node state of instance q at step j, in the caller's node numbering
-// (hanging nodes projected), as doubles: one device-to-host copy of the
-// instance's nodes.
-void fetch_state(Runtime& R, int q, int nnodes, int j, double* u)
+// State of instance q at the current step and the one before (either may be
+// null), in the caller's node numbering (hanging nodes projected), as doubles,
+// and beside them mfull if asked for.  The device writes the rows in the
+// caller's order into a ring of pinned chunks; host threads, as many as the
+// bytes are worth, move finished chunks into the caller's arrays (most of the
+// time of a large download is the first touch of those pages, which one
+// thread does at 4-5 GB/s) while the device fills the next.
+void fetch_states(Runtime& R, int q, int nnodes, double* u, double* up, const std::vector<double>* mfull,
+                  double* mout)
 {
-    const int na = R.inst_na[q], nb = R.inst_node_base[q];
-    const void* U = R.V.U[state_slot(j, R.state_depth)];
-    std::vector<double2> all(na);
-    if (R.precision == DMP_FP64) {
-        HIPCHECK(hipMemcpy(all.data(), static_cast<const double2*>(U) + nb, sizeof(double2) * na,
-                           hipMemcpyDeviceToHost));
-    } else {
-        std::vector<float4> f(na);
-        HIPCHECK(hipMemcpy(f.data(), static_cast<const float4*>(U) + nb, sizeof(float4) * na,
-                           hipMemcpyDeviceToHost));
-        for (int a = 0; a < na; ++a)
-            all[a] = make_double2((double)f[a].x + (double)f[a].z, (double)f[a].y + (double)f[a].w);
+    struct Piece {
+        const void* U;
+        int first, n;
+        double* dst;
+    };
+    std::vector<Piece> pieces;
+    double* const dst[2] = {u, up};
+    for (int k = 0; k < 2; ++k)
+        if (dst[k])
+            for (int f = 0; f < nnodes; f += R.schunk)
+                pieces.push_back({R.V.U[state_slot(R.step - k, R.state_depth)], f, std::min(R.schunk, nnodes - f),
+                                  dst[k] + 2 * (size_t)f});
+    const int np = (int)pieces.size();
+    const size_t mbytes = mout ? mfull->size() * sizeof(double) : 0;
+    const size_t bytes = mbytes + (size_t)((u ? 1 : 0) + (up ? 1 : 0)) * nnodes * sizeof(double2);
+    const int nthr = (int)std::max<size_t>(1, std::min<size_t>(bytes / kStateThreadBytes, setup_threads()));
+    // pieces whose rows are in the staging; -1: give up
+    std::atomic<int> ready{0};
+    std::vector<std::atomic<int>> left(np);   // threads yet to move their share of a piece
+    for (auto& l : left) l.store(nthr);
+    // thread w's share of the bytes [0, n)
+    auto share = [&](size_t n, int w) { return n / 64 * w / nthr * 64; };
+    auto move = [&](int w, int i) {
+        const Piece& p = pieces[i];
+        const size_t n = (size_t)p.n * sizeof(double2), lo = share(n, w), hi = w + 1 < nthr ? share(n, w + 1) : n;
+        std::memcpy(reinterpret_cast<char*>(p.dst) + lo,
+                    reinterpret_cast<const char*>(R.sstage + (size_t)(i % kStateChunks) * R.schunk) + lo, hi - lo);
+        left[i].fetch_sub(1, std::memory_order_release);
+    };
+    auto move_mass = [&](int w) {
+        const size_t lo = share(mbytes, w), hi = w + 1 < nthr ? share(mbytes, w + 1) : mbytes;
+        if (mbytes) std::memcpy(reinterpret_cast<char*>(mout) + lo, reinterpret_cast<const char*>(mfull->data()) + lo, hi - lo);
+    };
+    auto work = [&](int w) {
+        move_mass(w);
+        for (int i = 0; i < np; ++i) {
+            int r;
+            while ((r = ready.load(std::memory_order_acquire)) >= 0 && r <= i) std::this_thread::yield();
+            if (r < 0) return;
+            move(w, i);
+        }
+    };
+    struct Pool {
+        std::vector<std::thread> t;
+        std::atomic<int>& ready;
+        bool done = false;
+        ~Pool()
+        {
+            if (!done) ready.store(-1);
+            for (auto& x : t) x.join();
+        }
+    } pool{{}, ready};
+    auto launch = [&](int i) {
+        const Piece& p = pieces[i];
+        const int c = i % kStateChunks;
+        HIPCHECK(launch_state(R.precision, p.U, R.d_node_int + R.inst_nodes_base[q], R.d_vanch, p.first, p.n,
+                              R.inst_node_base[q], R.inst_vnode_base[q], R.sstage_dev + (size_t)c * R.schunk, R.stream));
+        HIPCHECK(hipEventRecord(R.sev[c], R.stream));
+    };
+    int launched = 0;
+    for (; launched < std::min(np, kStateChunks); ++launched) launch(launched);
+    for (int w = 1; w < nthr; ++w) pool.t.emplace_back(work, w);
+    move_mass(0);
+    for (int i = 0; i < np; ++i) {
+        wait_event(R.sev[i % kStateChunks]);
+        ready.store(i + 1, std::memory_order_release);
+        move(0, i);
+        if (launched < np) {   // the next piece takes this one's chunk
+            while (left[i].load(std::memory_order_acquire) > 0) std::this_thread::yield();
+            launch(launched++);
+        }
     }
-    std::fill(u, u + 2 * (size_t)nnodes, 0.0);
-    for (int a = 0; a < na; ++a) {
-        const int n = R.h_act_orig[nb + a];
-        u[2 * n] = all[a].x;
-        u[2 * n + 1] = all[a].y;
-    }
-    const int vb = R.inst_vnode_base[q];
-    const int nvq = (q + 1 < (int)R.inst_vnode_base.size() ? R.inst_vnode_base[q + 1] : R.V.nv) - vb;
-    for (int v = 0; v < nvq; ++v) {
-        const int2 an = R.host.vanch[vb + v];
-        const int n = R.h_virt_orig[vb + v];
-        const double2 x = all[an.x - nb], y = all[an.y - nb];
-        u[2 * n] = (x.x + y.x) / 2.0;
-        u[2 * n + 1] = (x.y + y.y) / 2.0;
-    }
+    pool.done = true;
 }
 
 template <class H> H* as(void* p) { return static_cast<H*>(p); }
@@ -2954,9 +3042,7 @@ int dmp_get_state(void* h, double* u, double* up, double* mfull)
         if (!I->rt) throw fail(DMP_ESTATE, "dmp_init must come first");
         HIPCHECK(hipSetDevice(I->device));
         Runtime& R = *I->rt;
-        if (u) fetch_state(R, 0, I->nnodes, R.step, u);
-        if (up) fetch_state(R, 0, I->nnodes, R.step - 1, up);
-        if (mfull) memcpy(mfull, I->mfull.data(), I->mfull.size() * sizeof(double));
+        fetch_states(R, 0, I->nnodes, u, up, &I->mfull, mfull);
     });
 }
 
@@ -3156,8 +3242,7 @@ int dmp_batch_get_state(void* b, const int* instance, double* u, double* up)
         HIPCHECK(hipSetDevice(B->rt->device));
         Runtime& R = *B->rt;
         const int q = *instance;
-        if (u) fetch_state(R, q, B->inst[q]->nnodes, R.step, u);
-        if (up) fetch_state(R, q, B->inst[q]->nnodes, R.step - 1, up);
+        fetch_states(R, q, B->inst[q]->nnodes, u, up, nullptr, nullptr);
     });
 }
 

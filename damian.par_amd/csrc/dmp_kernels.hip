@@ -1146,6 +1146,30 @@ __global__ void recv_kernel(DevView V, int j)
     out[1] = fz;
 }
 
+// Displacement of the nodes [first, first + n) of an instance in the caller's
+// numbering, as doubles: node_int holds a node's place in the instance's active
+// nodes (from `base` on), or -(v + 1) for its hanging node v, whose value is
+// the mean of its anchors (set_dispshanging).  One thread per node, in the
+// caller's order: the scattered accesses are the reads, in the caches behind
+// the L2s, and the rows go out to mapped host memory in whole lines.
+template <class P>
+__global__ void state_kernel(const void* U, const int* node_int, const int2* vanch, int first, int n, int base,
+                             int vbase, double2* out)
+{
+    const int i = (int)(blockIdx.x * blockDim.x + threadIdx.x);
+    if (i >= n) return;
+    const int id = node_int[first + i];
+    double2 r;
+    if (id >= 0) {
+        r = P::full(P::ld(U, base + id));
+    } else {
+        const int2 a = vanch[vbase - id - 1];
+        const double2 x = P::full(P::ld(U, a.x)), y = P::full(P::ld(U, a.y));
+        r = make_double2((x.x + y.x) / 2.0, (x.y + y.y) / 2.0);
+    }
+    out[i] = r;
+}
+
 // ---------------------------------------------------------------------------
 // Source tables.  The plane-wave and point-source terms depend on time and
 // geometry only, so they are evaluated ahead of the steps that use them, for
@@ -1278,6 +1302,17 @@ hipError_t launch_recv(const DevView& V, int precision, int j, hipStream_t st)
         hipLaunchKernelGGL(recv_kernel<PF64>, dim3(grid), dim3(256), 0, st, V, j);
     else
         hipLaunchKernelGGL(recv_kernel<PF32C>, dim3(grid), dim3(256), 0, st, V, j);
+    return hipGetLastError();
+}
+
+hipError_t launch_state(int precision, const void* U, const int* node_int, const int2* vanch, int first, int n,
+                        int base, int vbase, double2* out, hipStream_t st)
+{
+    const dim3 grid((n + 255) / 256), block(256);
+    if (precision == 0)
+        hipLaunchKernelGGL(state_kernel<PF64>, grid, block, 0, st, U, node_int, vanch, first, n, base, vbase, out);
+    else
+        hipLaunchKernelGGL(state_kernel<PF32C>, grid, block, 0, st, U, node_int, vanch, first, n, base, vbase, out);
     return hipGetLastError();
 }
 
