@@ -59,6 +59,9 @@ constexpr double kAnchorWeight = 5.0;
 constexpr int kTuneMaxRuns = 15;
 constexpr double kTuneMinSeconds = 2e-3;
 
+// Steps per launch of a mesh that one workgroup holds whole (build_tiles).
+constexpr int kWholeSteps = 32;
+
 // State downloads: nodes per chunk (2 MiB) and chunks of pinned staging, and
 // the bytes to write that are worth one more host thread (starting one takes
 // about 20 us, copying 2 MiB into pages not yet mapped about 500).
@@ -279,6 +282,10 @@ struct Runtime {
     std::vector<int> inst_na, inst_nrecv;
     PackedHost host;
     int tiles_block = 0, tiles_depth = 0;   // shape the tile arrays were built for
+    bool own_shape = true;         // the shape is dmp_init's, not one that the caller or the autotuner chose
+    bool tiles_own = true;         // own_shape when the tile arrays were built
+    bool no_whole = false;         // the mesh does not fit in one tile after all
+    bool whole = false;            // one tile holds the mesh: no rings, up to V.depth steps per launch
     int state_depth = kMaxDepth;   // depth whose state_slot() the state buffers are in
     std::vector<void*> tile_allocs;
     hipEvent_t ev0 = nullptr, ev1 = nullptr;
@@ -1025,7 +1032,17 @@ void build_tiles(Runtime& R)
     R.tiles_block = 0;   // no valid layout until this build completes
     R.tiles_depth = 0;
     const int NA = V.na, NV = V.nv;
-    const int B = R.tuning[0], K = R.tuning[3];
+    const int K = R.tuning[3];
+    // A mesh that one workgroup holds needs no rings, so a launch of several
+    // steps may take any number of them; what they read ahead (forces and free
+    // field) shares the LDS.  Where the caller asks for several steps per
+    // launch and tiles that small a mesh fits in, or has left the shape to the
+    // library, such a mesh is one tile: the two-material valley of 358 nodes
+    // takes 2.2 us a step in FP32C so, 3.8 in two tiles at three steps per
+    // launch; the layer of 861 nodes 2.1 against 3.4 in FP64, 1.8 against 3.3
+    // in FP32C.  Descriptors address no more slots.
+    R.whole = K > 1 && NA <= kMaxSlots && (R.tuning[0] >= NA || R.own_shape) && !R.no_whole;
+    const int B = R.whole ? std::max(NA, 1) : R.tuning[0];
     int ntiles = (NA + B - 1) / B;
     const int NR = (int)H.recv.size();
     const int NFF = (int)H.ff.size();
@@ -1554,6 +1571,10 @@ void build_tiles(Runtime& R)
     V.lds_recv = max_recv;
     V.lds_mat = 4;   // every tile loads its 4-entry table
     V.threads = std::max(V.threads, (2 * max_vrows + 63) / 64 * 64);   // two lanes per hanging-node row
+    // a mesh in one tile updates every node in every sub-step: a wave of its
+    // own samples the receivers beside (861-node layer, 49 receivers, FP64:
+    // 2.15 us a step against 2.69)
+    if (R.whole && max_recv > 0 && V.threads + 64 <= kMaxThreads) V.threads += 64;
     if (V.threads > kMaxThreads)
         throw fail(DMP_EUNSUPPORTED, "tiles need %d threads (max %d)", V.threads, kMaxThreads);
     // every index the kernel follows stays inside its array (checked before
@@ -1694,6 +1715,11 @@ void build_tiles(Runtime& R)
         });
         for (const PatchT& P : patch) V.patch_hetero |= P.hetero;
     }
+    if (R.whole) {
+        const size_t fixed = step_lds_bytes(V, R.precision), per = sizeof(double2) * (V.lds_force + V.lds_recv);
+        const size_t room = R.lds_limit > fixed ? (R.lds_limit - fixed) / std::max<size_t>(per, 1) : 0;
+        V.depth = std::min<int>(kWholeSteps, K + (int)std::min<size_t>(room, kWholeSteps));
+    }
     const size_t lds = step_lds_bytes(V, R.precision);
     if (std::getenv("DMP_LAYOUT_STATS")) {
         double ent = 0, ring = 0;
@@ -1800,33 +1826,46 @@ void build_tiles(Runtime& R)
         std::copy(U, U + kStateSlots, V.U);
     }
     R.state_depth = K;
-    R.tiles_block = B;
+    R.tiles_block = R.tuning[0];
     R.tiles_depth = K;
+    R.tiles_own = R.own_shape;
 }
 
 void prepare_graph(Runtime& R);
 
 void Runtime::apply_tuning()
 {
-    if (tiles_block != tuning[0] || tiles_depth != tuning[3]) build_tiles(*this);
+    if (tiles_block != tuning[0] || tiles_depth != tuning[3] || tiles_own != own_shape) {
+        no_whole = false;
+        try {
+            build_tiles(*this);
+        } catch (const Error& e) {
+            if (!whole || e.code != DMP_EUNSUPPORTED) throw;
+            no_whole = true;
+            build_tiles(*this);
+        }
+    }
     apply_launch_shape();
     // the receiver ring is part of the captured view: a layout built before
     // the ring exists gets its graph when the ring is allocated
     if (V.nrecv <= 0 || V.recv_interval <= 0 || V.recv_cap > 0) prepare_graph(*this);
 }
 
-// Switches to tuning t; a shape the layout cannot use leaves the previous one
+// Switches to tuning t (null: dmp_init's); a shape the layout cannot use leaves the previous one
 // in place and reports why.
 void set_tuning(Runtime& R, const int* t)
 {
     int old[4];
+    const bool old_own = R.own_shape;
+    R.own_shape = !t;
     for (int k = 0; k < 4; ++k) {
         old[k] = R.tuning[k];
-        R.tuning[k] = t[k];
+        R.tuning[k] = t ? t[k] : R.init_tuning[k];
     }
     try {
         R.apply_tuning();
     } catch (const Error&) {
+        R.own_shape = old_own;
         for (int k = 0; k < 4; ++k) R.tuning[k] = old[k];
         R.apply_tuning();
         throw;
@@ -2293,7 +2332,8 @@ void capture_graph(Runtime& R, int g, int k)
 int graph_length(const Runtime& R)
 {
     const DevView& V = R.V;
-    const int K = R.tuning[3];
+    const int K = V.depth;
+    if (R.whole) return 0;   // a launch takes as many steps as a graph would
     int G = std::min(R.tuning[2], V.chunk - 1);
     if (V.nrecv > 0 && V.recv_interval > 0)
         G = (int)std::min<long>(G, (V.recv_cap / 4 - 1) * (long)V.recv_interval);
@@ -2305,7 +2345,7 @@ int graph_length(const Runtime& R)
 void prepare_graph(Runtime& R)
 {
     const int G = graph_length(R);
-    if (G > 0 && (R.graph_steps != G || R.graph_k != R.tuning[3] || !R.gexec)) capture_graph(R, G, R.tuning[3]);
+    if (G > 0 && (R.graph_steps != G || R.graph_k != R.V.depth || !R.gexec)) capture_graph(R, G, R.V.depth);
 }
 
 // The source tables cover steps [a, b] (b - a < chunk); otherwise they are
@@ -2391,7 +2431,7 @@ int run_steps(Runtime& R, int n, double* out)
     const bool stream_out = out && nsamp > 0;
     const size_t row = (size_t)2 * V.nrecv;
     const long cap = V.recv_cap;
-    const int K = R.tuning[3];
+    const int K = V.depth;
     const int G = graph_length(R);
 
     // samples [q_lo, copied) are in out; a mark's event completes once the
@@ -2517,7 +2557,7 @@ int run_steps_noalloc(Runtime& R, int n, double* out)
         V.recv_buf = R.scratch;
         V.recv_cap = (int)slots;
     }
-    const int K = R.tuning[3];
+    const int K = V.depth;
     const bool end_sample = rec && (s + n) % I == 0 && (n > 0 || R.first_run);
     bool end_done = false;
     HIPCHECK(hipEventRecord(R.ev0, R.stream));
@@ -2711,6 +2751,7 @@ void autotune(Runtime& R, int nsteps, int* out)
         R.step = step0;
     };
     int best[4] = {R.tuning[0], R.tuning[1], R.tuning[2], R.tuning[3]};
+    R.own_shape = false;
     double best_t = 1e300;
     // tile sizes: 64, 128, 256, and those giving one or two tiles per compute
     // unit (small meshes are latency-bound: one tile per CU, no CU twice)
@@ -2725,6 +2766,11 @@ void autotune(Runtime& R, int nsteps, int* out)
                 std::find(cand_block.begin(), cand_block.end(), b) == cand_block.end())
                 cand_block.push_back(b);
         }
+    }
+    // and one tile, where it holds the whole mesh
+    if (R.V.na <= kMaxSlots) {
+        const int b = std::max(R.V.na, kMinBlock);
+        if (std::find(cand_block.begin(), cand_block.end(), b) == cand_block.end()) cand_block.push_back(b);
     }
     // many tiles per compute unit (bandwidth-bound): deep launches only add
     // ring work, so one and two steps per launch are tried
@@ -3134,9 +3180,8 @@ int dmp_set_tuning(void* h, const int* tuning)
     Instance* I = as<Instance>(h);
     return guarded(&I->err, [&] {
         if (!I->rt) throw fail(DMP_ESTATE, "dmp_init must come first");
-        const int* t = tuning ? tuning : I->rt->init_tuning;
-        check_tuning(t);
-        set_tuning(*I->rt, t);
+        if (tuning) check_tuning(tuning);
+        set_tuning(*I->rt, tuning);
     });
 }
 
@@ -3251,9 +3296,8 @@ int dmp_batch_set_tuning(void* b, const int* tuning)
     if (!b) return finish(nullptr, Error{DMP_EINVAL, "null handle"});
     Batch* B = as<Batch>(b);
     return guarded(&B->err, [&] {
-        const int* t = tuning ? tuning : B->rt->init_tuning;
-        check_tuning(t);
-        set_tuning(*B->rt, t);
+        if (tuning) check_tuning(tuning);
+        set_tuning(*B->rt, tuning);
     });
 }
 

@@ -167,7 +167,9 @@ int dmp_export_mesh(void *h, int *eptr, int *eind, bool *ediv, int *hanging, int
  * launch advances (1..8; each tile then carries that many rings of
  * neighbours in LDS).  dmp_init starts from {256, 1, 60, 3} ({256, 1, 60, 1}
  * above 200,000 nodes), falling back to smaller shapes where the mesh needs
- * it; NULL restores that initial shape.  The shape's graph is instantiated
+ * it; NULL restores that initial shape.  A mesh of at most 1023 nodes at this
+ * initial shape, or with tuning[0] no less than its nodes and tuning[3] above 1,
+ * is one tile, which takes up to 32 steps per launch.  The shape's graph is instantiated
  * here, so that no dmp_run pays for it.  A shape the mesh cannot use (LDS,
  * descriptor range) returns DMP_EUNSUPPORTED and leaves the previous shape in
  * place. */

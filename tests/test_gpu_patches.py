@@ -75,3 +75,38 @@ def test_state_across_layouts(prec):
     assert np.array_equal(np.concatenate(parts), r0)
     for a, b in ((u, u0), (up, up0), (u1, u0), (up1, up0)):
         assert np.array_equal(a, b)
+
+
+@pytest.mark.parametrize("prec", [0, 1])
+@pytest.mark.parametrize("name", ["f1", "f2het_buried", "pointd", "layer_1023"])
+def test_whole_mesh_in_one_tile(name, prec):
+    """Meshes of one tile, up to the largest (1023 nodes), take as many steps
+    per launch as the LDS holds source terms for: calls shorter, as long and
+    longer than a launch, sampled every step and every third, give the bits of
+    launches of few steps in several tiles."""
+    from damian_hip import cases, lib
+    if name == "layer_1023":
+        case = layer(cases, 32, 30, True)
+    elif name.endswith("_buried"):
+        case = cases.with_buried_receivers(cases.BUILDERS[name[:-len("_buried")]]())
+    else:
+        case = cases.BUILDERS[name]()
+    n = case.mesh.nnodes - len(case.hanging)
+    assert n <= 1023
+    for io in (1, 3):
+        ref = lib.Solver(case, precision=prec, io_interval=io)
+        ref.set_tuning(64, 0, 0, 2)
+        want = ref.run(200), ref.state()
+        ref.close()
+        assert np.abs(want[0]).max() > 0
+        for tuning in (None, (max(n, 32), 0, 12, 2)):
+            print(f"name={name} nodes={n} prec={prec} io={io} tuning={tuning}", flush=True)
+            s = lib.Solver(case, precision=prec, io_interval=io)
+            if tuning:
+                s.set_tuning(*tuning)
+            parts = [s.run(k) for k in (1, 1, 8, 31, 32, 33)] + [s.run(17, noalloc=True), s.run(77)]
+            got = s.state()
+            s.close()
+            assert np.array_equal(np.concatenate(parts), want[0])
+            for a, b in zip(got, want[1]):
+                assert np.array_equal(a, b)
