@@ -285,6 +285,7 @@ struct Runtime {
     bool own_shape = true;         // the shape is dmp_init's, not one that the caller or the autotuner chose
     bool tiles_own = true;         // own_shape when the tile arrays were built
     bool no_whole = false;         // the mesh does not fit in one tile after all
+    bool no_patches = false;       // the tiles between patches do not fit
     bool whole = false;            // one tile holds the mesh: no rings, up to V.depth steps per launch
     int state_depth = kMaxDepth;   // depth whose state_slot() the state buffers are in
     std::vector<void*> tile_allocs;
@@ -935,88 +936,107 @@ struct TileScratch {
     }
 };
 
-// One-step layouts: runs of kPatchNodes nodes that form a patch (PatchT), as
-// start nodes in ascending order, with the ring of each.  A run is a patch
-// where its nodes are an aligned cell of the Morton order of a uniform part
-// of the mesh: every node is updated by the plain formula, has four elements
-// without hanging corners, and its eight neighbours are the nodes that its
-// place in the patch says.  `taken` marks nodes that tiles need (the corners
-// by which receivers are given to tiles).
+// Runs of M x M nodes that form a patch (PatchT) for launches of up to D steps,
+// as start nodes in ascending order, with the nodes of the rings around each.
+// A run is a patch where its nodes are an aligned cell of the Morton order of
+// a uniform part of the mesh: every node that a launch updates for it (the run
+// and D - 1 rings) is updated by the plain formula and has four elements
+// without hanging corners, and the eight neighbours of each are those that its
+// place on the grid says.  `taken` marks nodes that tiles need (the corners by
+// which receivers are given to tiles).
 struct PatchRuns {
     std::vector<int> start;
-    std::vector<int> ring;      // kPatchRing per start
+    std::vector<int> ring;      // (M + 2 D)^2 - M^2 per start
+    int nodes = 0;              // M^2
 };
 
-PatchRuns find_patches(const PackedHost& H, int NA, const std::vector<char>& taken)
+PatchRuns find_patches(const PackedHost& H, int NA, const std::vector<char>& taken, int M, int D)
 {
-    constexpr int N = kPatch, W = N + 2;
-    // node n's neighbour at (x, z) offset d, from its four elements; -1 where
-    // n is not plain or the elements do not agree
+    const int W = M + 2 * D, N = M * M;
+    PatchRuns out;
+    out.nodes = N;
+    // nodes of the plain formula whose four elements agree on their neighbours
     std::vector<char> plain(NA, 0);
     auto corners = [&](int e) { return H.elem_corners[e]; };
     const int nblk = std::max(1, std::min(256, NA / 4096 + 1)), nth = setup_threads();
     parallel_items(nblk, nth, [&](int b) {
         for (int n = (int)((long)NA * b / nblk); n < (int)((long)NA * (b + 1) / nblk); ++n) {
             const int4 q = H.node_elems[n];
-            if (taken[n] || H.node_side[n] >= 0 || q.x < 0 || q.y < 0 || q.z < 0 || q.w < 0) continue;
+            if (H.node_side[n] >= 0 || q.x < 0 || q.y < 0 || q.z < 0 || q.w < 0) continue;
             const int4 a = corners(q.x), c = corners(q.y), d = corners(q.z), e = corners(q.w);
             bool ok = c.x == d.w && a.y == e.z && a.w == c.z && d.y == e.x;
             for (const int4& k : {a, c, d, e}) ok = ok && std::max(std::max(k.x, k.y), std::max(k.z, k.w)) < NA;
             plain[n] = ok;
         }
     });
-    int xof[kPatchNodes], zof[kPatchNodes];
-    for (int m = 0; m < kPatchNodes; ++m) {
-        xof[m] = zof[m] = 0;
-        for (int b = 0; (1 << (2 * b)) < kPatchNodes; ++b) {
-            zof[m] |= ((m >> (2 * b)) & 1) << b;
-            xof[m] |= ((m >> (2 * b + 1)) & 1) << b;
+    // place of node m of a run, and the positions of ring r >= 1 (of the square
+    // with r rings less that with r - 1), in the (M + 2 D)^2 image
+    std::vector<int> place(N);
+    for (int m = 0; m < N; ++m) {
+        int x = 0, z = 0;
+        for (int b = 0; (1 << (2 * b)) < N; ++b) {
+            z |= ((m >> (2 * b)) & 1) << b;
+            x |= ((m >> (2 * b + 1)) & 1) << b;
         }
+        place[m] = (x + D) * W + z + D;
     }
-    // fills the (N + 2)^2 image of the patch at s; false where it is none
-    auto image = [&](int s, int* img) {
-        std::fill(img, img + W * W, -1);
-        for (int m = 0; m < kPatchNodes; ++m) img[(xof[m] + 1) * W + zof[m] + 1] = s + m;
-        for (int m = 0; m < kPatchNodes; ++m) {
-            const int n = s + m;
-            if (!plain[n]) return false;
+    std::vector<int> order = place;   // image positions from the run outwards
+    for (int r = 1; r < D; ++r)
+        for (int x = D - r; x < D + M + r; ++x)
+            for (int z = D - r; z < D + M + r; ++z)
+                if (x == D - r || x == D + M + r - 1 || z == D - r || z == D + M + r - 1) order.push_back(x * W + z);
+    // fills the image of the run at s; false where it is no patch
+    auto image = [&](int s, std::vector<int>& img) {
+        std::fill(img.begin(), img.end(), -1);
+        for (int m = 0; m < N; ++m) img[place[m]] = s + m;
+        for (size_t i = 0; i < order.size(); ++i) {
+            const int at = order[i], n = img[at];
+            if (n < 0 || !plain[n] || (i < (size_t)N && taken[n])) return false;
             const int4 q = H.node_elems[n];
             const int4 a = corners(q.x), c = corners(q.y), d = corners(q.z), e = corners(q.w);
-            const int nb[8][3] = {{1, 0, a.y}, {1, 1, a.z}, {0, 1, a.w}, {-1, 0, c.x},
-                                  {-1, 1, c.w}, {-1, -1, d.x}, {0, -1, d.y}, {1, -1, e.y}};
+            const int nb[8][2] = {{W, a.y}, {W + 1, a.z}, {1, a.w}, {-W, c.x},
+                                  {-W + 1, c.w}, {-W - 1, d.x}, {-1, d.y}, {W - 1, e.y}};
             for (const auto& k : nb) {
-                int& at = img[(xof[m] + 1 + k[0]) * W + zof[m] + 1 + k[1]];
-                if (at < 0) at = k[2];
-                if (at != k[2]) return false;
+                int& p = img[at + k[0]];
+                if (p < 0) p = k[1];
+                if (p != k[1]) return false;
             }
         }
         return true;
     };
     std::vector<char> is(NA, 0);
     parallel_items(nblk, nth, [&](int b) {
-        int img[W * W];
+        std::vector<int> img((size_t)W * W);
         const int lo = (int)((long)NA * b / nblk), hi = (int)((long)NA * (b + 1) / nblk);
         for (int s = lo; s < hi; ++s)
-            if (s + kPatchNodes <= NA && plain[s] && plain[s + kPatchNodes - 1]) is[s] = image(s, img);
+            if (s + N <= NA && plain[s] && plain[s + N - 1]) is[s] = image(s, img);
     });
-    PatchRuns out;
     for (int s = 0; s < NA; ++s)
         if (is[s]) {
             out.start.push_back(s);
-            s += kPatchNodes - 1;
+            s += N - 1;
         }
-    const int np = (int)out.start.size();
-    out.ring.resize((size_t)np * kPatchRing);
-    parallel_items(std::max(1, std::min(np, nblk)), nth, [&](int b) {
-        const int nb = std::max(1, std::min(np, nblk));
-        int img[W * W];
+    const int np = (int)out.start.size(), len = W * W - N;
+    if ((size_t)np * len > (size_t)INT32_MAX) throw fail(DMP_EUNSUPPORTED, "patch ring lists too long");
+    out.ring.resize((size_t)np * len);
+    const int nb = std::max(1, std::min(np, nblk));
+    parallel_items(nb, nth, [&](int b) {
+        std::vector<int> img((size_t)W * W);
         for (int i = (int)((long)np * b / nb); i < (int)((long)np * (b + 1) / nb); ++i) {
             image(out.start[i], img);
-            int* r = &out.ring[(size_t)i * kPatchRing];
-            for (int z = 0; z <= N; ++z) *r++ = img[z];                       // x = -1
-            for (int x = 1; x <= N; ++x) *r++ = img[x * W];                   // z = -1
-            for (int x = 0; x <= N; ++x) *r++ = img[x * W + N + 1];           // z = N
-            for (int z = 0; z <= N + 1; ++z) *r++ = img[(N + 1) * W + z];     // x = N
+            int* r = &out.ring[(size_t)i * len];
+            if (D == 1) {   // kPatchLow order
+                for (int z = 0; z <= M; ++z) *r++ = img[z];                       // x = -1
+                for (int x = 1; x <= M; ++x) *r++ = img[x * W];                   // z = -1
+                for (int x = 0; x <= M; ++x) *r++ = img[x * W + M + 1];           // z = M
+                for (int z = 0; z <= M + 1; ++z) *r++ = img[(M + 1) * W + z];     // x = M
+            } else {
+                for (int e = N; e < W * W; ++e) {
+                    int x, z;
+                    block_patch_xz(e, x, z);
+                    *r++ = img[(x + D) * W + z + D];
+                }
+            }
         }
     });
     return out;
@@ -1060,47 +1080,53 @@ void build_tiles(Runtime& R)
     int ncu = 0;
     if (hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, R.device) != hipSuccess || ncu < 1)
         ncu = 256;
-    std::vector<int> tstart(ntiles + 1, 0), tend;
-    // one step per launch: uniform parts of the mesh as patches, the runs of
-    // nodes between them as tiles of at most B nodes
+    // Uniform parts of the mesh as patches: always at one step per launch; at
+    // several where there are more tiles than compute units, so that work in
+    // flight and not the slowest tile's latency bounds a launch.
     PatchRuns patches;
-    if (K == 1) {
+    if (!R.no_patches && (K == 1 || (ntiles > ncu && !R.whole))) {
         std::vector<char> taken(NA, 0);
         for (const RecvRec& x : H.recv) {
             const int c = x.c[0];
             if (c >= 0) taken[c < NA ? c : H.vanch[c - NA].x] = 1;
         }
-        patches = find_patches(H, NA, taken);
-        const int np = (int)patches.start.size();
-        tstart.clear();
-        for (int i = 0; i <= np; ++i) {
-            const int lo = i ? patches.start[i - 1] + kPatchNodes : 0, hi = i < np ? patches.start[i] : NA;
+        patches = find_patches(H, NA, taken, K == 1 ? kPatch : kBlockPatch, K);
+    }
+    // The runs of nodes between them as tiles.
+    const bool equal_work = K > 1 && ntiles <= 2 * ncu;
+    std::vector<double> cum(equal_work ? NA + 1 : 0, 0.0);
+    for (int i = 0; equal_work && i < NA; ++i) {
+        const int si = H.node_side[i];
+        const bool anchor = si >= 0 && H.side[si].tr_count > 0;
+        cum[i + 1] = cum[i] + 1.0 + (anchor ? kAnchorWeight : 0.0);
+    }
+    const double share = equal_work ? cum[NA] / ntiles : 0.0;
+    std::vector<int> tstart, tend;
+    for (size_t i = 0; i <= patches.start.size(); ++i) {
+        const int lo = i ? patches.start[i - 1] + patches.nodes : 0, hi = i < patches.start.size() ? patches.start[i] : NA;
+        if (lo >= hi) continue;
+        if (!equal_work) {
             for (int n = lo; n < hi; n += B) {
                 tstart.push_back(n);
                 tend.push_back(std::min(n + B, hi));
             }
+            continue;
         }
-        ntiles = (int)tstart.size();
-    } else if (ntiles > 2 * ncu) {
-        for (int t = 1; t <= ntiles; ++t) tstart[t] = std::min(t * B, NA);
-    } else {
-        std::vector<double> cum(NA + 1, 0.0);
-        for (int i = 0; i < NA; ++i) {
-            const int si = H.node_side[i];
-            const bool anchor = si >= 0 && H.side[si].tr_count > 0;
-            cum[i + 1] = cum[i] + 1.0 + (anchor ? kAnchorWeight : 0.0);
+        const double work = cum[hi] - cum[lo];
+        const int m = std::max(1, std::min(hi - lo, (int)std::ceil(work / share - 1e-6)));
+        for (int t = 1; t <= m; ++t) {
+            const int from = t == 1 ? lo : tend.back();
+            int to = hi;
+            if (t < m) {
+                to = (int)(std::lower_bound(cum.begin(), cum.end(), cum[lo] + work * t / m) - cum.begin());
+                to = std::max(to, from + 1);   // every tile keeps a node
+                to = std::min(to, hi - (m - t));
+            }
+            tstart.push_back(from);
+            tend.push_back(to);
         }
-        for (int t = 1; t < ntiles; ++t) {
-            const double goal = cum[NA] * t / ntiles;
-            int i = (int)(std::lower_bound(cum.begin(), cum.end(), goal) - cum.begin());
-            i = std::max(i, tstart[t - 1] + 1);   // every tile keeps a node
-            i = std::min(i, NA - (ntiles - t));
-            tstart[t] = i;
-        }
-        tstart[ntiles] = NA;
     }
-    if (K > 1) tend.assign(tstart.begin() + 1, tstart.end());
-    tstart.resize(ntiles);
+    ntiles = (int)tstart.size();
     auto tile_of = [&](int node) {
         return (int)(std::upper_bound(tstart.begin(), tstart.end(), node) - tstart.begin()) - 1;
     };
@@ -1685,7 +1711,14 @@ void build_tiles(Runtime& R)
     // uniform, else read per node
     V.patches = (int)patches.start.size();
     V.patch_hetero = 0;
-    V.patch_blocks = (V.patches + V.threads / 64 - 1) / (V.threads / 64);
+    if (K > 1 && V.patches) {   // a lane per entry that a launch updates
+        const int w = block_patch_width(K) - 2;
+        V.threads = std::max(V.threads, (w * w + 63) / 64 * 64);
+        if (V.threads > kMaxThreads) throw fail(DMP_EUNSUPPORTED, "patches need %d threads (max %d)", V.threads, kMaxThreads);
+    }
+    const int per_block = K == 1 ? V.threads / 64 : 1;
+    V.patch_blocks = (V.patches + per_block - 1) / per_block;
+    const int pn = patches.nodes, plen = V.patches ? (int)(patches.ring.size() / V.patches) : 0;
     std::vector<PatchT> patch(V.patches);
     {
         const int nblk = std::max(1, std::min(V.patches, 16 * setup_threads()));
@@ -1694,22 +1727,32 @@ void build_tiles(Runtime& R)
                 PatchT& P = patch[i];
                 P = PatchT{};
                 P.n0 = patches.start[i];
-                if (P.n0 < 0 || P.n0 + kPatchNodes > NA) throw fail(DMP_EINVAL, "internal: patch %d out of range", i);
-                const int* ring = &patches.ring[(size_t)i * kPatchRing];
+                if (P.n0 < 0 || P.n0 + pn > NA) throw fail(DMP_EINVAL, "internal: patch %d out of range", i);
+                const int* ring = &patches.ring[(size_t)i * plen];
                 P.lam = H.node_em[2 * (size_t)P.n0];
                 P.mu = H.node_em[2 * (size_t)P.n0 + 1];
                 P.invm = H.invm[P.n0];
-                auto same = [&](int n) {
+                auto moduli = [&](int n) {
                     if (H.node_em[2 * (size_t)n] != P.lam || H.node_em[2 * (size_t)n + 1] != P.mu) P.hetero = 1;
                 };
-                for (int m = 0; m < kPatchNodes; ++m) {
-                    same(P.n0 + m);
-                    if (H.invm[P.n0 + m] != P.invm) P.coefs = 1;
+                auto mass = [&](int n) {
+                    if (H.invm[n] != P.invm) P.coefs = 1;
+                };
+                for (int m = 0; m < pn; ++m) {
+                    moduli(P.n0 + m);
+                    mass(P.n0 + m);
                     core_coef[P.n0 + m] = H.invm[P.n0 + m];
                 }
-                for (int r = 0; r < kPatchRing; ++r) {
+                const int updated = K == 1 ? 0 : (block_patch_width(K) - 2) * (block_patch_width(K) - 2) - pn;
+                for (int r = 0; r < plen; ++r) {
                     if (ring[r] < 0 || ring[r] >= NA) throw fail(DMP_EINVAL, "internal: patch %d: ring node out of range", i);
-                    if (r < kPatchLow) same(ring[r]);
+                    if (r < updated) mass(ring[r]);
+                    // the outer ring: its nodes are corner 0 of elements that
+                    // a launch reads at its lower x and z sides
+                    int x = 0, z = 0;
+                    if (K > 1) block_patch_xz(pn + r, x, z);
+                    if (K == 1 ? r < kPatchLow : r < updated || ((x < 0 || z < 0) && x < kBlockPatch + K - 1 && z < kBlockPatch + K - 1))
+                        moduli(ring[r]);
                 }
             }
         });
@@ -1836,12 +1879,13 @@ void prepare_graph(Runtime& R);
 void Runtime::apply_tuning()
 {
     if (tiles_block != tuning[0] || tiles_depth != tuning[3] || tiles_own != own_shape) {
-        no_whole = false;
+        no_whole = no_patches = false;
         try {
             build_tiles(*this);
         } catch (const Error& e) {
-            if (!whole || e.code != DMP_EUNSUPPORTED) throw;
-            no_whole = true;
+            // a shape that plain tiles can take is taken
+            if (e.code != DMP_EUNSUPPORTED) throw;
+            no_whole = no_patches = true;
             build_tiles(*this);
         }
     }
@@ -2773,13 +2817,17 @@ void autotune(Runtime& R, int nsteps, int* out)
         if (std::find(cand_block.begin(), cand_block.end(), b) == cand_block.end()) cand_block.push_back(b);
     }
     // many tiles per compute unit (bandwidth-bound): deep launches only add
-    // ring work, so one and two steps per launch are tried
+    // ring work.  Basins of 141,000, 237,000 and 317,000 nodes, FP32C, best
+    // shape at 1, 2, 3 and 4 steps per launch: 7.3, 4.6, 3.9, 4.1; 7.6, 6.0,
+    // 5.6, 6.4; 7.9, 7.6, 6.9, 6.6 us a step; the 947,000-node uniform canyon
+    // 10.2, 14.2, 11.5, 14.1.
     std::vector<int> cand_depth = {1, 2, 3, 4, 6, 8};
     {
         int ncu = 0;
         if (hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, R.device) != hipSuccess || ncu < 1)
             ncu = 256;
-        if (R.V.na > 2 * 256 * ncu) cand_depth = {1, 2};
+        if (R.V.na > 6 * 256 * ncu) cand_depth = {1, 2};
+        else if (R.V.na > 2 * 256 * ncu) cand_depth = {1, 2, 3, 4};
     }
     for (int b : cand_block)
         for (int K : cand_depth) {

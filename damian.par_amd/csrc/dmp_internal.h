@@ -147,6 +147,38 @@ constexpr int kPatchSlots = (kPatch + 2) * kPatchPitch;
 // patch's lower x and z sides, whose moduli are read), then the rest.
 constexpr int kPatchLow = 2 * kPatch + 1;
 
+// Layouts of several steps per launch: a block patch of kBlockPatch x
+// kBlockPatch nodes, a Morton cell likewise, is one workgroup's work, with the
+// `depth` rings of nodes around it; all that a launch updates there (the patch
+// and its rings but the last) are nodes of the same kind on the same grid.
+// Entries: the patch's nodes in Morton order, then ring 1, 2, ..: ring r goes
+// round from (-r, -r) along z, x, back along z and x (block_patch_xz).
+constexpr int kBlockPatch = 16;
+constexpr int kBlockPatchNodes = kBlockPatch * kBlockPatch;
+// Coordinates in the patch of entry e.
+__host__ __device__ inline void block_patch_xz(int e, int& x, int& z)
+{
+    if (e < kBlockPatchNodes) {
+        x = z = 0;
+        for (int b = 0; (1 << (2 * b)) < kBlockPatchNodes; ++b) {
+            z |= ((e >> (2 * b)) & 1) << b;
+            x |= ((e >> (2 * b + 1)) & 1) << b;
+        }
+        return;
+    }
+    int r = 1;
+    while (e >= (kBlockPatch + 2 * r) * (kBlockPatch + 2 * r)) ++r;
+    const int L = kBlockPatch + 2 * r - 1;   // steps along a side
+    const int i = e - (L - 1) * (L - 1);
+    const int side = (i >= L) + (i >= 2 * L) + (i >= 3 * L), off = i - side * L;
+    const int hi = kBlockPatch - 1 + r;
+    x = side == 0 ? -r : side == 1 ? off - r : side == 2 ? hi : hi - off;
+    z = side == 0 ? off - r : side == 1 ? hi : side == 2 ? hi - off : -r;
+}
+// LDS image with its rings: width and pitch (4 mod 8, as kPatchPitch).
+__host__ __device__ inline int block_patch_width(int depth) { return kBlockPatch + 2 * depth; }
+__host__ __device__ inline int block_patch_pitch(int depth) { return (block_patch_width(depth) + 3) / 8 * 8 + 4; }
+
 struct PatchT {
     int n0;
     int hetero;          // 1: (lambda, mu) per element from node_em, 0: lam, mu
@@ -277,13 +309,14 @@ struct DevView {
     const RecvG* rg;          // receivers in global node ids
     void* U[kStateSlots];     // u_j in U[state_slot(j, depth)], 16 B per active node
     Ctrl* ctrl;
-    // one-step layouts: patches, beside the tiles
+    // patches, beside the tiles: one-step layouts threads / 64 to a workgroup,
+    // deeper ones (block patches) one
     int patches;
     int patch_hetero;    // some patch reads (lambda, mu) per element
-    int patch_blocks;    // workgroups of threads / 64 patches
+    int patch_blocks;    // workgroups
     int patch_blocks_per_xcd;
     const PatchT* patch;
-    const int* patch_ring;    // [patches][kPatchRing] nodes around each
+    const int* patch_ring;    // per patch the nodes around it: kPatchRing, or the block patch's ring entries
 };
 
 } // namespace dmp

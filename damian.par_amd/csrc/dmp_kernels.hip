@@ -643,10 +643,12 @@ __device__ __forceinline__ void load_entries(const DevView& V, int tile, const v
     }
 }
 
-// LDS of one patch: values, and moduli per element where a patch needs them.
+// LDS of one patch: values (of a block patch at two steps), and moduli per
+// element where a patch needs them.
 __host__ __device__ inline int patch_lds_bytes(const DevView& V, int real_bytes)
 {
-    return kPatchSlots * (16 + (V.patch_hetero ? 2 * real_bytes : 0));
+    const int slots = V.depth == 1 ? kPatchSlots : block_patch_width(V.depth) * block_patch_pitch(V.depth);
+    return slots * ((V.depth == 1 ? 16 : 32) + (V.patch_hetero ? 2 * real_bytes : 0));
 }
 
 // ---------------------------------------------------------------------------
@@ -670,6 +672,36 @@ __device__ __forceinline__ int patch_ring_slot(int r)
     if (r < kPatchLow) return (r - N) * W;                   // z = -1, x = 0 .. N-1
     if (r < kPatchLow + N + 1) return (r - kPatchLow) * W + N + 1;   // z = N, x = -1 .. N-1
     return (N + 1) * W + (r - kPatchLow - N - 1);            // x = N, z = -1 .. N
+}
+
+// -K u of a node whose neighbours lie at +-1 (z) and +-W (x) around it in an
+// LDS image, with the moduli of the patch's record or, per element, at the
+// element's corner 0 in the image m: element by element as Rows::apply.
+template <class P>
+__device__ __forceinline__ V2<typename P::real> grid_rows(const typename P::node_t* c, int W,
+                                                          typename P::node_t un, const PatchT& T,
+                                                          const V2<typename P::real>* m)
+{
+    using R = typename P::real;
+    using node_t = typename P::node_t;
+    const node_t xm = c[-W], xp = c[W], zm = c[-1], zp = c[1];
+    const node_t mm = c[-W - 1], mp = c[-W + 1], pm = c[W - 1], pp = c[W + 1];
+    // the element of which the node is corner 0, 1, 2, 3
+    const node_t c0[3] = {xp, pp, zp}, c1[3] = {xm, zp, mp}, c2[3] = {mm, zm, xm}, c3[3] = {zm, pm, xp};
+    V2<R> f{0, 0};
+    if (T.hetero) {
+        slot_rows_v<P, 0>(c0, m[0], un, f);
+        slot_rows_v<P, 1>(c1, m[-W], un, f);
+        slot_rows_v<P, 2>(c2, m[-W - 1], un, f);
+        slot_rows_v<P, 3>(c3, m[-1], un, f);
+    } else {
+        const V2<R> lm{R(T.lam), R(T.mu)};
+        slot_rows_v<P, 0>(c0, lm, un, f);
+        slot_rows_v<P, 1>(c1, lm, un, f);
+        slot_rows_v<P, 2>(c2, lm, un, f);
+        slot_rows_v<P, 3>(c3, lm, un, f);
+    }
+    return f;
 }
 
 template <class P>
@@ -724,25 +756,82 @@ __device__ __forceinline__ void patch_step(const DevView& V, int t, const void* 
         const node_t* c = val + at + (q >> 1) * 8 * W + (q & 1) * 8;
         const V2<R>* m = em + at + (q >> 1) * 8 * W + (q & 1) * 8;
         const node_t un = c[0];
-        const node_t xm = c[-W], xp = c[W], zm = c[-1], zp = c[1];
-        const node_t mm = c[-W - 1], mp = c[-W + 1], pm = c[W - 1], pp = c[W + 1];
-        // the element of which the node is corner 0, 1, 2, 3, as Rows::apply
-        const node_t c0[3] = {xp, pp, zp}, c1[3] = {xm, zp, mp}, c2[3] = {mm, zm, xm}, c3[3] = {zm, pm, xp};
-        V2<R> f{0, 0};
-        if (T.hetero) {
-            slot_rows_v<P, 0>(c0, m[0], un, f);
-            slot_rows_v<P, 1>(c1, m[-W], un, f);
-            slot_rows_v<P, 2>(c2, m[-W - 1], un, f);
-            slot_rows_v<P, 3>(c3, m[-1], un, f);
-        } else {
-            const V2<R> lm{R(T.lam), R(T.mu)};
-            slot_rows_v<P, 0>(c0, lm, un, f);
-            slot_rows_v<P, 1>(c1, lm, un, f);
-            slot_rows_v<P, 2>(c2, lm, un, f);
-            slot_rows_v<P, 3>(c3, lm, un, f);
-        }
+        const V2<R> f = grid_rows<P>(c, W, un, T, m);
         const R cf = T.coefs ? P::coef(V.core_coef, T.n0 + 64 * q + lane) : R(T.invm);
         P::st(Uk, T.n0 + 64 * q + lane, P::advance(un, p[q], over_mass(f, cf, cf)));
+    }
+}
+
+// ---------------------------------------------------------------------------
+// k <= depth steps of a block patch by one workgroup: lane e keeps entry e's
+// last two levels in registers, the LDS holds what neighbours read, at two
+// steps in turn (one barrier per step).
+//
+// Where a mesh has more tiles than compute units, a launch of several steps is
+// bound by the wavefronts in flight: a tile's share of registers, LDS and
+// instructions (descriptors, 12 corner reads, three barriers a step) allows
+// one or two tiles per compute unit, in several rounds.  Patches need a third
+// less of each: the 141,000-element basin takes 5.06 us a step in FP32C at 256
+// nodes per tile and 3 steps per launch against 7.63 with tiles only (FP64
+// 5.05 against 7.94), 3.86 at its best shape against 5.2.
+// ---------------------------------------------------------------------------
+template <class P>
+__device__ __forceinline__ void block_patch_steps(const DevView& V, int t, int k, const void* U0, const void* Um,
+                                                  void* Uk, void* Uk1, unsigned char* lds)
+{
+    using R = typename P::real;
+    using node_t = typename P::node_t;
+    const int D = V.depth, W = block_patch_width(D), S = block_patch_pitch(D);
+    const int nu = (W - 2) * (W - 2), ne = W * W;   // entries updated, entries
+    const int e = (int)threadIdx.x, NT = (int)blockDim.x;
+    const PatchT T = uniform_record(V.patch + t);
+    const int* ring = V.patch_ring + (size_t)t * (ne - kBlockPatchNodes);
+    node_t* cur = reinterpret_cast<node_t*>(lds);
+    node_t* nxt = cur + W * S;
+    V2<R>* em = reinterpret_cast<V2<R>*>(nxt + W * S);
+    // the outer ring, read only, on the lanes without an entry first
+    const int o = e >= nu ? e : e + NT;
+    int g = T.n0 + e, go = 0;
+    if (e >= kBlockPatchNodes && e < nu) g = ring[e - kBlockPatchNodes];
+    if (o < ne) go = ring[o - kBlockPatchNodes];
+    node_t un{}, up{}, uo{};
+    R cf = R(T.invm);
+    if (e < nu) {
+        un = P::ld(U0, g);
+        up = P::ld(Um, g);
+        if (T.coefs) cf = P::coef(V.core_coef, g);
+    }
+    if (o < ne) uo = P::ld(U0, go);
+    int x, z;
+    block_patch_xz(o < ne ? o : nu, x, z);
+    const int ato = (x + D) * S + z + D;
+    block_patch_xz(e < nu ? e : 0, x, z);
+    const int at = (x + D) * S + z + D;
+    if (T.hetero) {
+        if (e < nu) em[at] = P::lm(V.node_em, g);
+        if (o < ne) em[ato] = P::lm(V.node_em, go);
+    }
+    if (e < nu) cur[at] = un;
+    if (o < ne) cur[ato] = uo;
+    __syncthreads();
+    for (int s = 1; s <= k; ++s) {
+        const int w = kBlockPatch + 2 * (D - s);   // what is still exact after this step
+        if (e < w * w) {
+            const V2<R> f = grid_rows<P>(cur + at, S, un, T, em + at);
+            const node_t unew = P::advance(un, up, over_mass(f, cf, cf));
+            up = un;
+            un = unew;
+            if (s < k) nxt[at] = unew;
+        }
+        if (s == k) break;
+        __syncthreads();
+        node_t* q = cur;
+        cur = nxt;
+        nxt = q;
+    }
+    if (e < kBlockPatchNodes) {
+        P::st(Uk, g, un);
+        if (k > 1) P::st(Uk1, g, up);
     }
 }
 
@@ -1095,25 +1184,30 @@ __device__ void tile_steps(const DevView& V, int tile, int t0, int k, int end)
 // compiled for as many waves per SIMD as its registers allow without spills
 // (FP32C 7 with 72 VGPRs; FP64 6); the deeper one is latency-bound and keeps
 // the registers a 1024-thread workgroup leaves (4 waves per SIMD).
-template <class P, bool ONE, bool HANG>
+template <class P, bool ONE, bool HANG, bool PATCH>
 __global__ __launch_bounds__(kMaxThreads) __attribute__((amdgpu_waves_per_eu(ONE ? P::kOneWaves : 4)))
 void step_kernel(DevView V, int t0_arg, int use_base, int k, int end)
 {
     const int t0 = t0_arg + (use_base ? V.ctrl->base : 0);
     int b = blockIdx.x;
-    if (ONE) {
-        // tiles first (the longer work), then the patches
-        const int nb = V.xcd_remap ? 8 * V.tiles_per_xcd : V.node_tiles;
-        if (b >= nb) {
-            b -= nb;
-            const int blk = V.xcd_remap ? (b & 7) * V.patch_blocks_per_xcd + (b >> 3) : b;
+    // tiles first (the longer work), then the patches
+    const int nb = V.xcd_remap ? 8 * V.tiles_per_xcd : V.node_tiles;
+    if (PATCH && b >= nb) {
+        b -= nb;
+        const int blk = V.xcd_remap ? (b & 7) * V.patch_blocks_per_xcd + (b >> 3) : b;
+        extern __shared__ __align__(16) unsigned char smem[];
+        if (ONE) {
             const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
             const int t = blk * ((int)blockDim.x >> 6) + wave;
             if (blk >= V.patch_blocks || t >= V.patches || k < 1) return;
-            extern __shared__ __align__(16) unsigned char smem[];
-            patch_step<P>(V, t, V.U[state_slot(t0, 1)], V.U[state_slot(t0 - 1, 1)], V.U[state_slot(t0 + k, 1)], smem + wave * patch_lds_bytes(V, sizeof(typename P::real)));
-            return;
+            patch_step<P>(V, t, V.U[state_slot(t0, 1)], V.U[state_slot(t0 - 1, 1)], V.U[state_slot(t0 + k, 1)],
+                          smem + wave * patch_lds_bytes(V, sizeof(typename P::real)));
+        } else {
+            if (blk >= V.patches) return;
+            block_patch_steps<P>(V, blk, k, V.U[state_slot(t0, kMaxDepth)], V.U[state_slot(t0 - 1, kMaxDepth)],
+                                 V.U[state_slot(t0 + k, kMaxDepth)], V.U[state_slot(t0 + k - 1, kMaxDepth)], smem);
         }
+        return;
     }
     const int tile = V.xcd_remap ? (b & 7) * V.tiles_per_xcd + (b >> 3) : b;
     if (tile >= V.node_tiles) return;   // whole block exits together
@@ -1265,7 +1359,7 @@ static int node_grid(const DevView& V)
 size_t step_lds_bytes(const DevView& V, int precision)
 {
     const size_t rb = precision == 0 ? sizeof(double) : sizeof(float);
-    const size_t patches = V.patches ? (size_t)(V.threads / 64) * patch_lds_bytes(V, (int)rb) : 0;
+    const size_t patches = V.patches ? (size_t)(V.depth == 1 ? V.threads / 64 : 1) * patch_lds_bytes(V, (int)rb) : 0;
     return std::max(patches, (size_t)(V.depth > 1 ? 3 : 2) * V.lds_slots * 16 +
            (size_t)V.depth * V.lds_force * sizeof(double2) +
            (size_t)V.depth * V.lds_recv * sizeof(double2) +
@@ -1278,18 +1372,20 @@ template <class P>
 static void launch_one(const DevView& V, int grid, size_t lds, hipStream_t st, int t0, int use_base, int k,
                        int end)
 {
+    const auto go = [&](auto kernel) {
+        hipLaunchKernelGGL(kernel, dim3(grid), dim3(V.threads), lds, st, V, t0, use_base, k, V.depth == 1 ? 0 : end);
+    };
     // several steps per launch: meshes without hanging nodes have a kernel
     // without their phases, their barrier and a quarter of the registers
     // (40,000-element layer, FP64, 3 steps per launch: 2.95 us a step against
-    // 3.29 with the other)
-    if (V.depth == 1)
-        hipLaunchKernelGGL((step_kernel<P, true, true>), dim3(grid), dim3(V.threads), lds, st, V, t0, use_base, k, 0);
-    else if (V.nv > 0)
-        hipLaunchKernelGGL((step_kernel<P, false, true>), dim3(grid), dim3(V.threads), lds, st, V, t0, use_base, k,
-                           end);
-    else
-        hipLaunchKernelGGL((step_kernel<P, false, false>), dim3(grid), dim3(V.threads), lds, st, V, t0, use_base,
-                           k, end);
+    // 3.29 with the other), and layouts without patches, where the slowest
+    // tile bounds the launch, one without the branch to them (canyon
+    // quadtree, FP32C: 3.21 against 3.23)
+    if (V.depth == 1) go(step_kernel<P, true, true, true>);
+    else if (V.nv > 0 && V.patches) go(step_kernel<P, false, true, true>);
+    else if (V.nv > 0) go(step_kernel<P, false, true, false>);
+    else if (V.patches) go(step_kernel<P, false, false, true>);
+    else go(step_kernel<P, false, false, false>);
 }
 
 hipError_t launch_step(const DevView& V, int precision, int t0, int use_base, int k, hipStream_t st, int end)
@@ -1332,12 +1428,16 @@ hipError_t launch_state(int precision, const void* U, const int* node_int, const
 // budget (the most any layout may then need).
 hipError_t configure_kernels(size_t* max_lds)
 {
-    const void* fns[6] = {reinterpret_cast<const void*>(step_kernel<PF64, true, true>),
-                          reinterpret_cast<const void*>(step_kernel<PF32C, true, true>),
-                          reinterpret_cast<const void*>(step_kernel<PF64, false, true>),
-                          reinterpret_cast<const void*>(step_kernel<PF32C, false, true>),
-                          reinterpret_cast<const void*>(step_kernel<PF64, false, false>),
-                          reinterpret_cast<const void*>(step_kernel<PF32C, false, false>)};
+    const void* fns[] = {reinterpret_cast<const void*>(step_kernel<PF64, true, true, true>),
+                         reinterpret_cast<const void*>(step_kernel<PF64, false, true, true>),
+                         reinterpret_cast<const void*>(step_kernel<PF64, false, true, false>),
+                         reinterpret_cast<const void*>(step_kernel<PF64, false, false, true>),
+                         reinterpret_cast<const void*>(step_kernel<PF64, false, false, false>),
+                         reinterpret_cast<const void*>(step_kernel<PF32C, true, true, true>),
+                         reinterpret_cast<const void*>(step_kernel<PF32C, false, true, true>),
+                         reinterpret_cast<const void*>(step_kernel<PF32C, false, true, false>),
+                         reinterpret_cast<const void*>(step_kernel<PF32C, false, false, true>),
+                         reinterpret_cast<const void*>(step_kernel<PF32C, false, false, false>)};
     size_t budget = *max_lds;
     for (const void* f : fns) {
         hipFuncAttributes a{};

@@ -161,9 +161,10 @@ int dmp_export_mesh(void *h, int *eptr, int *eind, bool *ediv, int *hanging, int
 /* Launch parameters (4 ints).  tuning[0] = nodes per tile on average (32..1024;
  * each workgroup owns one of ceil(nodes / tuning[0]) tiles; with several steps
  * per launch and at most two tiles per compute unit the tiles are cut at equal
- * work, so tiles holding hanging-node anchors are smaller; with one step per
- * launch 8 x 8 patches of uniform parts of the mesh are cut out first), tuning[1] = XCD-aware tile remap (0/1), tuning[2] = steps
- * per captured hipGraph (0 = eager launches), tuning[3] = time steps one
+ * work, so tiles holding hanging-node anchors are smaller; uniform parts of the
+ * mesh are cut out first, as patches of 8 x 8 nodes with one step per launch and
+ * of 16 x 16 with several and more tiles than compute units), tuning[1] =
+ * XCD-aware tile remap (0/1), tuning[2] = steps per captured hipGraph (0 = eager launches), tuning[3] = time steps one
  * launch advances (1..8; each tile then carries that many rings of
  * neighbours in LDS).  dmp_init starts from {256, 1, 60, 3} ({256, 1, 60, 1}
  * above 200,000 nodes), falling back to smaller shapes where the mesh needs
@@ -178,8 +179,8 @@ int dmp_get_tuning(void *h, int *tuning);
 
 /* Times the candidate launch shapes (nodes per tile 64/128/256 and the sizes
  * giving one or two tiles per compute unit, 1, 2, 3, 4, 6 or 8 steps per
- * launch -- 1 or 2 when the layout has more than 2 x 256 nodes per compute
- * unit --, XCD remap on/off, eager launches or graphs of min(*nsteps, 60)
+ * launch -- 1 to 4 when the layout has more than 2 x 256 nodes per compute
+ * unit, 1 or 2 above 6 x 256 --, XCD remap on/off, eager launches or graphs of min(*nsteps, 60)
  * steps in whole launches) on this instance for *nsteps steps each, once to
  * warm up, then timed until there are two runs and 2 ms of them (at most 15)
  * (state is restored afterwards), and keeps the shape with the shortest lower

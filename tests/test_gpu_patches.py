@@ -110,3 +110,36 @@ def test_whole_mesh_in_one_tile(name, prec):
             assert np.array_equal(np.concatenate(parts), want[0])
             for a, b in zip(got, want[1]):
                 assert np.array_equal(a, b)
+
+
+# more tiles than compute units (32 nodes each): 16 x 16 patches with 2 to 8
+# rings, uniform and with moduli per element, and in a mesh with hanging nodes
+@pytest.mark.parametrize("name", ["layer", "layer_het", "basin"])
+@pytest.mark.parametrize("prec", [0, 1])
+def test_block_patches(name, prec):
+    from damian_hip import cases, lib
+    import oracle_ctypes as O
+    case = cases.c4_valley(62.0, "SV", 10.0) if name == "basin" else layer(cases, 143, 77, name == "layer_het")
+    n = 61
+    ref = lib.Solver(case, precision=prec)
+    ref.set_tuning(128, 1, 0, 3)   # fewer tiles than compute units: no patches
+    ref.run(400 if name == "basin" else 60)
+    want = (ref.run(n),) + ref.state()[:2]
+    ref.close()
+    assert np.abs(want[1]).max() > 1e-3
+    if name == "layer_het":
+        u_o, _, _, rec_o = O.run(case, nsteps=60 + n, recv_interval=1)
+        assert rel_l2(want[0], rec_o[61:]) <= TOL[prec]
+    for tuning in ((32, 0, 0, 2), (32, 1, 12, 3), (33, 1, 0, 4), (40, 1, 0, 5), (32, 1, 0, 8)):
+        print(f"name={name} prec={prec} tuning={tuning}", flush=True)
+        s = lib.Solver(case, precision=prec)
+        try:
+            s.set_tuning(*tuning)
+        except lib.DmpError as e:   # hanging nodes widen the rings of deep launches
+            assert name == "basin" and tuning[3] > 4 and e.code == -4
+            continue
+        s.run(400 if name == "basin" else 60)
+        got = (s.run(n),) + s.state()[:2]
+        s.close()
+        for a, b in zip(got, want):
+            assert np.array_equal(a, b)
