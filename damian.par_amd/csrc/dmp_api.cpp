@@ -59,6 +59,15 @@ constexpr double kAnchorWeight = 5.0;
 constexpr int kTuneMaxRuns = 15;
 constexpr double kTuneMinSeconds = 2e-3;
 
+// One-step layouts: nodes per tile outside patches (at most), and wavefronts
+// per workgroup.  A workgroup's LDS is what the larger of a tile and four
+// patches needs: tiles of 64 nodes need no more than the patches, so that these
+// fill the compute units (2.47M-element sweep, FP32C, tiles of 32, 64, 128 and
+// 256 nodes: 26.4, 24.2, 30.8 and 28.7 us a step).  One and two wavefronts: 25.5
+// and 25.5 (the uniform canyon 11.1 and 10.6 against 10.8 with four).
+constexpr int kRestBlock = 64;
+constexpr int kPatchWaves = 4;
+
 // Steps per launch of a mesh that one workgroup holds whole (build_tiles).
 constexpr int kWholeSteps = 32;
 
@@ -222,6 +231,9 @@ struct LocalLayout {
     std::vector<std::array<int, 2>> seis;      // (internal elem, kind) in input order
     std::vector<double> lm;                    // (lambda, mu) per material entry
     std::vector<int> emat;
+    // per active node with four elements of one size: its column and row on
+    // that size's grid, and the size in units of the smallest (0: no such node)
+    std::vector<std::array<int, 3>> grid;
     std::vector<double> invm;                  // per active node (regular) or 0
     std::vector<int> side_of;                  // per active node: side index or -1
     std::vector<HostSide> side;
@@ -240,6 +252,8 @@ struct PackedHost {
     std::vector<int4> node_elems, vnode_elems, elem_corners;
     std::vector<int> elem_mat;
     std::vector<int2> vanch;
+    std::vector<std::array<int, 3>> grid;   // LocalLayout::grid
+    std::vector<int> inst_base;      // first active node of each instance
     std::vector<int> node_side;      // HostSide index, or -1 for a plain node
     std::vector<double> invm;        // plain nodes: 1 / e_mfull
     std::vector<HostSide> side;      // drm = global pair first
@@ -638,6 +652,19 @@ void build_local(Instance& I)
         }
     }
 
+    L.grid.assign(L.na, {0, 0, 0});
+    for (int a = 0; a < L.na; ++a) {
+        const auto& q = L.node_elems[a];
+        if (q[0] < 0 || q[1] < 0 || q[2] < 0 || q[3] < 0) continue;
+        const double s = h[L.elem_orig[q[0]]];
+        bool one = true;
+        for (int k = 1; k < 4; ++k) one = one && std::fabs(h[L.elem_orig[q[k]]] - s) <= 1e-6 * s;
+        if (!one) continue;
+        const double* x = &I.nodes[2 * L.act_orig[a]];
+        L.grid[a] = {(int)std::llround((x[0] - xmin) / s), (int)std::llround((x[1] - zmin) / s),
+                     (int)std::min<long long>(std::llround(s / hmin), 1 << 30)};
+    }
+
     // ---- materials
     const bool per_elem = !I.eprops.empty();
     std::vector<std::array<double, 5>> emc(ne);
@@ -936,7 +963,155 @@ struct TileScratch {
     }
 };
 
-// Runs of M x M nodes that form a patch (PatchT) for launches of up to D steps,
+// Nodes of the plain formula with four elements that have no hanging corner and
+// agree on the node's eight neighbours.
+std::vector<char> plain_nodes(const PackedHost& H, int NA)
+{
+    std::vector<char> plain(NA, 0);
+    const int nblk = std::max(1, std::min(256, NA / 4096 + 1));
+    parallel_items(nblk, setup_threads(), [&](int b) {
+        for (int n = (int)((long)NA * b / nblk); n < (int)((long)NA * (b + 1) / nblk); ++n) {
+            const int4 q = H.node_elems[n];
+            if (H.node_side[n] >= 0 || q.x < 0 || q.y < 0 || q.z < 0 || q.w < 0) continue;
+            const int4 a = H.elem_corners[q.x], c = H.elem_corners[q.y], d = H.elem_corners[q.z],
+                       e = H.elem_corners[q.w];
+            bool ok = c.x == d.w && a.y == e.z && a.w == c.z && d.y == e.x;
+            for (const int4& k : {a, c, d, e}) ok = ok && std::max(std::max(k.x, k.y), std::max(k.z, k.w)) < NA;
+            plain[n] = ok;
+        }
+    });
+    return plain;
+}
+
+// The eight neighbours of a plain node, as (offset in an image of pitch W,
+// node) pairs.
+std::array<std::array<int, 2>, 8> grid_neighbours(const PackedHost& H, int n, int W)
+{
+    const int4 q = H.node_elems[n];
+    const int4 a = H.elem_corners[q.x], c = H.elem_corners[q.y], d = H.elem_corners[q.z], e = H.elem_corners[q.w];
+    return {{{W, a.y}, {W + 1, a.z}, {1, a.w}, {-W, c.x}, {-W + 1, c.w}, {-W - 1, d.x}, {-1, d.y}, {W - 1, e.y}}};
+}
+
+// One-step layouts: the patches (PatchT), and the nodes left to the tiles.
+// Plain nodes are gathered by the cell of kPatch x kPatch places that the
+// mesh's own grid gives them (consecutive among the nodes of one element size
+// along the Morton order); a cell is a patch where the neighbours of each of
+// its nodes are those that its place says.  `taken` marks nodes that tiles
+// need (the corners by which receivers are given to tiles).
+struct PatchCells {
+    std::vector<PatchT> patch;
+    std::vector<int> ring, list;   // kPatchRing per patch, kPatchNodes per listed one
+    std::vector<int> rest;
+};
+
+PatchCells find_cells(const PackedHost& H, int NA, const std::vector<char>& taken)
+{
+    constexpr int M = kPatch, W = M + 2;
+    const std::vector<char> plain = plain_nodes(H, NA);
+    std::vector<int> cell_of(NA, -1);
+    int nc = 0;
+    {
+        struct Open {
+            int size, x, z, cell;
+        };
+        std::vector<Open> open;   // per element size the cell that the order is in
+        size_t inst = 0;
+        for (int n = 0; n < NA; ++n) {
+            while (inst < H.inst_base.size() && n >= H.inst_base[inst]) {
+                open.clear();
+                ++inst;
+            }
+            const auto& g = H.grid[n];
+            if (!plain[n] || taken[n] || g[2] == 0) continue;
+            auto o = std::find_if(open.begin(), open.end(), [&](const Open& q) { return q.size == g[2]; });
+            if (o == open.end()) o = open.insert(o, Open{g[2], -1, -1, -1});
+            if (o->x != g[0] / M || o->z != g[1] / M || o->cell < 0) *o = Open{g[2], g[0] / M, g[1] / M, nc++};
+            cell_of[n] = o->cell;
+        }
+    }
+    std::vector<int> first(nc + 1, 0), member;
+    for (int n = 0; n < NA; ++n)
+        if (cell_of[n] >= 0) ++first[cell_of[n] + 1];
+    for (int c = 0; c < nc; ++c) first[c + 1] += first[c];
+    member.resize(first[nc]);
+    {
+        std::vector<int> at(first.begin(), first.end() - 1);
+        for (int n = 0; n < NA; ++n)
+            if (cell_of[n] >= 0) member[at[cell_of[n]]++] = n;
+    }
+    // per cell: the patch (list >= 0: a part of a cell), its ring and places
+    std::vector<char> good(nc, 0);
+    std::vector<PatchT> patch(nc);
+    std::vector<int> ring((size_t)nc * kPatchRing), place((size_t)nc * kPatchNodes);
+    const int nblk = std::max(1, std::min(256, nc / 256 + 1));
+    parallel_items(nblk, setup_threads(), [&](int b) {
+        for (int c = (int)((long)nc * b / nblk); c < (int)((long)nc * (b + 1) / nblk); ++c) {
+            const int lo = first[c], hi = first[c + 1];
+            if (hi - lo < kPatchFew) continue;
+            int img[W * W];
+            std::fill(img, img + W * W, -1);
+            bool ok = true;
+            auto put = [&](int p, int n) {
+                if (img[p] < 0) img[p] = n;
+                ok = ok && img[p] == n;
+            };
+            auto pos = [&](int n) { return (H.grid[n][0] % M + 1) * W + H.grid[n][1] % M + 1; };
+            for (int i = lo; ok && i < hi; ++i) {
+                put(pos(member[i]), member[i]);
+                for (const auto& k : grid_neighbours(H, member[i], W)) put(pos(member[i]) + k[0], k[1]);
+            }
+            if (!ok) continue;
+            PatchT& P = patch[c];
+            P = PatchT{};
+            const int m0 = member[lo];
+            P.lam = H.node_em[2 * (size_t)m0];
+            P.mu = H.node_em[2 * (size_t)m0 + 1];
+            P.invm = H.invm[m0];
+            for (int i = lo; i < hi; ++i) {
+                if (H.invm[member[i]] != P.invm) P.coefs = 1;
+                for (int d : {0, -1, -W, -W - 1}) {   // corners 0 of the node's elements
+                    const size_t n = img[pos(member[i]) + d];
+                    if (H.node_em[2 * n] != P.lam || H.node_em[2 * n + 1] != P.mu) P.hetero = 1;
+                }
+            }
+            int* w = &place[(size_t)c * kPatchNodes];
+            bool whole = hi - lo == kPatchNodes;
+            for (int m = 0; m < kPatchNodes; ++m) {
+                int x = 0, z = 0;
+                for (int b2 = 0; (1 << (2 * b2)) < kPatchNodes; ++b2) {
+                    z |= ((m >> (2 * b2)) & 1) << b2;
+                    x |= ((m >> (2 * b2 + 1)) & 1) << b2;
+                }
+                const int n = img[(x + 1) * W + z + 1];
+                w[m] = n < 0 ? -1 : cell_of[n] == c ? n : n | kPrevFlag;
+                whole = whole && n == m0 + m;
+            }
+            P.n0 = whole ? m0 : -1;
+            P.list = whole ? -1 : 0;
+            int* r = &ring[(size_t)c * kPatchRing];
+            for (int z = 0; z <= M; ++z) *r++ = img[z];                       // x = -1
+            for (int x = 1; x <= M; ++x) *r++ = img[x * W];                   // z = -1
+            for (int x = 0; x <= M; ++x) *r++ = img[x * W + M + 1];           // z = M
+            for (int z = 0; z <= M + 1; ++z) *r++ = img[(M + 1) * W + z];     // x = M
+            good[c] = 1;
+        }
+    });
+    PatchCells out;
+    for (int c = 0; c < nc; ++c) {
+        if (!good[c]) continue;
+        if (patch[c].list >= 0) {
+            patch[c].list = (int)(out.list.size() / kPatchNodes);
+            out.list.insert(out.list.end(), &place[(size_t)c * kPatchNodes], &place[(size_t)(c + 1) * kPatchNodes]);
+        }
+        out.patch.push_back(patch[c]);
+        out.ring.insert(out.ring.end(), &ring[(size_t)c * kPatchRing], &ring[(size_t)(c + 1) * kPatchRing]);
+    }
+    for (int n = 0; n < NA; ++n)
+        if (cell_of[n] < 0 || !good[cell_of[n]]) out.rest.push_back(n);
+    return out;
+}
+
+// Runs of M x M nodes that form a block patch for launches of up to D steps,
 // as start nodes in ascending order, with the nodes of the rings around each.
 // A run is a patch where its nodes are an aligned cell of the Morton order of
 // a uniform part of the mesh: every node that a launch updates for it (the run
@@ -955,20 +1130,8 @@ PatchRuns find_patches(const PackedHost& H, int NA, const std::vector<char>& tak
     const int W = M + 2 * D, N = M * M;
     PatchRuns out;
     out.nodes = N;
-    // nodes of the plain formula whose four elements agree on their neighbours
-    std::vector<char> plain(NA, 0);
-    auto corners = [&](int e) { return H.elem_corners[e]; };
+    const std::vector<char> plain = plain_nodes(H, NA);
     const int nblk = std::max(1, std::min(256, NA / 4096 + 1)), nth = setup_threads();
-    parallel_items(nblk, nth, [&](int b) {
-        for (int n = (int)((long)NA * b / nblk); n < (int)((long)NA * (b + 1) / nblk); ++n) {
-            const int4 q = H.node_elems[n];
-            if (H.node_side[n] >= 0 || q.x < 0 || q.y < 0 || q.z < 0 || q.w < 0) continue;
-            const int4 a = corners(q.x), c = corners(q.y), d = corners(q.z), e = corners(q.w);
-            bool ok = c.x == d.w && a.y == e.z && a.w == c.z && d.y == e.x;
-            for (const int4& k : {a, c, d, e}) ok = ok && std::max(std::max(k.x, k.y), std::max(k.z, k.w)) < NA;
-            plain[n] = ok;
-        }
-    });
     // place of node m of a run, and the positions of ring r >= 1 (of the square
     // with r rings less that with r - 1), in the (M + 2 D)^2 image
     std::vector<int> place(N);
@@ -992,11 +1155,7 @@ PatchRuns find_patches(const PackedHost& H, int NA, const std::vector<char>& tak
         for (size_t i = 0; i < order.size(); ++i) {
             const int at = order[i], n = img[at];
             if (n < 0 || !plain[n] || (i < (size_t)N && taken[n])) return false;
-            const int4 q = H.node_elems[n];
-            const int4 a = corners(q.x), c = corners(q.y), d = corners(q.z), e = corners(q.w);
-            const int nb[8][2] = {{W, a.y}, {W + 1, a.z}, {1, a.w}, {-W, c.x},
-                                  {-W + 1, c.w}, {-W - 1, d.x}, {-1, d.y}, {W - 1, e.y}};
-            for (const auto& k : nb) {
+            for (const auto& k : grid_neighbours(H, n, W)) {
                 int& p = img[at + k[0]];
                 if (p < 0) p = k[1];
                 if (p != k[1]) return false;
@@ -1025,17 +1184,10 @@ PatchRuns find_patches(const PackedHost& H, int NA, const std::vector<char>& tak
         for (int i = (int)((long)np * b / nb); i < (int)((long)np * (b + 1) / nb); ++i) {
             image(out.start[i], img);
             int* r = &out.ring[(size_t)i * len];
-            if (D == 1) {   // kPatchLow order
-                for (int z = 0; z <= M; ++z) *r++ = img[z];                       // x = -1
-                for (int x = 1; x <= M; ++x) *r++ = img[x * W];                   // z = -1
-                for (int x = 0; x <= M; ++x) *r++ = img[x * W + M + 1];           // z = M
-                for (int z = 0; z <= M + 1; ++z) *r++ = img[(M + 1) * W + z];     // x = M
-            } else {
-                for (int e = N; e < W * W; ++e) {
-                    int x, z;
-                    block_patch_xz(e, x, z);
-                    *r++ = img[(x + D) * W + z + D];
-                }
+            for (int e = N; e < W * W; ++e) {
+                int x, z;
+                block_patch_xz(e, x, z);
+                *r++ = img[(x + D) * W + z + D];
             }
         }
     });
@@ -1062,7 +1214,7 @@ void build_tiles(Runtime& R)
     // launch; the layer of 861 nodes 2.1 against 3.4 in FP64, 1.8 against 3.3
     // in FP32C.  Descriptors address no more slots.
     R.whole = K > 1 && NA <= kMaxSlots && (R.tuning[0] >= NA || R.own_shape) && !R.no_whole;
-    const int B = R.whole ? std::max(NA, 1) : R.tuning[0];
+    const int B = R.whole ? std::max(NA, 1) : K == 1 && !R.no_patches ? std::min(R.tuning[0], kRestBlock) : R.tuning[0];
     int ntiles = (NA + B - 1) / B;
     const int NR = (int)H.recv.size();
     const int NFF = (int)H.ff.size();
@@ -1083,15 +1235,30 @@ void build_tiles(Runtime& R)
     // Uniform parts of the mesh as patches: always at one step per launch; at
     // several where there are more tiles than compute units, so that work in
     // flight and not the slowest tile's latency bounds a launch.
+    // One step per launch: tiles of B nodes each of the list of nodes outside
+    // patches.
     PatchRuns patches;
-    if (!R.no_patches && (K == 1 || (ntiles > ncu && !R.whole))) {
+    PatchCells cells;
+    std::vector<int> gen_of(K == 1 ? NA : 0, -1);   // place of a node in that list
+    if (K == 1 || (ntiles > ncu && !R.whole)) {
         std::vector<char> taken(NA, 0);
         for (const RecvRec& x : H.recv) {
             const int c = x.c[0];
             if (c >= 0) taken[c < NA ? c : H.vanch[c - NA].x] = 1;
         }
-        patches = find_patches(H, NA, taken, K == 1 ? kPatch : kBlockPatch, K);
+        if (R.no_patches) {
+            if (K == 1) {
+                cells.rest.resize(NA);
+                std::iota(cells.rest.begin(), cells.rest.end(), 0);
+            }
+        } else if (K == 1) {
+            cells = find_cells(H, NA, taken);
+        } else {
+            patches = find_patches(H, NA, taken, kBlockPatch, K);
+        }
+        for (size_t i = 0; i < cells.rest.size(); ++i) gen_of[cells.rest[i]] = (int)i;
     }
+    const int NG = K == 1 ? (int)cells.rest.size() : NA;   // nodes that tiles have, or between patches
     // The runs of nodes between them as tiles.
     const bool equal_work = K > 1 && ntiles <= 2 * ncu;
     std::vector<double> cum(equal_work ? NA + 1 : 0, 0.0);
@@ -1103,7 +1270,7 @@ void build_tiles(Runtime& R)
     const double share = equal_work ? cum[NA] / ntiles : 0.0;
     std::vector<int> tstart, tend;
     for (size_t i = 0; i <= patches.start.size(); ++i) {
-        const int lo = i ? patches.start[i - 1] + patches.nodes : 0, hi = i < patches.start.size() ? patches.start[i] : NA;
+        const int lo = i ? patches.start[i - 1] + patches.nodes : 0, hi = i < patches.start.size() ? patches.start[i] : NG;
         if (lo >= hi) continue;
         if (!equal_work) {
             for (int n = lo; n < hi; n += B) {
@@ -1135,12 +1302,14 @@ void build_tiles(Runtime& R)
     std::vector<std::vector<int>> tile_recv(std::max(ntiles, 1));
     for (int r = 0; r < NR; ++r) {
         const int c = H.recv[r].c[0];
-        const int owner = c < 0 ? 0 : tile_of(c < NA ? c : H.vanch[c - NA].x);
+        const int node = c < 0 ? 0 : c < NA ? c : H.vanch[c - NA].x;
+        const int owner = c < 0 ? 0 : tile_of(K == 1 ? gen_of[node] : node);
         tile_recv[owner].push_back(r);
     }
 
-    std::vector<uint32_t> core_full(8 * (size_t)NA, 0);   // per node, written by its tile
-    std::vector<double> core_coef(NA, 0.0);
+    std::vector<uint32_t> core_full(8 * (size_t)NG, 0);   // per node, written by its tile
+    std::vector<double> core_coef(NG, 0.0);
+    auto core_node = [&](int i) { return K == 1 ? cells.rest[i] : i; };
 
     // one tile into part P (offsets local to P)
     auto build_one = [&](int t, TileScratch& S, TilePart& P) {
@@ -1166,7 +1335,7 @@ void build_tiles(Runtime& R)
         // ring 0: the core; ring 1: what the core reads, and the stored nodes
         // of the tile's receivers (sampled at sub-steps 0 .. k-1, while ring 1
         // is still exact); ring j+1: what ring j reads
-        for (int i = 0; i < cnt; ++i) add_ent(n0 + i);
+        for (int i = 0; i < cnt; ++i) add_ent(core_node(n0 + i));
         T.lev_end[0] = (int)ent.size();
         size_t lo = 0;
         for (int j = 1; j <= kMaxDepth; ++j) {
@@ -1358,8 +1527,8 @@ void build_tiles(Runtime& R)
             return -(double)(P.sides.size() - T.side_off);   // -(tile-local index + 1)
         };
         for (int i = 0; i < cnt; ++i) {
-            pack(H.node_elems[n0 + i], &core_full[8 * (size_t)(n0 + i)]);
-            core_coef[n0 + i] = coef_of(n0 + i);
+            pack(H.node_elems[core_node(n0 + i)], &core_full[8 * (size_t)(n0 + i)]);
+            core_coef[n0 + i] = coef_of(core_node(n0 + i));
         }
         T.n_ent = N;
         T.ring_off = (int)P.ring_gid.size();
@@ -1544,7 +1713,7 @@ void build_tiles(Runtime& R)
         *out = make_uint4(to_word(full, 0, mode), to_word(full, 1, mode), to_word(full, 2, mode),
                           to_word(full, 3, mode));
     };
-    std::vector<uint4> core_desc(NA), ring_desc(ring_gid.size());
+    std::vector<uint4> core_desc(NG), ring_desc(ring_gid.size());
     bool has_elem = false;
     for (const TileInfo& T : tiles) has_elem = has_elem || T.mat_mode;
     {
@@ -1612,7 +1781,8 @@ void build_tiles(Runtime& R)
         auto check_tile = [&](int t) {
             const TileInfo& T = tiles[t];
             const int cnt = T.cnt;
-            if (T.n0 != tstart[t] || cnt < 1 || T.n0 + cnt != tend[t] || tend[t] > NA || cnt > V.threads)
+            if (T.n0 != tstart[t] || cnt < 1 || T.n0 + cnt != tend[t] || tend[t] > NG || cnt > V.threads ||
+                (K == 1 && (T.n0 != t * B || cnt != std::min(B, NG - t * B))))
                 throw bad(t, "core range");
             const int nslots = T.n_ent + T.n_virt;
             if (T.n_ent < cnt || T.lev_end[K - 1] > V.threads || nslots > V.lds_slots || nslots > kMaxSlots)
@@ -1707,26 +1877,30 @@ void build_tiles(Runtime& R)
             for (int t = t0; t < t1; ++t) check_tile(t);
         });
     }
-    // patches: uniform moduli and mass term in the record where they are
+    // block patches: uniform moduli and mass term in the record where they are
     // uniform, else read per node
-    V.patches = (int)patches.start.size();
-    V.patch_hetero = 0;
+    V.patches = (int)(K == 1 ? cells.patch.size() : patches.start.size());
     if (K > 1 && V.patches) {   // a lane per entry that a launch updates
         const int w = block_patch_width(K) - 2;
         V.threads = std::max(V.threads, (w * w + 63) / 64 * 64);
         if (V.threads > kMaxThreads) throw fail(DMP_EUNSUPPORTED, "patches need %d threads (max %d)", V.threads, kMaxThreads);
     }
+    if (K == 1 && V.patches) V.threads = std::max(V.threads, 64 * kPatchWaves);
     const int per_block = K == 1 ? V.threads / 64 : 1;
     V.patch_blocks = (V.patches + per_block - 1) / per_block;
-    const int pn = patches.nodes, plen = V.patches ? (int)(patches.ring.size() / V.patches) : 0;
-    std::vector<PatchT> patch(V.patches);
-    {
+    std::vector<PatchT> patch = std::move(cells.patch);
+    const std::vector<int>& patch_ring = K == 1 ? cells.ring : patches.ring;
+    if (K > 1) {
+        patch.resize(V.patches);
+        const int pn = patches.nodes, plen = V.patches ? (int)(patches.ring.size() / V.patches) : 0;
+        const int updated = (block_patch_width(K) - 2) * (block_patch_width(K) - 2) - pn;
         const int nblk = std::max(1, std::min(V.patches, 16 * setup_threads()));
         parallel_items(nblk, setup_threads(), [&](int b) {
             for (int i = (int)((long)V.patches * b / nblk); i < (int)((long)V.patches * (b + 1) / nblk); ++i) {
                 PatchT& P = patch[i];
                 P = PatchT{};
                 P.n0 = patches.start[i];
+                P.list = -1;
                 if (P.n0 < 0 || P.n0 + pn > NA) throw fail(DMP_EINVAL, "internal: patch %d out of range", i);
                 const int* ring = &patches.ring[(size_t)i * plen];
                 P.lam = H.node_em[2 * (size_t)P.n0];
@@ -1743,20 +1917,34 @@ void build_tiles(Runtime& R)
                     mass(P.n0 + m);
                     core_coef[P.n0 + m] = H.invm[P.n0 + m];
                 }
-                const int updated = K == 1 ? 0 : (block_patch_width(K) - 2) * (block_patch_width(K) - 2) - pn;
                 for (int r = 0; r < plen; ++r) {
                     if (ring[r] < 0 || ring[r] >= NA) throw fail(DMP_EINVAL, "internal: patch %d: ring node out of range", i);
                     if (r < updated) mass(ring[r]);
                     // the outer ring: its nodes are corner 0 of elements that
                     // a launch reads at its lower x and z sides
-                    int x = 0, z = 0;
-                    if (K > 1) block_patch_xz(pn + r, x, z);
-                    if (K == 1 ? r < kPatchLow : r < updated || ((x < 0 || z < 0) && x < kBlockPatch + K - 1 && z < kBlockPatch + K - 1))
+                    int x, z;
+                    block_patch_xz(pn + r, x, z);
+                    if (r < updated || ((x < 0 || z < 0) && x < kBlockPatch + K - 1 && z < kBlockPatch + K - 1))
                         moduli(ring[r]);
                 }
             }
         });
-        for (const PatchT& P : patch) V.patch_hetero |= P.hetero;
+    } else {
+        for (int i = 0; i < V.patches; ++i) {
+            const PatchT& P = patch[i];
+            if (P.n0 >= 0 ? P.n0 + kPatchNodes > NA : P.list < 0 || (size_t)(P.list + 1) * kPatchNodes > cells.list.size())
+                throw fail(DMP_EINVAL, "internal: patch %d out of range", i);
+        }
+        for (int g : patch_ring)
+            if (g < -1 || g >= NA) throw fail(DMP_EINVAL, "internal: patch ring node out of range");
+        for (int g : cells.list)
+            if (g != -1 && (g & (kPrevFlag - 1)) >= NA) throw fail(DMP_EINVAL, "internal: patch node out of range");
+    }
+    V.patch_hetero = 0;
+    bool patch_coefs = false;
+    for (const PatchT& P : patch) {
+        V.patch_hetero |= P.hetero;
+        patch_coefs = patch_coefs || P.coefs;
     }
     if (R.whole) {
         const size_t fixed = step_lds_bytes(V, R.precision), per = sizeof(double2) * (V.lds_force + V.lds_recv);
@@ -1787,11 +1975,37 @@ void build_tiles(Runtime& R)
     if (lds > R.lds_limit)
         throw fail(DMP_EUNSUPPORTED, "tiles of %d nodes for %d steps per launch need %zu B of LDS "
                    "(limit %zu)", B, K, lds, R.lds_limit);
+    // lists at a fixed stride per tile: rows of the force table, free-field
+    // points of the receivers, and the ring entries of one-step layouts
+    if (NA >= kPrevFlag) throw fail(DMP_EUNSUPPORTED, "more than %d active nodes", kPrevFlag - 1);
+    {
+        std::vector<int> fs((size_t)ntiles * V.lds_force, -1), rf((size_t)ntiles * V.lds_recv, -1), rg;
+        V.ring_cap = 0;
+        if (K == 1)
+            for (const TileInfo& T : tiles) V.ring_cap = std::max(V.ring_cap, T.n_ent - T.cnt);
+        rg.assign((size_t)ntiles * V.ring_cap, -1);
+        for (int t = 0; t < ntiles; ++t) {
+            TileInfo& T = tiles[t];
+            for (int q = 0; q < T.n_force; ++q) fs[(size_t)t * V.lds_force + q] = force_slots[T.force_off + q];
+            T.force_off = t * V.lds_force;
+            for (int q = 0; q < T.n_recv; ++q) rf[(size_t)t * V.lds_recv + q] = recvs[T.recv_off + q].ff;
+            if (K == 1)
+                for (int e = T.cnt; e < T.n_ent; ++e)
+                    rg[(size_t)t * V.ring_cap + e - T.cnt] =
+                        ring_gid[T.ring_off + e - T.cnt] | (e < T.prv_end ? kPrevFlag : 0);
+        }
+        V.force_slots = R.upload_tile(fs);
+        V.recv_ff = R.upload_tile(rf);
+        V.ring_gid = R.upload_tile(rg);
+    }
+    V.block = B;
+    V.ngen = NG;
+    V.core_gid = K == 1 ? R.upload_tile(cells.rest) : nullptr;
     V.tiles = R.upload_tile(tiles);
     V.patch = R.upload_tile(patch);
-    V.patch_ring = R.upload_tile(patches.ring);
+    V.patch_ring = R.upload_tile(patch_ring);
+    V.patch_list = R.upload_tile(cells.list);
     V.core_desc = R.upload_tile(core_desc);
-    V.ring_gid = R.upload_tile(ring_gid);
     V.elist = nullptr;
     V.elist_cap = 0;
     if (K > 1) {
@@ -1799,7 +2013,6 @@ void build_tiles(Runtime& R)
         // the bandwidth-bound one-step layouts keep the ring list instead)
         int cap = 1;
         for (const TileInfo& T : tiles) cap = std::max(cap, T.n_ent);
-        if (NA >= kPrevFlag) throw fail(DMP_EUNSUPPORTED, "more than %d active nodes", kPrevFlag - 1);
         std::vector<int> elist((size_t)ntiles * cap, -1);
         for (int t = 0; t < ntiles; ++t) {
             const TileInfo& T = tiles[t];
@@ -1819,6 +2032,16 @@ void build_tiles(Runtime& R)
         std::vector<float> c32(core_coef.begin(), core_coef.end()), r32(ring_coef.begin(), ring_coef.end());
         V.core_coef = R.upload_tile(c32);
         V.ring_coef = R.upload_tile(r32);
+    }
+    // mass terms of patch nodes by node: the tiles' own array where it is one
+    // value per active node
+    V.node_coef = K > 1 ? V.core_coef : nullptr;
+    if (K == 1 && patch_coefs) {
+        if (R.precision == DMP_FP64) {
+            V.node_coef = R.upload_tile(H.invm);
+        } else {
+            V.node_coef = R.upload_tile(std::vector<float>(H.invm.begin(), H.invm.end()));
+        }
     }
     V.side = R.upload_tile(sides);
     V.vrows = R.upload_tile(vrows);
@@ -1846,7 +2069,6 @@ void build_tiles(Runtime& R)
             V.virt_em = R.upload_tile(v32);
         }
     }
-    V.force_slots = R.upload_tile(force_slots);
     V.recvs = R.upload_tile(recvs);
     // the two live state levels to where launches of this depth look for them
     // (buffers change places, nothing is copied)
@@ -1968,6 +2190,8 @@ void build_runtime(Runtime& R, const std::vector<Instance*>& insts)
     std::vector<FFNode> ffn(NF);
     std::vector<RecvRec> recv(NR);
     std::vector<InstParams> ip(ninst);
+    R.host.grid.resize(NA);
+    R.host.inst_base = R.inst_node_base;
     int mb = 0, sb = 0, tb = 0, deb = 0, fb = 0;
     for (int q = 0; q < ninst; ++q) {
         const LocalLayout& L = *insts[q]->L;
@@ -1979,6 +2203,7 @@ void build_runtime(Runtime& R, const std::vector<Instance*>& insts)
         for (int a = 0; a < L.na; ++a) {
             node_elems[nb + a] = e4(L.node_elems[a]);
             act_orig[nb + a] = L.act_orig[a];
+            R.host.grid[nb + a] = L.grid[a];
             invm[nb + a] = L.invm[a];
             node_side[nb + a] = L.side_of[a] < 0 ? -1 : sb + L.side_of[a];
         }

@@ -110,16 +110,17 @@ struct DrmElem {
 // bits 30-31; a tile with more (mat_mode 1) reads an element's (lambda, mu)
 // from LDS at the slot of the element's corner 0, loaded per slot from
 // node_em / virt_em.
-constexpr int kPrevFlag = 1 << 30;   // entry-list word: u_{t0-1} is read as well
+constexpr int kPrevFlag = 1 << 30;   // entry-list word: u_{t0-1} is read as well; patch_list: not updated
 
 struct TileInfo {
-    int n0, cnt;                 // core: active nodes n0 .. n0 + cnt - 1 (entries 0 .. cnt - 1)
+    int n0, cnt;                 // core: active nodes n0 .. n0 + cnt - 1 (entries 0 .. cnt - 1); one-step
+                                 // layouts: places n0 .. in core_gid
     int n_ent;                   // entries; those >= cnt are ring entries
     int ring_off;                // ring entries in ring_gid / ring_desc / ring_coef
     int lev_end[kMaxDepth + 1];  // entries in rings <= j
     int virt_off, n_virt;        // hanging nodes: anchor slots in virt
     int vrow_off, n_vrow;        // hanging nodes whose reactions the tile's anchors take
-    int force_off, n_force;      // forced nodes: rows of the force table in force_slots
+    int force_off, n_force;      // forced nodes: rows of the force table in force_slots (lds_force per tile)
     int recv_off, n_recv;        // receivers sampled by the tile
     int side_off, n_side;        // SideT of the tile's entries (coef = -(index - side_off + 1))
     int mat_off, n_mat;          // materials of the rows the tile evaluates (host bookkeeping)
@@ -128,13 +129,19 @@ struct TileInfo {
     int pad[3];
 };
 
-// One-step layouts: a patch of kPatch x kPatch nodes of a uniform part of the
-// mesh, one wavefront's work.  Its nodes are an aligned cell of the Morton
-// order, n0 + m for the node whose x and z bits interleave to m (z in the even
-// bits); each has four elements, none with a hanging corner, and needs the
-// plain update only (no side record), and the tile samples no receiver.  The
-// neighbours of a node then sit at fixed distances from it in the patch and no
-// descriptor is needed.
+// One-step layouts: a patch of kPatch x kPatch places of a uniform part of the
+// mesh, one wavefront's work, one place per lane: lane m has the place whose x
+// and z bits interleave to m (z in the even bits), an aligned cell of the
+// Morton order.  The nodes at those places that have four elements, none with
+// a hanging corner, need the plain update only (no side record) and give no
+// receiver to a tile are the patch's; a whole cell of them is nodes n0 + m, a
+// part of one is listed.  A node's neighbours then sit at fixed distances from
+// it in the patch, and neither a descriptor (16 B) nor, where uniform, a mass
+// term is read.  8 x 8 against 16 x 16 (four nodes per lane), whole cells only,
+// on the uniform canyon: 10.9 against 11.4 us a step in FP32C, 12.0 against
+// 12.5 in FP64; the smaller patch fits more of the mesh (97 against 93 % of its
+// nodes) and overlaps loads and arithmetic of more wavefronts, which outweighs
+// its longer ring.
 constexpr int kPatch = 8;
 constexpr int kPatchNodes = kPatch * kPatch;
 constexpr int kPatchRing = 4 * kPatch + 4;
@@ -146,6 +153,10 @@ constexpr int kPatchSlots = (kPatch + 2) * kPatchPitch;
 // Ring order: x = -1 and then z = -1 (the corners 0 of the elements at the
 // patch's lower x and z sides, whose moduli are read), then the rest.
 constexpr int kPatchLow = 2 * kPatch + 1;
+// A cell with fewer nodes than this leaves them to the tiles: a wavefront costs
+// the same however many of its lanes have a node, and a tile about four times
+// as much per node.
+constexpr int kPatchFew = 16;
 
 // Layouts of several steps per launch: a block patch of kBlockPatch x
 // kBlockPatch nodes, a Morton cell likewise, is one workgroup's work, with the
@@ -180,10 +191,11 @@ __host__ __device__ inline int block_patch_width(int depth) { return kBlockPatch
 __host__ __device__ inline int block_patch_pitch(int depth) { return (block_patch_width(depth) + 3) / 8 * 8 + 4; }
 
 struct PatchT {
-    int n0;
+    int n0;              // first node of a whole cell, or -1
     int hetero;          // 1: (lambda, mu) per element from node_em, 0: lam, mu
-    int coefs;           // 1: 1 / e_mfull per node from core_coef, 0: invm
-    int pad;
+    int coefs;           // 1: 1 / e_mfull per node from node_coef, 0: invm
+    int list;            // part of a cell: its places in patch_list (node, with kPrevFlag where the
+                         // patch only reads it, -1 where there is none)
     double lam, mu, invm;
     double pad2;
 };
@@ -275,9 +287,9 @@ struct DevView {
     const void* node_em;      // per active node: (lambda, mu) of the element whose corner 0 it is
     const void* virt_em;      // per entry of the tiles' hanging-node lists: the same
     const TileInfo* tiles;
-    const uint4* core_desc;   // per active node
-    const void* core_coef;    // per active node: 1/mfull, or -(tile side + 1)
-    const int* ring_gid;      // ring entries (one-step layouts)
+    const uint4* core_desc;   // per node of the tiles (TileInfo::n0 onwards)
+    const void* core_coef;    // the same: 1/mfull, or -(tile side + 1)
+    const int* ring_gid;      // one-step layouts: ring entries, ring_cap per tile (as elist)
     // several steps per launch: every entry of a tile, at a fixed stride (so
     // the loads need not wait for the tile record): node | kPrevFlag when
     // u_{t0-1} is read too, -1 past the tile's last entry
@@ -316,7 +328,16 @@ struct DevView {
     int patch_blocks;    // workgroups
     int patch_blocks_per_xcd;
     const PatchT* patch;
-    const int* patch_ring;    // per patch the nodes around it: kPatchRing, or the block patch's ring entries
+    const int* patch_ring;    // per patch the nodes around it: kPatchRing (-1: none there), or the block patch's ring entries
+    const int* patch_list;    // kPatchNodes per listed patch
+    const void* node_coef;    // per active node: 1 / mfull (plain nodes)
+    // one-step layouts: tiles are `block` nodes each of a list of the nodes
+    // outside patches; what a tile loads is at a fixed stride per tile, so that
+    // no load waits for the tile record to know its address
+    const int* core_gid;
+    int block, ngen;          // nodes per tile, nodes in the list
+    int ring_cap;
+    const int* recv_ff;       // lds_recv per tile: free-field point of its receivers, or -1
 };
 
 } // namespace dmp

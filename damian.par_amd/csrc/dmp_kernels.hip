@@ -661,8 +661,12 @@ __host__ __device__ inline int patch_lds_bytes(const DevView& V, int real_bytes)
 // spends some 100 more instructions on decoding descriptors and on the 12
 // corner reads that are 8 here, all at fixed offsets from one LDS address; and
 // a wavefront on its own needs no barrier.  The uniform 944,492-element canyon
-// takes 10.9 us a step in FP32C (4.2 TB/s of those 48 B) against 16.0 with
-// tiles only, and 12.0 against 17.2 in FP64.
+// takes 10.6 us a step in FP32C (4.3 TB/s of those 48 B) against 16.0 with
+// tiles only, and 11.6 against 17.2 in FP64.  Parts of cells count where much
+// of a mesh lies along sides, source layers and refinement fronts: whole cells
+// only leave 10 % of a basin's nodes to small tiles that take as long as the
+// rest, parts of cells 3 % (2.47M-element sweep, FP32C: 24.2 us a step against
+// 28.8, tiles only 37.5; FP64 28.0, 33.0 and 43.7).
 // ---------------------------------------------------------------------------
 // Ring position r (kPatchRing of them) in the patch's LDS image.
 __device__ __forceinline__ int patch_ring_slot(int r)
@@ -715,51 +719,39 @@ __device__ __forceinline__ void patch_step(const DevView& V, int t, const void* 
     node_t* val = reinterpret_cast<node_t*>(lds);
     V2<R>* em = reinterpret_cast<V2<R>*>(val + kPatchSlots);
     const PatchT T = uniform_record(V.patch + t);
-    const int* ring = V.patch_ring + (size_t)t * kPatchRing;
-    const int g0 = lane < kPatchRing ? ring[lane] : T.n0;
-    int g1 = 0;
-    if (lane < kPatchRing - 64) g1 = ring[64 + lane];
-    // node m = 64 q + lane: the lane's six bits are its place in an 8 x 8
-    // block, q the block (bit 0: z, bit 1: x)
+    static_assert(Q == 1 && kPatchRing <= 64, "a place and a ring node per lane");
+    const int gr = lane < kPatchRing ? V.patch_ring[(size_t)t * kPatchRing + lane] : -1;
+    const int w = T.n0 >= 0 ? T.n0 + lane : V.patch_list[(size_t)T.list * kPatchNodes + lane];
+    const int g = w & (kPrevFlag - 1);
+    const bool held = w >= 0, own = held && !(w & kPrevFlag);
     const int x = ((lane >> 1) & 1) | ((lane >> 2) & 2) | ((lane >> 3) & 4);
     const int z = (lane & 1) | ((lane >> 1) & 2) | ((lane >> 2) & 4);
     const int at = (x + 1) * W + z + 1;
-    node_t u[Q], p[Q];
-#pragma unroll
-    for (int q = 0; q < Q; ++q) u[q] = P::ld(U0, T.n0 + 64 * q + lane);
-#pragma unroll
-    for (int q = 0; q < Q; ++q) p[q] = P::ld(Um, T.n0 + 64 * q + lane);
-    const node_t r0 = P::ld(U0, g0);
-    node_t r1{};
-    if (lane < kPatchRing - 64) r1 = P::ld(U0, g1);
-    if (T.hetero) {
-        V2<R> e[Q];
-#pragma unroll
-        for (int q = 0; q < Q; ++q) e[q] = P::lm(V.node_em, T.n0 + 64 * q + lane);
-        V2<R> er{0, 0};
-        if (lane < kPatchLow) er = P::lm(V.node_em, g0);
-#pragma unroll
-        for (int q = 0; q < Q; ++q) em[at + (q >> 1) * 8 * W + (q & 1) * 8] = e[q];
-        if (lane < kPatchLow) em[patch_ring_slot(lane)] = er;
+    node_t un{}, up{}, ur{};
+    R cf = R(T.invm);
+    if (held) un = P::ld(U0, g);
+    if (own) {
+        up = P::ld(Um, g);
+        if (T.coefs) cf = P::coef(V.node_coef, g);
     }
-#pragma unroll
-    for (int q = 0; q < Q; ++q) val[at + (q >> 1) * 8 * W + (q & 1) * 8] = u[q];
-    if (lane < kPatchRing) val[patch_ring_slot(lane)] = r0;
-    if (lane < kPatchRing - 64) val[patch_ring_slot(64 + lane)] = r1;
+    if (gr >= 0) ur = P::ld(U0, gr);
+    if (T.hetero) {
+        V2<R> e{0, 0}, er{0, 0};
+        if (held) e = P::lm(V.node_em, g);
+        if (gr >= 0 && lane < kPatchLow) er = P::lm(V.node_em, gr);
+        if (held) em[at] = e;
+        if (gr >= 0 && lane < kPatchLow) em[patch_ring_slot(lane)] = er;
+    }
+    if (held) val[at] = un;
+    if (gr >= 0) val[patch_ring_slot(lane)] = ur;
     // the wavefront reads what its own lanes wrote: LDS operations of a
     // wavefront complete in order, so only the compiler has to keep them so
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
     __builtin_amdgcn_wave_barrier();
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-#pragma unroll
-    for (int q = 0; q < Q; ++q) {
-        const node_t* c = val + at + (q >> 1) * 8 * W + (q & 1) * 8;
-        const V2<R>* m = em + at + (q >> 1) * 8 * W + (q & 1) * 8;
-        const node_t un = c[0];
-        const V2<R> f = grid_rows<P>(c, W, un, T, m);
-        const R cf = T.coefs ? P::coef(V.core_coef, T.n0 + 64 * q + lane) : R(T.invm);
-        P::st(Uk, T.n0 + 64 * q + lane, P::advance(un, p[q], over_mass(f, cf, cf)));
-    }
+    if (!own) return;
+    const V2<R> f = grid_rows<P>(val + at, W, un, T, em + at);
+    P::st(Uk, g, P::advance(un, up, over_mass(f, cf, cf)));
 }
 
 // ---------------------------------------------------------------------------
@@ -799,7 +791,7 @@ __device__ __forceinline__ void block_patch_steps(const DevView& V, int t, int k
     if (e < nu) {
         un = P::ld(U0, g);
         up = P::ld(Um, g);
-        if (T.coefs) cf = P::coef(V.core_coef, g);
+        if (T.coefs) cf = P::coef(V.node_coef, g);
     }
     if (o < ne) uo = P::ld(U0, go);
     int x, z;
@@ -848,7 +840,8 @@ __device__ void tile_steps(const DevView& V, int tile, int t0, int k, int end)
     const int NT = blockDim.x;
     const int tid = threadIdx.x;
     const TileInfo T = uniform_record(V.tiles + tile);
-    const int n0 = T.n0, cnt = T.cnt;
+    const int n0 = ONE ? tile * V.block : T.n0;
+    const int cnt = ONE ? min(V.block, V.ngen - n0) : T.cnt;
     const int n_virt = HANG ? T.n_virt : 0, n_vrow = HANG ? T.n_vrow : 0;
     const int S = V.lds_slots;
     const int D = ONE ? 1 : V.depth;
@@ -891,28 +884,35 @@ __device__ void tile_steps(const DevView& V, int tile, int t0, int k, int end)
     // values of every entry (the outer ring is read, never updated), and the
     // lane's entry, updated while it is inside the exact rings
     const int e = tid;
+    int gid = n0 + e;   // the lane's node
     RowsT rows{};
     R cf = 0;
     if (ONE) {
         // one step: only the core is updated (one entry per lane, the
-        // workgroup being at least as wide as the tile); its values,
-        // descriptor and coefficient are issued first, the ring entries
-        // after the tile record
+        // workgroup being at least as wide as the tile).  Two dependent
+        // round trips bring everything: node lists, descriptors, mass terms
+        // and the tile record, then values, side records and source terms.
+        constexpr int kNode = kPrevFlag - 1;
         node_t cu{}, cp{};
         uint4 d0{};
         if (e < cnt) {
-            cu = P::ld(U0, n0 + e);
-            cp = P::ld(Um, n0 + e);
+            gid = V.core_gid[n0 + e];
             d0 = V.core_desc[n0 + e];
             cf = P::coef(V.core_coef, n0 + e);
         }
-        for (int q = cnt + tid; q < T.n_ent; q += NT) {
-            const int gid = V.ring_gid[T.ring_off + q - cnt];
-            buf[q] = P::ld(U0, gid);
-            if (q < T.prv_end) buf[S + q] = P::ld(Um, gid);
-            if (elem) em[q] = P::lm(V.node_em, gid);
+        int w = tid < V.ring_cap ? V.ring_gid[(size_t)tile * V.ring_cap + tid] : -1;
+        if (e < cnt) {
+            cu = P::ld(U0, gid);
+            cp = P::ld(Um, gid);
         }
-        if (elem && e < cnt) em[e] = P::lm(V.node_em, n0 + e);
+        for (int q = tid; q < V.ring_cap; q += NT) {
+            if (q != tid) w = V.ring_gid[(size_t)tile * V.ring_cap + q];
+            if (w < 0) break;
+            buf[cnt + q] = P::ld(U0, w & kNode);
+            if (w & kPrevFlag) buf[S + cnt + q] = P::ld(Um, w & kNode);
+            if (elem) em[cnt + q] = P::lm(V.node_em, w & kNode);
+        }
+        if (elem && e < cnt) em[e] = P::lm(V.node_em, gid);
         if (e < cnt) {
             buf[e] = cu;
             buf[S + e] = cp;
@@ -978,21 +978,38 @@ __device__ void tile_steps(const DevView& V, int tile, int t0, int k, int end)
     }
     // forces of steps t0+1 .. t0+k and the receivers' free field of the steps
     // the launch samples, t0 .. t0+max(k,1)-1, from the tables
-    for (int q = copy_lane<ONE>(3 * 64); q < k * T.n_force; q += NT) {
-        const int s1 = q / T.n_force, f = q - s1 * T.n_force;
-        const int slot = V.force_slots[T.force_off + f];
-        frc[q] = V.ftab[(size_t)((t0 + s1 + 1) % V.chunk) * V.nforce + slot];
+    if (ONE) {
+        for (int q = tid; q < V.lds_force; q += NT) {
+            const int slot = V.force_slots[(size_t)tile * V.lds_force + q];
+            if (slot >= 0) frc[q] = V.ftab[(size_t)((t0 + 1) % V.chunk) * V.nforce + slot];
+        }
+    } else {
+        for (int q = copy_lane<ONE>(3 * 64); q < k * T.n_force; q += NT) {
+            const int s1 = q / T.n_force, f = q - s1 * T.n_force;
+            const int slot = V.force_slots[T.force_off + f];
+            frc[q] = V.ftab[(size_t)((t0 + s1 + 1) % V.chunk) * V.nforce + slot];
+        }
     }
     const int rlane = recv_lane<ONE>();
     // end (several-step layouts, k < depth): the launch also samples step
     // t0 + k, ring 1 being still exact after its k sub-steps
     const int srows = max(k, 1) + (!ONE && end ? 1 : 0);
-    for (int q = rlane; q < srows * T.n_recv; q += NT) {
-        const int s = q / T.n_recv, r = q - s * T.n_recv;
-        const int ff = V.recvs[T.recv_off + r].ff;
-        if (ff >= 0) {
-            const double4 g = V.fftab[(size_t)((t0 + s) % V.chunk) * V.nff + ff];
-            rff[q] = make_double2(g.x, g.y);
+    if (ONE) {
+        for (int q = rlane; q < V.lds_recv; q += NT) {
+            const int ff = V.recv_ff[(size_t)tile * V.lds_recv + q];
+            if (ff >= 0) {
+                const double4 g = V.fftab[(size_t)(t0 % V.chunk) * V.nff + ff];
+                rff[q] = make_double2(g.x, g.y);
+            }
+        }
+    } else {
+        for (int q = rlane; q < srows * T.n_recv; q += NT) {
+            const int s = q / T.n_recv, r = q - s * T.n_recv;
+            const int ff = V.recvs[T.recv_off + r].ff;
+            if (ff >= 0) {
+                const double4 g = V.fftab[(size_t)((t0 + s) % V.chunk) * V.nff + ff];
+                rff[q] = make_double2(g.x, g.y);
+            }
         }
     }
     // one step: the lane's side record goes to registers, issued before the
@@ -1154,7 +1171,7 @@ __device__ void tile_steps(const DevView& V, int tile, int t0, int k, int end)
             if (s < k || (!ONE && end)) nxt[e] = unew;
             // the core's u_{t0+k} is stored here only when no barrier follows
             // (a barrier would wait for the store); u_{t0+k-1} after the loop
-            if (s == k && e < cnt && (ONE || !end)) P::st(Uk, n0 + e, unew);
+            if (s == k && e < cnt && (ONE || !end)) P::st(Uk, gid, unew);
         }
         if (s == k) {
             if (!ONE && end) {
@@ -1172,8 +1189,8 @@ __device__ void tile_steps(const DevView& V, int tile, int t0, int k, int end)
     // after the last sub-step: cur holds u_{t0+k-1} and, with end, nxt holds
     // u_{t0+k} (no lane writes either after its last barrier)
     if (e < cnt) {
-        if (!ONE && end) P::st(Uk, n0 + e, nxt[e]);
-        if (k > 1) P::st(Uk1, n0 + e, cur[e]);
+        if (!ONE && end) P::st(Uk, gid, nxt[e]);
+        if (!ONE && k > 1) P::st(Uk1, gid, cur[e]);
     }
     flush_receivers(V, rff, rcv, n_recv, t0, srows, rlane);
 }

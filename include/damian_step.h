@@ -161,19 +161,20 @@ int dmp_export_mesh(void *h, int *eptr, int *eind, bool *ediv, int *hanging, int
 /* Launch parameters (4 ints).  tuning[0] = nodes per tile on average (32..1024;
  * each workgroup owns one of ceil(nodes / tuning[0]) tiles; with several steps
  * per launch and at most two tiles per compute unit the tiles are cut at equal
- * work, so tiles holding hanging-node anchors are smaller; uniform parts of the
- * mesh are cut out first, as patches of 8 x 8 nodes with one step per launch and
- * of 16 x 16 with several and more tiles than compute units), tuning[1] =
- * XCD-aware tile remap (0/1), tuning[2] = steps per captured hipGraph (0 = eager launches), tuning[3] = time steps one
- * launch advances (1..8; each tile then carries that many rings of
- * neighbours in LDS).  dmp_init starts from {256, 1, 60, 3} ({256, 1, 60, 1}
- * above 200,000 nodes), falling back to smaller shapes where the mesh needs
- * it; NULL restores that initial shape.  A mesh of at most 1023 nodes at this
- * initial shape, or with tuning[0] no less than its nodes and tuning[3] above 1,
- * is one tile, which takes up to 32 steps per launch.  The shape's graph is instantiated
- * here, so that no dmp_run pays for it.  A shape the mesh cannot use (LDS,
- * descriptor range) returns DMP_EUNSUPPORTED and leaves the previous shape in
- * place. */
+ * work, so tiles holding hanging-node anchors are smaller).  Uniform parts of
+ * the mesh are cut out first, as patches of 8 x 8 nodes with one step per
+ * launch (the tiles then hold at most 64 of the nodes between) and of 16 x 16
+ * with several and more tiles than compute units.  tuning[1] = XCD-aware tile
+ * remap (0/1), tuning[2] = steps per captured hipGraph (0 = eager launches),
+ * tuning[3] = time steps one launch advances (1..8; each tile then carries that
+ * many rings of neighbours in LDS).  dmp_init starts from {256, 1, 60, 3}
+ * ({256, 1, 60, 1} above 200,000 nodes), falling back to smaller shapes where
+ * the mesh needs it; NULL restores that initial shape.  A mesh of at most 1023
+ * nodes at this initial shape, or with tuning[0] no less than its nodes and
+ * tuning[3] above 1, is one tile, which takes up to 32 steps per launch.  The
+ * shape's graph is instantiated here, so that no dmp_run pays for it.  A shape
+ * the mesh cannot use (LDS, descriptor range) returns DMP_EUNSUPPORTED and
+ * leaves the previous shape in place. */
 int dmp_set_tuning(void *h, const int *tuning);
 int dmp_get_tuning(void *h, int *tuning);
 
