@@ -30,8 +30,8 @@
 
 namespace dmp {
 hipError_t launch_step(const DevView& V, int precision, int t0, int use_base, int k, hipStream_t st,
-                       int end = 0);
-hipError_t launch_recv(const DevView& V, int precision, int j, hipStream_t st);
+                       int end = 0, uint32_t call = 0);
+hipError_t launch_recv(const DevView& V, int precision, int j, uint32_t call, hipStream_t st);
 size_t step_lds_bytes(const DevView& V, int precision);
 hipError_t launch_state(int precision, const void* U, const int* node_int, const int2* vanch, int first, int n,
                         int base, int vbase, double2* out, hipStream_t st);
@@ -305,6 +305,11 @@ struct Runtime {
     std::vector<void*> tile_allocs;
     hipEvent_t ev0 = nullptr, ev1 = nullptr;
     float last_ms = 0.0f;          // device time of the last run (events on `stream`)
+    bool ms_pending = false;       // last_ms is still to be read off the events
+    // completion word of run calls (report_done), mapped host memory, and the
+    // number of the last call that used it
+    uint32_t* done = nullptr;
+    uint32_t calls = 0;
     double* scratch = nullptr;     // this device's receiver-sample scratch (allocation-free runs)
     // receiver samples: the kernels write them straight into a ring of
     // mapped pinned host memory (V.recv_buf is its device address); the host
@@ -350,6 +355,8 @@ struct Runtime {
         ev0 = ev1 = nullptr;
         for (hipEvent_t e : free_ev) (void)hipEventDestroy(e);
         free_ev.clear();
+        if (done) (void)hipHostFree(done);
+        done = nullptr;
         if (hstage) (void)hipHostFree(hstage);
         hstage = nullptr;
         hstage_cap = 0;
@@ -2485,6 +2492,14 @@ void build_runtime(Runtime& R, const std::vector<Instance*>& insts)
             }
         }
     }
+    {
+        void* p = nullptr;
+        HIPCHECK(hipHostMalloc(&p, sizeof(uint32_t), hipHostMallocMapped));
+        R.done = static_cast<uint32_t*>(p);
+        *R.done = 0;
+        HIPCHECK(hipHostGetDevicePointer(&p, R.done, 0));
+        V.done = static_cast<uint32_t*>(p);
+    }
     V.ctrl = R.dalloc<Ctrl>(1);
     HIPCHECK(hipMemset(V.ctrl, 0, sizeof(Ctrl)));
     R.dev_base = 0;
@@ -2667,6 +2682,22 @@ void wait_event(hipEvent_t e)
     HIPCHECK(st);
 }
 
+// Waits for the completion word of run call `call`; now and then for the event
+// behind it too, so that a failed kernel ends the wait.
+void wait_done(Runtime& R, uint32_t call, hipEvent_t e)
+{
+    for (;;) {
+        for (int i = 0; i < 4096; ++i) {
+            if (__atomic_load_n(R.done, __ATOMIC_ACQUIRE) == call) return;
+            __builtin_ia32_pause();
+        }
+        const hipError_t st = hipEventQuery(e);
+        if (st == hipErrorNotReady) continue;
+        HIPCHECK(st);
+        return;
+    }
+}
+
 hipEvent_t take_event(Runtime& R)
 {
     if (!R.free_ev.empty()) {
@@ -2772,12 +2803,15 @@ int run_steps(Runtime& R, int n, double* out)
     // the layout's depth samples it itself, otherwise a receivers-only kernel
     const bool end_sample = rec && (s + n) % I == 0 && (n > 0 || R.first_run);
     bool end_done = false;
+    uint32_t call = 0;
     while (done < n) {
         const int k = std::min(K, n - done);
         const int end = end_sample && done + k == n && k < V.depth ? 1 : 0;
         ensure_tables(R, s + done, s + done + k + end);
         before(last_sample(s + done, k + end));
-        HIPCHECK(launch_step(V, R.precision, s + done, 0, k, R.stream, end));
+        const bool recv_follows = end_sample && !end;
+        if (R.whole && done + k == n && !recv_follows) call = ++R.calls ? R.calls : ++R.calls;
+        HIPCHECK(launch_step(V, R.precision, s + done, 0, k, R.stream, end, call));
         done += k;
         after(last_sample(s + done, end) + 1);
         end_done = end_done || end;
@@ -2785,14 +2819,17 @@ int run_steps(Runtime& R, int n, double* out)
     if (end_sample && !end_done) {
         ensure_tables(R, s + n, s + n);
         before(q_hi);
-        HIPCHECK(launch_recv(V, R.precision, s + n, R.stream));
+        call = ++R.calls ? R.calls : ++R.calls;   // never 0
+        HIPCHECK(launch_recv(V, R.precision, s + n, call, R.stream));
         after(q_hi + 1);
     }
     HIPCHECK(hipEventRecord(R.ev1, R.stream));
     while (mhead < marks.size()) retire();   // copies overlap the launches still running
-    wait_event(R.ev1);
+    // a last kernel of one workgroup reports the end itself
+    if (call) wait_done(R, call, R.ev1);
+    else wait_event(R.ev1);
     if (stream_out) copy_out(q_hi + 1);
-    HIPCHECK(hipEventElapsedTime(&R.last_ms, R.ev0, R.ev1));
+    R.ms_pending = true;
     R.step = s + n;
     R.first_run = false;
     return (int)nsamp;
@@ -2840,7 +2877,7 @@ int run_steps_noalloc(Runtime& R, int n, double* out)
     }
     if (end_sample && !end_done) {
         ensure_tables(R, s + n, s + n);
-        HIPCHECK(launch_recv(V, R.precision, s + n, R.stream));
+        HIPCHECK(launch_recv(V, R.precision, s + n, 0, R.stream));
     }
     if (out && nsamp > 0) {
         const long cap = V.recv_cap;
@@ -2855,6 +2892,7 @@ int run_steps_noalloc(Runtime& R, int n, double* out)
     HIPCHECK(hipEventRecord(R.ev1, R.stream));
     HIPCHECK(hipEventSynchronize(R.ev1));
     HIPCHECK(hipEventElapsedTime(&R.last_ms, R.ev0, R.ev1));
+    R.ms_pending = false;
     // no kernel writes the samples of receivers in no element; the scratch
     // may hold another call's samples there
     if (out)
@@ -2951,6 +2989,17 @@ void fetch_states(Runtime& R, int q, int nnodes, double* u, double* up, const st
         }
     }
     pool.done = true;
+}
+
+// Device time of the last run call.
+float run_ms(Runtime& R)
+{
+    if (R.ms_pending) {
+        HIPCHECK(hipEventSynchronize(R.ev1));
+        HIPCHECK(hipEventElapsedTime(&R.last_ms, R.ev0, R.ev1));
+        R.ms_pending = false;
+    }
+    return R.last_ms;
 }
 
 template <class H> H* as(void* p) { return static_cast<H*>(p); }
@@ -3370,15 +3419,14 @@ int dmp_last_run_ms(void* h, float* ms)
     if (!h || !ms) return DMP_EINVAL;
     Instance* I = as<Instance>(h);
     if (!I->rt) return DMP_ESTATE;
-    *ms = I->rt->last_ms;
-    return DMP_OK;
+    return guarded(&I->err, [&] { *ms = run_ms(*I->rt); });
 }
 
 int dmp_batch_last_run_ms(void* b, float* ms)
 {
     if (!b || !ms) return DMP_EINVAL;
-    *ms = as<Batch>(b)->rt->last_ms;
-    return DMP_OK;
+    Batch* B = as<Batch>(b);
+    return guarded(&B->err, [&] { *ms = run_ms(*B->rt); });
 }
 
 int dmp_get_step(void* h, int* step)

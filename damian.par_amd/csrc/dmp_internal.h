@@ -338,6 +338,7 @@ struct DevView {
     int block, ngen;          // nodes per tile, nodes in the list
     int ring_cap;
     const int* recv_ff;       // lds_recv per tile: free-field point of its receivers, or -1
+    uint32_t* done;           // mapped host word: number of the last run call whose work is complete
 };
 
 } // namespace dmp

@@ -1195,21 +1195,40 @@ __device__ void tile_steps(const DevView& V, int tile, int t0, int k, int end)
     flush_receivers(V, rff, rcv, n_recv, t0, srows, rlane);
 }
 
+// Tells the host that run call `call` is complete: the last kernel of the
+// call, in one workgroup, once its own stores are out.  What earlier kernels
+// of the call stored (samples in mapped host memory) precedes this kernel in
+// the stream, so that the release at system scope, which is cumulative, orders
+// it before the word too; the host reads the word with acquire.  It sees it
+// before an event recorded after the kernel: one-step calls of the 861-node
+// layer 22.0 -> 19.4 us, 20-step calls of the canyon quadtree 83.4 -> 80.0.
+__device__ __forceinline__ void report_done(const DevView& V, uint32_t call)
+{
+    if (!call) return;
+    __threadfence_system();
+    __syncthreads();
+    if (threadIdx.x == 0) __hip_atomic_store(V.done, call, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+
+// What a layout consists of: tiles, tiles and patches, or one tile that holds
+// the whole mesh.
+enum class Parts { kTiles, kPatches, kWhole };
+
 // Advances every tile from step t0 = t0_arg (+ the graph base) by k steps and
 // samples the receivers at steps t0 .. t0 + k - 1 (and t0 + k when end is set,
 // which needs k < depth).  The one-step kernel is bandwidth-bound, so it is
 // compiled for as many waves per SIMD as its registers allow without spills
 // (FP32C 7 with 72 VGPRs; FP64 6); the deeper one is latency-bound and keeps
 // the registers a 1024-thread workgroup leaves (4 waves per SIMD).
-template <class P, bool ONE, bool HANG, bool PATCH>
+template <class P, bool ONE, bool HANG, Parts PARTS>
 __global__ __launch_bounds__(kMaxThreads) __attribute__((amdgpu_waves_per_eu(ONE ? P::kOneWaves : 4)))
-void step_kernel(DevView V, int t0_arg, int use_base, int k, int end)
+void step_kernel(DevView V, int t0_arg, int use_base, int k, int end, uint32_t call)
 {
     const int t0 = t0_arg + (use_base ? V.ctrl->base : 0);
     int b = blockIdx.x;
     // tiles first (the longer work), then the patches
     const int nb = V.xcd_remap ? 8 * V.tiles_per_xcd : V.node_tiles;
-    if (PATCH && b >= nb) {
+    if (PARTS == Parts::kPatches && b >= nb) {
         b -= nb;
         const int blk = V.xcd_remap ? (b & 7) * V.patch_blocks_per_xcd + (b >> 3) : b;
         extern __shared__ __align__(16) unsigned char smem[];
@@ -1229,36 +1248,38 @@ void step_kernel(DevView V, int t0_arg, int use_base, int k, int end)
     const int tile = V.xcd_remap ? (b & 7) * V.tiles_per_xcd + (b >> 3) : b;
     if (tile >= V.node_tiles) return;   // whole block exits together
     tile_steps<P, ONE, HANG>(V, tile, t0, k, end);
+    if (PARTS == Parts::kWhole) report_done(V, call);
 }
 
 // Receivers at step j (j % recv_interval == 0) straight from the state level
 // in HBM: the last step of a run call, which no step launch of the call
-// starts from.
+// starts from.  One workgroup; call: as report_done, or 0.
 template <class P>
-__global__ void recv_kernel(DevView V, int j)
+__global__ __launch_bounds__(kMaxThreads) void recv_kernel(DevView V, int j, uint32_t call)
 {
-    const int r = (int)(blockIdx.x * blockDim.x + threadIdx.x);
-    if (r >= V.nrecv) return;
-    const RecvG g = V.rg[r];
     const void* U = V.U[state_slot(j, V.depth)];
-    double fx = 0.0, fz = 0.0;
-    if (g.found) {
+    for (int r = (int)threadIdx.x; r < V.nrecv; r += (int)blockDim.x) {
+        const RecvG g = V.rg[r];
+        double fx = 0.0, fz = 0.0;
+        if (g.found) {
 #pragma unroll
-        for (int c = 0; c < 4; ++c) {
-            const bool hang = (g.hang >> c) & 1;
-            const double2 a = P::full(P::ld(U, g.a[c]));
-            const double2 b = hang ? P::full(P::ld(U, g.b[c])) : a;
-            recv_accum(a, b, hang, g.w[c], fx, fz);
+            for (int c = 0; c < 4; ++c) {
+                const bool hang = (g.hang >> c) & 1;
+                const double2 a = P::full(P::ld(U, g.a[c]));
+                const double2 b = hang ? P::full(P::ld(U, g.b[c])) : a;
+                recv_accum(a, b, hang, g.w[c], fx, fz);
+            }
+            if (g.ff >= 0) {
+                const double4 f = V.fftab[(size_t)(j % V.chunk) * V.nff + g.ff];
+                fx = fx + f.x;
+                fz = fz + f.y;
+            }
         }
-        if (g.ff >= 0) {
-            const double4 f = V.fftab[(size_t)(j % V.chunk) * V.nff + g.ff];
-            fx = fx + f.x;
-            fz = fz + f.y;
-        }
+        double* out = recv_slot(V, j, r);
+        out[0] = fx;
+        out[1] = fz;
     }
-    double* out = recv_slot(V, j, r);
-    out[0] = fx;
-    out[1] = fz;
+    report_done(V, call);
 }
 
 // Displacement of the nodes [first, first + n) of an instance in the caller's
@@ -1387,45 +1408,50 @@ size_t step_lds_bytes(const DevView& V, int precision)
 
 template <class P>
 static void launch_one(const DevView& V, int grid, size_t lds, hipStream_t st, int t0, int use_base, int k,
-                       int end)
+                       int end, uint32_t call)
 {
     const auto go = [&](auto kernel) {
-        hipLaunchKernelGGL(kernel, dim3(grid), dim3(V.threads), lds, st, V, t0, use_base, k, V.depth == 1 ? 0 : end);
+        hipLaunchKernelGGL(kernel, dim3(grid), dim3(V.threads), lds, st, V, t0, use_base, k, V.depth == 1 ? 0 : end, call);
     };
     // several steps per launch: meshes without hanging nodes have a kernel
     // without their phases, their barrier and a quarter of the registers
     // (40,000-element layer, FP64, 3 steps per launch: 2.95 us a step against
-    // 3.29 with the other), and layouts without patches, where the slowest
-    // tile bounds the launch, one without the branch to them (canyon
-    // quadtree, FP32C: 3.21 against 3.23)
-    if (V.depth == 1) go(step_kernel<P, true, true, true>);
-    else if (V.nv > 0 && V.patches) go(step_kernel<P, false, true, true>);
-    else if (V.nv > 0) go(step_kernel<P, false, true, false>);
-    else if (V.patches) go(step_kernel<P, false, false, true>);
-    else go(step_kernel<P, false, false, false>);
+    // 3.29 with the other); layouts of tiles only, where the slowest tile
+    // bounds the launch, one without the branch to patches and the report of
+    // the call's end (canyon quadtree, FP32C: 3.21 against 3.23)
+    const Parts parts = V.patches ? Parts::kPatches : call ? Parts::kWhole : Parts::kTiles;
+    if (V.depth == 1) go(step_kernel<P, true, true, Parts::kPatches>);
+    else if (V.nv > 0 && parts == Parts::kPatches) go(step_kernel<P, false, true, Parts::kPatches>);
+    else if (V.nv > 0 && parts == Parts::kWhole) go(step_kernel<P, false, true, Parts::kWhole>);
+    else if (V.nv > 0) go(step_kernel<P, false, true, Parts::kTiles>);
+    else if (parts == Parts::kPatches) go(step_kernel<P, false, false, Parts::kPatches>);
+    else if (parts == Parts::kWhole) go(step_kernel<P, false, false, Parts::kWhole>);
+    else go(step_kernel<P, false, false, Parts::kTiles>);
 }
 
-hipError_t launch_step(const DevView& V, int precision, int t0, int use_base, int k, hipStream_t st, int end)
+hipError_t launch_step(const DevView& V, int precision, int t0, int use_base, int k, hipStream_t st, int end,
+                       uint32_t call)
 {
     const int grid = node_grid(V);
     if (grid == 0) return hipSuccess;
     if (end && k >= V.depth) return hipErrorInvalidValue;   // ring 1 would not be exact at t0 + k
+    if (call && (V.node_tiles != 1 || V.depth == 1 || V.patches)) return hipErrorInvalidValue;   // the one tile reports
     const size_t lds = step_lds_bytes(V, precision);
     if (precision == 0)
-        launch_one<PF64>(V, grid, lds, st, t0, use_base, k, end);
+        launch_one<PF64>(V, grid, lds, st, t0, use_base, k, end, call);
     else
-        launch_one<PF32C>(V, grid, lds, st, t0, use_base, k, end);
+        launch_one<PF32C>(V, grid, lds, st, t0, use_base, k, end, call);
     return hipGetLastError();
 }
 
-hipError_t launch_recv(const DevView& V, int precision, int j, hipStream_t st)
+hipError_t launch_recv(const DevView& V, int precision, int j, uint32_t call, hipStream_t st)
 {
     if (V.nrecv <= 0) return hipSuccess;
-    const int grid = (V.nrecv + 255) / 256;
+    const dim3 block(std::min(kMaxThreads, (V.nrecv + 63) / 64 * 64));
     if (precision == 0)
-        hipLaunchKernelGGL(recv_kernel<PF64>, dim3(grid), dim3(256), 0, st, V, j);
+        hipLaunchKernelGGL(recv_kernel<PF64>, dim3(1), block, 0, st, V, j, call);
     else
-        hipLaunchKernelGGL(recv_kernel<PF32C>, dim3(grid), dim3(256), 0, st, V, j);
+        hipLaunchKernelGGL(recv_kernel<PF32C>, dim3(1), block, 0, st, V, j, call);
     return hipGetLastError();
 }
 
@@ -1445,16 +1471,20 @@ hipError_t launch_state(int precision, const void* U, const int* node_int, const
 // budget (the most any layout may then need).
 hipError_t configure_kernels(size_t* max_lds)
 {
-    const void* fns[] = {reinterpret_cast<const void*>(step_kernel<PF64, true, true, true>),
-                         reinterpret_cast<const void*>(step_kernel<PF64, false, true, true>),
-                         reinterpret_cast<const void*>(step_kernel<PF64, false, true, false>),
-                         reinterpret_cast<const void*>(step_kernel<PF64, false, false, true>),
-                         reinterpret_cast<const void*>(step_kernel<PF64, false, false, false>),
-                         reinterpret_cast<const void*>(step_kernel<PF32C, true, true, true>),
-                         reinterpret_cast<const void*>(step_kernel<PF32C, false, true, true>),
-                         reinterpret_cast<const void*>(step_kernel<PF32C, false, true, false>),
-                         reinterpret_cast<const void*>(step_kernel<PF32C, false, false, true>),
-                         reinterpret_cast<const void*>(step_kernel<PF32C, false, false, false>)};
+    const void* fns[] = {reinterpret_cast<const void*>(step_kernel<PF64, true, true, Parts::kPatches>),
+                         reinterpret_cast<const void*>(step_kernel<PF64, false, true, Parts::kTiles>),
+                         reinterpret_cast<const void*>(step_kernel<PF64, false, true, Parts::kPatches>),
+                         reinterpret_cast<const void*>(step_kernel<PF64, false, true, Parts::kWhole>),
+                         reinterpret_cast<const void*>(step_kernel<PF64, false, false, Parts::kTiles>),
+                         reinterpret_cast<const void*>(step_kernel<PF64, false, false, Parts::kPatches>),
+                         reinterpret_cast<const void*>(step_kernel<PF64, false, false, Parts::kWhole>),
+                         reinterpret_cast<const void*>(step_kernel<PF32C, true, true, Parts::kPatches>),
+                         reinterpret_cast<const void*>(step_kernel<PF32C, false, true, Parts::kTiles>),
+                         reinterpret_cast<const void*>(step_kernel<PF32C, false, true, Parts::kPatches>),
+                         reinterpret_cast<const void*>(step_kernel<PF32C, false, true, Parts::kWhole>),
+                         reinterpret_cast<const void*>(step_kernel<PF32C, false, false, Parts::kTiles>),
+                         reinterpret_cast<const void*>(step_kernel<PF32C, false, false, Parts::kPatches>),
+                         reinterpret_cast<const void*>(step_kernel<PF32C, false, false, Parts::kWhole>)};
     size_t budget = *max_lds;
     for (const void* f : fns) {
         hipFuncAttributes a{};
