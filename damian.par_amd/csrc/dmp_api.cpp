@@ -1773,10 +1773,17 @@ void build_tiles(Runtime& R)
     V.lds_recv = max_recv;
     V.lds_mat = 4;   // every tile loads its 4-entry table
     V.threads = std::max(V.threads, (2 * max_vrows + 63) / 64 * 64);   // two lanes per hanging-node row
-    // a mesh in one tile updates every node in every sub-step: a wave of its
-    // own samples the receivers beside (861-node layer, 49 receivers, FP64:
-    // 2.15 us a step against 2.69)
-    if (R.whole && max_recv > 0 && V.threads + 64 <= kMaxThreads) V.threads += 64;
+    // A mesh in one tile updates every node in every sub-step: its hanging-node
+    // rows and receivers, which the kernel gives to the last waves, get waves
+    // of their own (358-node valley, FP64 1.93 us a step against 2.34; 861-node
+    // layer, 49 receivers, 2.04 against 2.69).  In other layouts they cost more
+    // at the start of each launch than they save (canyon quadtree, FP32C, 3.24
+    // against 3.19).
+    if (R.whole) {
+        auto waves = [](int lanes) { return (lanes + 63) / 64; };
+        V.threads = std::max(V.threads, std::min(64 * (waves(max_ent) + waves(2 * max_vrows) + (max_recv ? 1 : 0)),
+                                                 kMaxThreads));
+    }
     if (V.threads > kMaxThreads)
         throw fail(DMP_EUNSUPPORTED, "tiles need %d threads (max %d)", V.threads, kMaxThreads);
     // every index the kernel follows stays inside its array (checked before

@@ -492,22 +492,6 @@ __device__ __forceinline__ T uniform_record(const T* p)
     return __builtin_bit_cast(T, r);
 }
 
-// Receiver samples of step j = t0 + s (visu_field, visualization.f90:156-181)
-// from the tile's values at that step; the free field is added in the
-// exterior region.
-// Lane of receiver work (sampling, free-field loads): several steps per
-// launch put it on the last wave of the workgroup, which forms no
-// hanging-node values or rows (one lane each, from lane 0 up; tiles hold a
-// few dozen, at most a few hundred), so that sampling overlaps those phases;
-// in the one-step kernel every wave has core nodes to update and the lane is
-// the thread index.
-template <bool ONE>
-__device__ __forceinline__ int recv_lane()
-{
-    const int t = (int)threadIdx.x, nt = (int)blockDim.x;
-    return ONE || nt == 64 ? t : (t + 64) % nt;
-}
-
 // First lane of a small list copied into LDS during the load phase, the lane
 // order rotated by `off` lanes: in a multi-step launch wave 0 has the longest
 // chain of dependent loads (its entry loads, then the lists whose lanes
@@ -541,6 +525,9 @@ __device__ __forceinline__ double* recv_slot(const DevView& V, int j, int r)
     return V.recv_buf + 2 * ((size_t)(q % V.recv_cap) * V.nrecv + r);
 }
 
+// Receiver samples of step j = t0 + s (visu_field, visualization.f90:156-181)
+// from the tile's values at that step; the free field is added in the
+// exterior region.
 // Samples the tile's receivers at step t0 + s from the LDS values into
 // rff[s][q], in place of that receiver's free field (read once, here, by the
 // same thread).  The samples go out to the ring in flush_receivers at the end
@@ -842,6 +829,10 @@ __device__ void tile_steps(const DevView& V, int tile, int t0, int k, int end)
     const TileInfo T = uniform_record(V.tiles + tile);
     const int n0 = ONE ? tile * V.block : T.n0;
     const int cnt = ONE ? min(V.block, V.ngen - n0) : T.cnt;
+    // Several steps per launch: -K u of the ring entries beside the hanging-node
+    // rows, which it does not need; what they give is added behind the barrier
+    // (canyon quadtree FP64 3.32 -> 3.25 us a step, FP32C 3.21 -> 3.19)
+    constexpr bool BESIDE = !ONE && HANG;
     const int n_virt = HANG ? T.n_virt : 0, n_vrow = HANG ? T.n_vrow : 0;
     const int S = V.lds_slots;
     const int D = ONE ? 1 : V.depth;
@@ -959,8 +950,11 @@ __device__ void tile_steps(const DevView& V, int tile, int t0, int k, int end)
     if (!ONE && tid < n_virt) my_va = V.virt[T.virt_off + tid];
     for (int q = copy_lane<ONE>(7 * 64); q < n_virt; q += NT) va[q] = V.virt[T.virt_off + q];
     // two lanes per hanging-node row: lane 2 r + side takes half of row r's
-    // element terms and the transfer term of its anchor `side`
-    const int vr = tid >> 1, vside = tid & 1;
+    // element terms and the transfer term of its anchor `side`; the lanes are
+    // of lane index rl.  Several steps per launch: from the last wave down,
+    // whose ring entries stop being updated first
+    const int rl = ONE ? tid : NT - 64 - (tid & ~63) + (tid & 63);
+    const int vr = rl >> 1, vside = rl & 1;
     const bool has_vr = vr < n_vrow;
     RowsT vrow{};
     int v_slot = 0, v_force = -1;
@@ -990,7 +984,12 @@ __device__ void tile_steps(const DevView& V, int tile, int t0, int k, int end)
             frc[q] = V.ftab[(size_t)((t0 + s1 + 1) % V.chunk) * V.nforce + slot];
         }
     }
-    const int rlane = recv_lane<ONE>();
+    // Lane of receiver work (sampling, free-field loads): several steps per
+    // launch put it on the last wave, or on those below the ones of the
+    // hanging-node rows, so that sampling overlaps them; in the one-step kernel every wave has core nodes
+    // to update and the lane is the thread index
+    const int roff = 2 * n_vrow > NT - 64 ? 0 : (2 * n_vrow + 63) / 64 * 64;
+    const int rlane = ONE ? tid : !HANG ? (tid + 64) % NT : rl >= roff ? rl - roff : rl - roff + NT;
     // end (several-step layouts, k < depth): the launch also samples step
     // t0 + k, ring 1 being still exact after its k sub-steps
     const int srows = max(k, 1) + (!ONE && end ? 1 : 0);
@@ -1099,15 +1098,19 @@ __device__ void tile_steps(const DevView& V, int tile, int t0, int k, int end)
                 V2<R> g = gv;
                 g.x += v_a1m * (R(2) * du.x - dp.x) + v_a2c0 * (dp.x - R(2) * vel.x);
                 g.y += v_a1m * (R(2) * du.y - dp.y) + v_a2c1 * (dp.y - R(2) * vel.y);
-                ft[tid] = {R(0.5) * g.x, R(0.5) * g.y};   // ft[2 * row + side]
+                ft[rl] = {R(0.5) * g.x, R(0.5) * g.y};   // ft[2 * row + side]
             }
             if (recv_in_rows) sample_receivers<P>(V, cur, rff, rcv, n_recv, t0, s - 1, rlane);
-            __syncthreads();
+            if (!BESIDE) __syncthreads();
         }
-        if (e < (ONE ? cnt : lev_end(D - s))) {
+        const bool upd = e < (ONE ? cnt : lev_end(D - s));
+        V2<R> f{0, 0};
+        if (BESIDE && upd) f = rows.apply_pairs(cur, cur[e], e, lmt, em, elem);
+        if (BESIDE && n_vrow) __syncthreads();
+        if (upd) {
             const node_t un = cur[e], upn = prv[e];
-            V2<R> f = ONE ? rows.apply(cur, un, e, lmt, em, elem)
-                          : rows.apply_pairs(cur, un, e, lmt, em, elem);   // -K u
+            if (!BESIDE)
+                f = ONE ? rows.apply(cur, un, e, lmt, em, elem) : rows.apply_pairs(cur, un, e, lmt, em, elem);
             V2<R> corr;
             int point = 0;
             double pz = 0.0;
