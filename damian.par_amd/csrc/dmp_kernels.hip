@@ -297,16 +297,20 @@ struct Rows {
     // Two elements at a time: the six corner reads are issued before any of
     // them is used (an absent element reads the node's own slot, whose
     // differences are exactly 0, with a zero material, so it adds +0 as
-    // skipping it would).
-    template <int K0>
+    // skipping it would).  MREG: the moduli are in mr already.
+    template <int K0, bool MREG>
     __device__ void pair_rows(const typename P::node_t* val, typename P::node_t uref, int self,
-                              const V2<R>* lmt, const V2<R>* em, bool elem, V2<R>& f) const
+                              const V2<R>* lmt, const V2<R>* em, bool elem, const V2<R> (&mr)[4], V2<R>& f) const
     {
         using node_t = typename P::node_t;
         const uint32_t sw = (uint32_t)self * ((1u << 20) | (1u << 10) | 1u);
         const bool p0 = present(K0), p1 = present(K0 + 1);
         const uint32_t w0 = p0 ? w[K0] : sw, w1 = p1 ? w[K0 + 1] : sw;
-        const V2<R> m0 = mat(K0, lmt, em, self, elem), m1 = mat(K0 + 1, lmt, em, self, elem);
+        V2<R> m0 = mr[K0], m1 = mr[K0 + 1];
+        if (!MREG) {
+            m0 = mat(K0, lmt, em, self, elem);
+            m1 = mat(K0 + 1, lmt, em, self, elem);
+        }
         node_t c0[3], c1[3];
 #pragma unroll
         for (int q = 0; q < 3; ++q) {
@@ -314,15 +318,16 @@ struct Rows {
             c1[q] = val[(w1 >> (10 * q)) & 1023];
         }
         __builtin_amdgcn_sched_barrier(0);
-        slot_rows_v<P, K0>(c0, p0 ? m0 : V2<R>{0, 0}, uref, f);
-        slot_rows_v<P, K0 + 1>(c1, p1 ? m1 : V2<R>{0, 0}, uref, f);
+        slot_rows_v<P, K0>(c0, MREG || p0 ? m0 : V2<R>{0, 0}, uref, f);
+        slot_rows_v<P, K0 + 1>(c1, MREG || p1 ? m1 : V2<R>{0, 0}, uref, f);
     }
+    template <bool MREG>
     __device__ V2<R> apply_pairs(const typename P::node_t* val, typename P::node_t uref, int self,
-                                 const V2<R>* lmt, const V2<R>* em, bool elem) const
+                                 const V2<R>* lmt, const V2<R>* em, bool elem, const V2<R> (&mr)[4]) const
     {
         V2<R> f{0, 0};
-        pair_rows<0>(val, uref, self, lmt, em, elem, f);
-        pair_rows<2>(val, uref, self, lmt, em, elem, f);
+        pair_rows<0, MREG>(val, uref, self, lmt, em, elem, mr, f);
+        pair_rows<2, MREG>(val, uref, self, lmt, em, elem, mr, f);
         return f;
     }
     // Rows (2K, 2K+1) of corner K's element from a word whose slots are in
@@ -528,28 +533,34 @@ __device__ __forceinline__ double* recv_slot(const DevView& V, int j, int r)
 // Receiver samples of step j = t0 + s (visu_field, visualization.f90:156-181)
 // from the tile's values at that step; the free field is added in the
 // exterior region.
-// Samples the tile's receivers at step t0 + s from the LDS values into
-// rff[s][q], in place of that receiver's free field (read once, here, by the
+// Samples the tile's receivers at step t0 + s, if it is `due` (which then
+// becomes the next one), from the LDS values into rff[s][q], in place of that receiver's free field (read once, here, by the
 // same thread).  The samples go out to the ring in flush_receivers at the end
 // of the launch: a barrier waits for every global store its wave has issued
-// (stores count in vmcnt), so nothing is stored while barriers remain.
+// (stores count in vmcnt), so nothing is stored while barriers remain.  Bound by
+// the chain of LDS reads on one wave, which the others wait for at the next
+// barrier: the corners' values are read together, and what a sub-step samples
+// is counted instead of divided out (40,000-element layer, FP64, 2.86 -> 2.73
+// us a step; canyon quadtree FP64 3.22 -> 3.10, FP32C 3.09 -> 2.96).
 template <class P>
 __device__ void sample_receivers(const DevView& V, const typename P::node_t* cur, double2* rff,
-                                 const RecvT* rcv, int n_recv, int t0, int s, int lane)
+                                 const RecvT* rcv, int n_recv, int s, int& due, int lane)
 {
-    const int I = V.recv_interval;
-    const int j = t0 + s;
-    if (I <= 0 || (j % I) != 0) return;
+    if (s != due) return;
+    due += V.recv_interval;
     for (int q = lane; q < n_recv; q += blockDim.x) {
         const RecvT& Rc = rcv[q];
         double fx = 0.0, fz = 0.0;
+        const int hangs = Rc.hang;
+        typename P::node_t a[4], b[4];
 #pragma unroll
-        for (int c = 0; c < 4; ++c) {
-            const bool hang = (Rc.hang >> c) & 1;
-            const double2 a = P::full(cur[Rc.s[c].x]);
-            const double2 b = hang ? P::full(cur[Rc.s[c].y]) : a;
-            recv_accum(a, b, hang, Rc.w[c], fx, fz);
+        for (int c = 0; c < 4; ++c) b[c] = a[c] = cur[Rc.s[c].x];
+        if (hangs) {
+#pragma unroll
+            for (int c = 0; c < 4; ++c) b[c] = cur[(hangs >> c) & 1 ? Rc.s[c].y : Rc.s[c].x];
         }
+#pragma unroll
+        for (int c = 0; c < 4; ++c) recv_accum(P::full(a[c]), P::full(b[c]), (hangs >> c) & 1, Rc.w[c], fx, fz);
         if (Rc.ff >= 0) {
             const double2 g = rff[s * n_recv + q];
             fx = fx + g.x;
@@ -559,19 +570,18 @@ __device__ void sample_receivers(const DevView& V, const typename P::node_t* cur
     }
 }
 
-// Stores the samples of rows 0 .. rows-1 (steps t0 .. t0 + rows - 1) that
+// Stores the samples of rows first, first + interval, .. below rows (steps
+// t0 + row; first < 0: none) that
 // sample_receivers left in rff; the same lane mapping, so each thread stores
 // what it computed and no barrier is needed.
 __device__ void flush_receivers(const DevView& V, const double2* rff, const RecvT* rcv, int n_recv, int t0,
-                                int rows, int lane)
+                                int rows, int first, int lane)
 {
-    const int I = V.recv_interval;
-    if (I <= 0) return;
+    if (first < 0) return;
     for (int q = lane; q < n_recv; q += blockDim.x) {
         const int r = rcv[q].r;
-        for (int s = 0; s < rows; ++s) {
+        for (int s = first; s < rows; s += V.recv_interval) {
             const int j = t0 + s;
-            if (j % I != 0) continue;
             const double2 v = rff[s * n_recv + q];
             double* out = recv_slot(V, j, r);
             out[0] = v.x;
@@ -861,20 +871,22 @@ __device__ void tile_steps(const DevView& V, int tile, int t0, int k, int end)
     // material table: 4 per tile at a fixed stride (no dependence on the
     // tile record)
     if (tid < 4) lmt[tid] = P::lm(V.tile_lm, 4 * tile + tid);
-    // T.lev_end[j] as scalars and register selects (a dynamic index would put
-    // the tile record on the scratch stack)
-    static_assert(kMaxDepth == 8, "ring levels read as nine scalars");
-    const int le0 = T.lev_end[0], le1 = T.lev_end[1], le2 = T.lev_end[2], le3 = T.lev_end[3],
-              le4 = T.lev_end[4], le5 = T.lev_end[5], le6 = T.lev_end[6], le7 = T.lev_end[7],
-              le8 = T.lev_end[8];
-    auto lev_end = [=](int j) {
-        return j <= 0 ? le0 : j == 1 ? le1 : j == 2 ? le2 : j == 3 ? le3 : j == 4 ? le4
-             : j == 5 ? le5 : j == 6 ? le6 : j == 7 ? le7 : le8;
-    };
-    const int upd_end = lev_end(D - 1);   // entries ever updated
     // values of every entry (the outer ring is read, never updated), and the
     // lane's entry, updated while it is inside the exact rings
     const int e = tid;
+    // the last sub-step that updates the lane's entry: a ring-r value at
+    // sub-step s serves core values at k (ring 1 with end) when r <= k - s.
+    // Found once: looked up by s in each sub-step it is a chain of scalar
+    // branches that every wave waits for (canyon quadtree FP32C 3.19 -> 3.11
+    // us a step, FP64 3.25 -> 3.22)
+    static_assert(kMaxDepth == 8, "ring levels");
+    int last = 0;
+    if (!ONE) {
+        int rings = 0;   // levels j < D the entry lies in
+#pragma unroll
+        for (int j = 0; j < kMaxDepth; ++j) rings += j < D && e < T.lev_end[j];
+        last = e < cnt ? k : max(0, rings - (D - k) + (end ? 1 : 0));
+    }
     int gid = n0 + e;   // the lane's node
     RowsT rows{};
     R cf = 0;
@@ -918,7 +930,7 @@ __device__ void tile_steps(const DevView& V, int tile, int t0, int k, int end)
     }
     if (elem)
         for (int q = tid; q < n_virt; q += NT) em[T.n_ent + q] = P::lm(V.virt_em, T.virt_off + q);
-    if (!ONE && e < upd_end) {
+    if (last > 0) {
         uint4 d0{};
         if (e < cnt) {
             d0 = V.core_desc[n0 + e];
@@ -992,6 +1004,9 @@ __device__ void tile_steps(const DevView& V, int tile, int t0, int k, int end)
     const int rlane = ONE ? tid : !HANG ? (tid + 64) % NT : rl >= roff ? rl - roff : rl - roff + NT;
     // end (several-step layouts, k < depth): the launch also samples step
     // t0 + k, ring 1 being still exact after its k sub-steps
+    // the first sampled step is t0 + first
+    const int first = V.recv_interval > 0 ? (V.recv_interval - t0 % V.recv_interval) % V.recv_interval : -1;
+    int due = first;
     const int srows = max(k, 1) + (!ONE && end ? 1 : 0);
     if (ONE) {
         for (int q = rlane; q < V.lds_recv; q += NT) {
@@ -1040,9 +1055,20 @@ __device__ void tile_steps(const DevView& V, int tile, int t0, int k, int end)
     // once (FP64 reads them from LDS: its registers are nearly all in use)
     constexpr bool kSideRegs = !ONE && sizeof(R) == sizeof(float);
     R m_invm0 = 0, m_invm1 = 0, m_c20 = 0, m_c21 = 0;
+    // the moduli of the entry's elements too (zero where there is none), but
+    // not in FP64 with hanging nodes, whose registers do not hold them
+    // (40,000-element layer FP64 2.91 -> 2.86 us a step, canyon quadtree
+    // FP32C 3.04 -> 2.99)
+    constexpr bool kMatRegs = !ONE && (sizeof(R) == sizeof(float) || !HANG);
+    V2<R> mr[4] = {};
     for (int s = 1; s <= (ONE ? min(k, 1) : k); ++s) {
         if (!ONE && s == 1) {
             __syncthreads();
+            if (kMatRegs && last > 0) {
+#pragma unroll
+                for (int q = 0; q < 4; ++q)
+                    if (rows.present(q)) mr[q] = rows.mat(q, lmt, em, e, elem);
+            }
             if (side) {
                 const SideT& q = sides[sidx];
                 if (kSideRegs) {
@@ -1060,7 +1086,7 @@ __device__ void tile_steps(const DevView& V, int tile, int t0, int k, int end)
         }
         // (a mesh without hanging nodes has no phase here and no barrier, so
         // that the last wave samples beside the others' node updates)
-        if (!recv_in_rows) sample_receivers<P>(V, cur, rff, rcv, n_recv, t0, s - 1, rlane);
+        if (!recv_in_rows) sample_receivers<P>(V, cur, rff, rcv, n_recv, s - 1, due, rlane);
         // hanging-node values at t0+s-1 (means of anchors)
         const int vb = T.n_ent;
         if (ONE) {
@@ -1100,17 +1126,17 @@ __device__ void tile_steps(const DevView& V, int tile, int t0, int k, int end)
                 g.y += v_a1m * (R(2) * du.y - dp.y) + v_a2c1 * (dp.y - R(2) * vel.y);
                 ft[rl] = {R(0.5) * g.x, R(0.5) * g.y};   // ft[2 * row + side]
             }
-            if (recv_in_rows) sample_receivers<P>(V, cur, rff, rcv, n_recv, t0, s - 1, rlane);
+            if (recv_in_rows) sample_receivers<P>(V, cur, rff, rcv, n_recv, s - 1, due, rlane);
             if (!BESIDE) __syncthreads();
         }
-        const bool upd = e < (ONE ? cnt : lev_end(D - s));
+        const bool upd = ONE ? e < cnt : s <= last;
         V2<R> f{0, 0};
-        if (BESIDE && upd) f = rows.apply_pairs(cur, cur[e], e, lmt, em, elem);
+        if (BESIDE && upd) f = rows.template apply_pairs<kMatRegs>(cur, cur[e], e, lmt, em, elem, mr);
         if (BESIDE && n_vrow) __syncthreads();
         if (upd) {
             const node_t un = cur[e], upn = prv[e];
             if (!BESIDE)
-                f = ONE ? rows.apply(cur, un, e, lmt, em, elem) : rows.apply_pairs(cur, un, e, lmt, em, elem);
+                f = ONE ? rows.apply(cur, un, e, lmt, em, elem) : rows.template apply_pairs<kMatRegs>(cur, un, e, lmt, em, elem, mr);
             V2<R> corr;
             int point = 0;
             double pz = 0.0;
@@ -1179,7 +1205,7 @@ __device__ void tile_steps(const DevView& V, int tile, int t0, int k, int end)
         if (s == k) {
             if (!ONE && end) {
                 __syncthreads();
-                sample_receivers<P>(V, nxt, rff, rcv, n_recv, t0, k, rlane);
+                sample_receivers<P>(V, nxt, rff, rcv, n_recv, k, due, rlane);
             }
             break;
         }
@@ -1195,7 +1221,7 @@ __device__ void tile_steps(const DevView& V, int tile, int t0, int k, int end)
         if (!ONE && end) P::st(Uk, gid, nxt[e]);
         if (!ONE && k > 1) P::st(Uk1, gid, cur[e]);
     }
-    flush_receivers(V, rff, rcv, n_recv, t0, srows, rlane);
+    flush_receivers(V, rff, rcv, n_recv, t0, srows, first, rlane);
 }
 
 // Tells the host that run call `call` is complete: the last kernel of the
