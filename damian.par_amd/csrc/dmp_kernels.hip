@@ -605,41 +605,6 @@ __device__ double2 drm_pair(const DrmElem& E, const double4* fs)
     return make_double2(px, pz);
 }
 
-// Several steps per launch: the values of a tile's entries into LDS from its
-// fixed-stride entry list (slot q for list word q), two list words per lane
-// at a time so that their loads overlap.
-template <class P>
-__device__ __forceinline__ void load_entries(const DevView& V, int tile, const void* U0, const void* Um,
-                                             typename P::node_t* buf, int S)
-{
-    using node_t = typename P::node_t;
-    constexpr int kNode = kPrevFlag - 1;
-    const int NT = blockDim.x, cap = V.elist_cap;
-    const int* L = V.elist + (size_t)tile * cap;
-    for (int q0 = threadIdx.x; q0 < cap; q0 += 2 * NT) {
-        const int q1 = q0 + NT;
-        const int w0 = L[q0];
-        const int w1 = q1 < cap ? L[q1] : -1;
-        node_t a0{}, b0{}, a1{}, b1{};
-        if (w0 >= 0) {
-            a0 = P::ld(U0, w0 & kNode);
-            if (w0 & kPrevFlag) b0 = P::ld(Um, w0 & kNode);
-        }
-        if (w1 >= 0) {
-            a1 = P::ld(U0, w1 & kNode);
-            if (w1 & kPrevFlag) b1 = P::ld(Um, w1 & kNode);
-        }
-        if (w0 >= 0) {
-            buf[q0] = a0;
-            if (w0 & kPrevFlag) buf[S + q0] = b0;
-        }
-        if (w1 >= 0) {
-            buf[q1] = a1;
-            if (w1 & kPrevFlag) buf[S + q1] = b1;
-        }
-    }
-}
-
 // LDS of one patch: values (of a block patch at two steps), and moduli per
 // element where a patch needs them.
 __host__ __device__ inline int patch_lds_bytes(const DevView& V, int real_bytes)
@@ -870,7 +835,25 @@ __device__ void tile_steps(const DevView& V, int tile, int t0, int k, int end)
     // ---- phase 0: every global load of the launch
     // material table: 4 per tile at a fixed stride (no dependence on the
     // tile record)
-    if (tid < 4) lmt[tid] = P::lm(V.tile_lm, 4 * tile + tid);
+    // Several steps per launch: the load phase, 3 of a launch's 12 us, is bound
+    // by the loads that wait for others.  The first words of every list go to
+    // registers in straight-line code, each issued as soon as its address is
+    // known, and to LDS together; what a list has beyond one word per lane is
+    // copied behind that.  Copied list by list the compiler waits for each
+    // before the next (canyon quadtree FP32C 2.85 -> 2.81 us a step, FP64 2.96
+    // -> 2.91; 40,000-element layer FP64 2.67 -> 2.57; 141,000-element basin at
+    // 2 steps per launch 4.74 -> 4.51).  Not initialised: a register would be
+    // written behind its load, which then is waited for at once.
+    node_t a0, b0, a1, b1;
+    V2<R> m0, m1, vm;
+    int w0 = -1, w1 = -1;
+    if (!ONE) {
+        const int* L = V.elist + (size_t)tile * V.elist_cap;
+        if (tid < V.elist_cap) w0 = L[tid];
+        if (tid + NT < V.elist_cap) w1 = L[tid + NT];
+    }
+    V2<R> my_lm;
+    if (tid < 4) my_lm = P::lm(V.tile_lm, 4 * tile + tid);
     // values of every entry (the outer ring is read, never updated), and the
     // lane's entry, updated while it is inside the exact rings
     const int e = tid;
@@ -922,45 +905,59 @@ __device__ void tile_steps(const DevView& V, int tile, int t0, int k, int end)
             rows.load(d0);
         }
     } else {
-        load_entries<P>(V, tile, U0, Um, buf, S);
-        if (elem) {
-            const int* L = V.elist + (size_t)tile * V.elist_cap;
-            for (int q = tid; q < T.n_ent; q += NT) em[q] = P::lm(V.node_em, L[q] & (kPrevFlag - 1));
+        // slot q of the fixed-stride entry list, two per lane
+        constexpr int kNode = kPrevFlag - 1;
+        if (w0 >= 0) {
+            a0 = P::ld(U0, w0 & kNode);
+            if (w0 & kPrevFlag) b0 = P::ld(Um, w0 & kNode);
+            if (elem) m0 = P::lm(V.node_em, w0 & kNode);
         }
+        if (w1 >= 0) {
+            a1 = P::ld(U0, w1 & kNode);
+            if (w1 & kPrevFlag) b1 = P::ld(Um, w1 & kNode);
+            if (elem) m1 = P::lm(V.node_em, w1 & kNode);
+        }
+        if (elem && tid < n_virt) vm = P::lm(V.virt_em, T.virt_off + tid);
     }
     if (elem)
-        for (int q = tid; q < n_virt; q += NT) em[T.n_ent + q] = P::lm(V.virt_em, T.virt_off + q);
+        for (int q = ONE ? tid : tid + NT; q < n_virt; q += NT) em[T.n_ent + q] = P::lm(V.virt_em, T.virt_off + q);
     if (last > 0) {
-        uint4 d0{};
+        // (scalar addresses, which the compiler would else select by lane
+        // before it loads them, per lane)
+        const uint4* rd = V.ring_desc;
+        const void* rc = V.ring_coef;
+        asm("" : "+s"(rd), "+s"(rc));
+        uint4 d0;
         if (e < cnt) {
             d0 = V.core_desc[n0 + e];
             cf = P::coef(V.core_coef, n0 + e);
         } else {
             const int r = T.ring_off + e - cnt;
-            d0 = V.ring_desc[r];
-            cf = P::coef(V.ring_coef, r);
+            d0 = rd[r];
+            cf = P::coef(rc, r);
         }
         rows.load(d0);
     }
-    {
-        // side records and receivers, copied as 16-byte words
-        constexpr int SW = sizeof(SideT) / 16, RW = sizeof(RecvT) / 16;
-        if (!ONE) {
-            const uint4* src = reinterpret_cast<const uint4*>(V.side + T.side_off);
-            uint4* dst = reinterpret_cast<uint4*>(sides);
-            for (int q = tid; q < SW * T.n_side; q += NT) dst[q] = src[q];
-        }
-        const uint4* rsrc = reinterpret_cast<const uint4*>(V.recvs + T.recv_off);
-        uint4* rdst = reinterpret_cast<uint4*>(rcv);
-        for (int q = copy_lane<ONE>(8 * 64); q < RW * T.n_recv; q += NT) rdst[q] = rsrc[q];
+    // side records and receivers, copied as 16-byte words; anchor slots of the
+    // hanging nodes (a multi-step launch keeps entry q in registers of lane q
+    // too)
+    constexpr int SW = sizeof(SideT) / 16, RW = sizeof(RecvT) / 16;
+    const uint4* ssrc = reinterpret_cast<const uint4*>(V.side + T.side_off);
+    uint4* sdst = reinterpret_cast<uint4*>(sides);
+    const uint4* rsrc = reinterpret_cast<const uint4*>(V.recvs + T.recv_off);
+    uint4* rdst = reinterpret_cast<uint4*>(rcv);
+    const int rq = copy_lane<ONE>(8 * 64), vq = copy_lane<ONE>(7 * 64);
+    uint4 sword, rword;
+    int2 vword, my_va{0, 0};
+    if (!ONE) {
+        if (tid < SW * T.n_side) sword = ssrc[tid];
+        if (rq < RW * T.n_recv) rword = rsrc[rq];
+        if (vq < n_virt) vword = V.virt[T.virt_off + vq];
+        if (tid < n_virt) my_va = V.virt[T.virt_off + tid];
+    } else {
+        for (int q = rq; q < RW * T.n_recv; q += NT) rdst[q] = rsrc[q];
+        for (int q = vq; q < n_virt; q += NT) va[q] = V.virt[T.virt_off + q];
     }
-    // anchor slots of the hanging nodes: in a multi-step launch lane q keeps
-    // entry q in registers for its sub-steps, loaded without a wait (the LDS
-    // copy serves lists longer than the workgroup, and the one-step kernel,
-    // which saves the registers)
-    int2 my_va{0, 0};
-    if (!ONE && tid < n_virt) my_va = V.virt[T.virt_off + tid];
-    for (int q = copy_lane<ONE>(7 * 64); q < n_virt; q += NT) va[q] = V.virt[T.virt_off + q];
     // two lanes per hanging-node row: lane 2 r + side takes half of row r's
     // element terms and the transfer term of its anchor `side`; the lanes are
     // of lane index rl.  Several steps per launch: from the last wave down,
@@ -984,17 +981,20 @@ __device__ void tile_steps(const DevView& V, int tile, int t0, int k, int end)
     }
     // forces of steps t0+1 .. t0+k and the receivers' free field of the steps
     // the launch samples, t0 .. t0+max(k,1)-1, from the tables
+    const int fq = copy_lane<ONE>(3 * 64);
+    double2 fval, gval;
+    auto force_of = [&](int q) {
+        const int s1 = q / T.n_force, f = q - s1 * T.n_force;
+        const int slot = V.force_slots[T.force_off + f];
+        return V.ftab[(size_t)((t0 + s1 + 1) % V.chunk) * V.nforce + slot];
+    };
     if (ONE) {
         for (int q = tid; q < V.lds_force; q += NT) {
             const int slot = V.force_slots[(size_t)tile * V.lds_force + q];
             if (slot >= 0) frc[q] = V.ftab[(size_t)((t0 + 1) % V.chunk) * V.nforce + slot];
         }
     } else {
-        for (int q = copy_lane<ONE>(3 * 64); q < k * T.n_force; q += NT) {
-            const int s1 = q / T.n_force, f = q - s1 * T.n_force;
-            const int slot = V.force_slots[T.force_off + f];
-            frc[q] = V.ftab[(size_t)((t0 + s1 + 1) % V.chunk) * V.nforce + slot];
-        }
+        if (fq < k * T.n_force) fval = force_of(fq);
     }
     // Lane of receiver work (sampling, free-field loads): several steps per
     // launch put it on the last wave, or on those below the ones of the
@@ -1017,15 +1017,49 @@ __device__ void tile_steps(const DevView& V, int tile, int t0, int k, int end)
             }
         }
     } else {
-        for (int q = rlane; q < srows * T.n_recv; q += NT) {
+        // (a receiver without a free field: any value, none is added)
+        auto field_of = [&](int q) {
             const int s = q / T.n_recv, r = q - s * T.n_recv;
             const int ff = V.recvs[T.recv_off + r].ff;
+            double2 f{};
             if (ff >= 0) {
                 const double4 g = V.fftab[(size_t)((t0 + s) % V.chunk) * V.nff + ff];
-                rff[q] = make_double2(g.x, g.y);
+                f = make_double2(g.x, g.y);
             }
+            return f;
+        };
+        if (rlane < srows * T.n_recv) gval = field_of(rlane);
+        // all of it to LDS
+        constexpr int kNode = kPrevFlag - 1;
+        if (w0 >= 0) {
+            buf[tid] = a0;
+            if (w0 & kPrevFlag) buf[S + tid] = b0;
+            if (elem) em[tid] = m0;
         }
+        if (w1 >= 0) {
+            buf[tid + NT] = a1;
+            if (w1 & kPrevFlag) buf[S + tid + NT] = b1;
+            if (elem) em[tid + NT] = m1;
+        }
+        if (elem && tid < n_virt) em[T.n_ent + tid] = vm;
+        if (tid < SW * T.n_side) sdst[tid] = sword;
+        if (rq < RW * T.n_recv) rdst[rq] = rword;
+        if (vq < n_virt) va[vq] = vword;
+        if (fq < k * T.n_force) frc[fq] = fval;
+        if (rlane < srows * T.n_recv) rff[rlane] = gval;
+        for (int q = tid + 2 * NT; q < T.n_ent; q += NT) {
+            const int w = V.elist[(size_t)tile * V.elist_cap + q], g = w & kNode;
+            buf[q] = P::ld(U0, g);
+            if (w & kPrevFlag) buf[S + q] = P::ld(Um, g);
+            if (elem) em[q] = P::lm(V.node_em, g);
+        }
+        for (int q = tid + NT; q < SW * T.n_side; q += NT) sdst[q] = ssrc[q];
+        for (int q = rq + NT; q < RW * T.n_recv; q += NT) rdst[q] = rsrc[q];
+        for (int q = vq + NT; q < n_virt; q += NT) va[q] = V.virt[T.virt_off + q];
+        for (int q = fq + NT; q < k * T.n_force; q += NT) frc[q] = force_of(q);
+        for (int q = rlane + NT; q < srows * T.n_recv; q += NT) rff[q] = field_of(q);
     }
+    if (tid < 4) lmt[tid] = my_lm;
     // one step: the lane's side record goes to registers, issued before the
     // barrier
     const bool side = cf < R(0);
@@ -1253,7 +1287,13 @@ template <class P, bool ONE, bool HANG, Parts PARTS>
 __global__ __launch_bounds__(kMaxThreads) __attribute__((amdgpu_waves_per_eu(ONE ? P::kOneWaves : 4)))
 void step_kernel(DevView V, int t0_arg, int use_base, int k, int end, uint32_t call)
 {
-    const int t0 = t0_arg + (use_base ? V.ctrl->base : 0);
+    // One argument of each 64 bytes is asked for here, so that the lines arrive
+    // together and not one after the other (canyon quadtree FP32C 2.97 -> 2.85
+    // us a step, FP64 3.09 -> 2.96; one step per launch, uniform canyon FP32C
+    // 10.95 -> 10.69, FP64 11.78 -> 11.46)
+    asm volatile("" ::"s"(V.node_tiles), "s"(V.tiles), "s"(V.side), "s"(V.fftab), "s"(V.lds_mat), "s"(V.U[3]),
+                 "s"(V.ctrl), "s"(t0_arg), "s"(use_base));
+    const int t0 = t0_arg + (use_base ? uniform_record(V.ctrl).base : 0);
     int b = blockIdx.x;
     // tiles first (the longer work), then the patches
     const int nb = V.xcd_remap ? 8 * V.tiles_per_xcd : V.node_tiles;
