@@ -623,8 +623,8 @@ __host__ __device__ inline int patch_lds_bytes(const DevView& V, int real_bytes)
 // spends some 100 more instructions on decoding descriptors and on the 12
 // corner reads that are 8 here, all at fixed offsets from one LDS address; and
 // a wavefront on its own needs no barrier.  The uniform 944,492-element canyon
-// takes 10.6 us a step in FP32C (4.3 TB/s of those 48 B) against 16.0 with
-// tiles only, and 11.6 against 17.2 in FP64.  Parts of cells count where much
+// takes 10.5 us a step in FP32C (4.3 TB/s of those 48 B) against 16.0 with
+// tiles only, and 11.3 against 17.2 in FP64.  Parts of cells count where much
 // of a mesh lies along sides, source layers and refinement fronts: whole cells
 // only leave 10 % of a basin's nodes to small tiles that take as long as the
 // rest, parts of cells 3 % (2.47M-element sweep, FP32C: 24.2 us a step against
@@ -689,16 +689,18 @@ __device__ __forceinline__ void patch_step(const DevView& V, int t, const void* 
     const int x = ((lane >> 1) & 1) | ((lane >> 2) & 2) | ((lane >> 3) & 4);
     const int z = (lane & 1) | ((lane >> 1) & 2) | ((lane >> 2) & 4);
     const int at = (x + 1) * W + z + 1;
-    node_t un{}, up{}, ur{};
+    // (both levels in one branch and nothing initialised, so that no load waits
+    // for another: uniform canyon FP32C 10.67 -> 10.49 us a step)
+    node_t un, up, ur;
     R cf = R(T.invm);
-    if (held) un = P::ld(U0, g);
-    if (own) {
+    if (held) {
+        un = P::ld(U0, g);
         up = P::ld(Um, g);
-        if (T.coefs) cf = P::coef(V.node_coef, g);
     }
     if (gr >= 0) ur = P::ld(U0, gr);
+    if (own && T.coefs) cf = P::coef(V.node_coef, g);
+    V2<R> e, er;
     if (T.hetero) {
-        V2<R> e{0, 0}, er{0, 0};
         if (held) e = P::lm(V.node_em, g);
         if (gr >= 0 && lane < kPatchLow) er = P::lm(V.node_em, gr);
         if (held) em[at] = e;
@@ -1292,7 +1294,7 @@ void step_kernel(DevView V, int t0_arg, int use_base, int k, int end, uint32_t c
     // us a step, FP64 3.09 -> 2.96; one step per launch, uniform canyon FP32C
     // 10.95 -> 10.69, FP64 11.78 -> 11.46)
     asm volatile("" ::"s"(V.node_tiles), "s"(V.tiles), "s"(V.side), "s"(V.fftab), "s"(V.lds_mat), "s"(V.U[3]),
-                 "s"(V.ctrl), "s"(t0_arg), "s"(use_base));
+                 "s"(V.ctrl), "s"(V.patch), "s"(t0_arg), "s"(use_base));
     const int t0 = t0_arg + (use_base ? uniform_record(V.ctrl).base : 0);
     int b = blockIdx.x;
     // tiles first (the longer work), then the patches
