@@ -71,6 +71,13 @@ constexpr int kPatchWaves = 4;
 // Steps per launch of a mesh that one workgroup holds whole (build_tiles).
 constexpr int kWholeSteps = 32;
 
+// Several steps per launch: lanes of a workgroup of which a compute unit's
+// registers hold two (16 wavefronts of 128), and what share of the tiles may be
+// halved to stay below, how often.
+constexpr int kPairThreads = 512;
+constexpr int kWideShare = 4;
+constexpr int kHalvings = 3;
+
 // State downloads: nodes per chunk (2 MiB) and chunks of pinned staging, and
 // the bytes to write that are worth one more host thread (starting one takes
 // about 20 us, copying 2 MiB into pages not yet mapped about 500).
@@ -1201,7 +1208,9 @@ PatchRuns find_patches(const PackedHost& H, int NA, const std::vector<char>& tak
     return out;
 }
 
-void build_tiles(Runtime& R)
+// build_tiles with the tiles that hold the nodes `halves` ended before them.
+// False, with more such nodes: to be built again (at most kHalvings times).
+bool try_tiles(Runtime& R, std::vector<int>& halves, int pass)
 {
     PhaseTimer pt("tiles");
     const PackedHost& H = R.host;
@@ -1299,6 +1308,12 @@ void build_tiles(Runtime& R)
             tstart.push_back(from);
             tend.push_back(to);
         }
+    }
+    for (int h : halves) {   // ascending
+        const size_t t = std::upper_bound(tstart.begin(), tstart.end(), h) - tstart.begin() - 1;
+        if (tstart[t] == h || h >= tend[t]) continue;
+        tstart.insert(tstart.begin() + t + 1, h);
+        tend.insert(tend.begin() + t, h);
     }
     ntiles = (int)tstart.size();
     auto tile_of = [&](int node) {
@@ -1621,6 +1636,24 @@ void build_tiles(Runtime& R)
         for (auto& th : pool) th.join();
         for (auto& e : errs)
             if (e) std::rethrow_exception(e);
+    }
+    // A workgroup has as many lanes as its layout's widest tile.  With more
+    // workgroups than compute units, two share one while neither has more than
+    // kPairThreads lanes, so the few tiles that need more (hanging nodes widen
+    // their rings) are halved: 256 nodes per tile, 3 steps per launch, basins of
+    // 141,000 and 187,000 nodes FP32C 4.60 -> 3.43 and 5.59 -> 4.30 us a step,
+    // FP64 4.78 -> 3.55 and 5.90 -> 4.88; the canyon refined to 134,000 nodes
+    // 4.66 -> 3.43.  Where many do, halving would only add tiles.
+    if (K > 1 && !R.whole && ntiles + (int)patches.start.size() > ncu && pass < kHalvings) {
+        std::vector<int> wide;
+        for (const TilePart& P : parts)
+            for (const TileInfo& T : P.tiles)
+                if (T.lev_end[K - 1] > kPairThreads && T.cnt > 1) wide.push_back(T.n0 + T.cnt / 2);
+        if (!wide.empty() && (long)wide.size() * kWideShare <= ntiles) {
+            halves.insert(halves.end(), wide.begin(), wide.end());
+            std::sort(halves.begin(), halves.end());
+            return false;
+        }
     }
     std::vector<TileInfo> tiles;
     std::vector<int> ring_gid;
@@ -2108,6 +2141,13 @@ void build_tiles(Runtime& R)
     R.tiles_block = R.tuning[0];
     R.tiles_depth = K;
     R.tiles_own = R.own_shape;
+    return true;
+}
+
+void build_tiles(Runtime& R)
+{
+    std::vector<int> halves;
+    for (int pass = 0; !try_tiles(R, halves, pass); ++pass) {}
 }
 
 void prepare_graph(Runtime& R);

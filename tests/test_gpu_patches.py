@@ -143,3 +143,32 @@ def test_block_patches(name, prec):
         s.close()
         for a, b in zip(got, want):
             assert np.array_equal(a, b)
+
+
+@pytest.mark.parametrize("prec", [0, 1])
+@pytest.mark.parametrize("name", ["valley", "canyon"])
+def test_halved_tiles(name, prec):
+    """Layouts with more workgroups than compute units halve the few tiles
+    that need more than 512 lanes (those that hanging nodes widen)."""
+    from damian_hip import cases, lib
+    case = cases.c4_valley(200.0, "SV", 10.0) if name == "valley" else cases.BUILDERS["c2"]()
+    n = 41
+    ref = lib.Solver(case, precision=prec)
+    ref.set_tuning(256, 1, 0, 1)
+    ref.run(300)
+    want = (ref.run(n),) + ref.state()[:2]
+    ref.close()
+    assert np.abs(want[0]).max() > 0
+    for tuning in ((256, 1, 0, 3), (200, 1, 0, 4), (170, 0, 12, 4), (140, 1, 0, 4)):
+        print(f"name={name} prec={prec} tuning={tuning}", flush=True)
+        s = lib.Solver(case, precision=prec)
+        try:
+            s.set_tuning(*tuning)
+        except lib.DmpError as e:   # hanging nodes widen the rings of deep launches
+            assert e.code == -4
+            continue
+        s.run(300)
+        got = (s.run(n),) + s.state()[:2]
+        s.close()
+        for a, b in zip(got, want):
+            assert np.array_equal(a, b)
