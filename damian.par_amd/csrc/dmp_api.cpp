@@ -1226,9 +1226,10 @@ bool try_tiles(Runtime& R, std::vector<int>& halves, int pass)
     // field) shares the LDS.  Where the caller asks for several steps per
     // launch and tiles that small a mesh fits in, or has left the shape to the
     // library, such a mesh is one tile: the two-material valley of 358 nodes
-    // takes 2.2 us a step in FP32C so, 3.8 in two tiles at three steps per
-    // launch; the layer of 861 nodes 2.1 against 3.4 in FP64, 1.8 against 3.3
-    // in FP32C.  Descriptors address no more slots.
+    // takes 1.79 us a step in FP32C so, 3.2 in two tiles at three steps per
+    // launch and 2.3 at eight; the layer of 861 nodes 1.91 against 2.56 and 1.83
+    // in FP64, 1.78 against 2.50 and 1.74 in FP32C, in half the launches.
+    // Descriptors address no more slots.
     R.whole = K > 1 && NA <= kMaxSlots && (R.tuning[0] >= NA || R.own_shape) && !R.no_whole;
     const int B = R.whole ? std::max(NA, 1) : K == 1 && !R.no_patches ? std::min(R.tuning[0], kRestBlock) : R.tuning[0];
     int ntiles = (NA + B - 1) / B;
@@ -1808,10 +1809,9 @@ bool try_tiles(Runtime& R, std::vector<int>& halves, int pass)
     V.threads = std::max(V.threads, (2 * max_vrows + 63) / 64 * 64);   // two lanes per hanging-node row
     // A mesh in one tile updates every node in every sub-step: its hanging-node
     // rows and receivers, which the kernel gives to the last waves, get waves
-    // of their own (358-node valley, FP64 1.93 us a step against 2.34; 861-node
-    // layer, 49 receivers, 2.04 against 2.69).  In other layouts they cost more
-    // at the start of each launch than they save (canyon quadtree, FP32C, 3.24
-    // against 3.19).
+    // of their own (358-node valley, FP64 1.68 us a step against 2.06; 861-node
+    // layer, 49 receivers, 1.72 against 2.00).  In other layouts they cost more
+    // at the start of each launch than they save (canyon quadtree, FP32C, 1.5 %).
     if (R.whole) {
         auto waves = [](int lanes) { return (lanes + 63) / 64; };
         V.threads = std::max(V.threads, std::min(64 * (waves(max_ent) + waves(2 * max_vrows) + (max_recv ? 1 : 0)),
@@ -3139,9 +3139,9 @@ void autotune(Runtime& R, int nsteps, int* out)
     }
     // many tiles per compute unit (bandwidth-bound): deep launches only add
     // ring work.  Basins of 141,000, 237,000 and 317,000 nodes, FP32C, best
-    // shape at 1, 2, 3 and 4 steps per launch: 7.3, 4.6, 3.9, 4.1; 7.6, 6.0,
-    // 5.6, 6.4; 7.9, 7.6, 6.9, 6.6 us a step; the 947,000-node uniform canyon
-    // 10.2, 14.2, 11.5, 14.1.
+    // shape at 1, 2, 3 and 4 steps per launch: 7.4, 4.5, 3.4, 3.5; 7.8, 5.7,
+    // 5.3, 6.0; 8.1, 7.0, 6.4, 6.0 us a step; the 947,000-node uniform canyon
+    // 10.3, 14.0, 11.6, 16.6.
     std::vector<int> cand_depth = {1, 2, 3, 4, 6, 8};
     {
         int ncu = 0;

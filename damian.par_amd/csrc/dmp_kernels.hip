@@ -624,7 +624,7 @@ __host__ __device__ inline int patch_lds_bytes(const DevView& V, int real_bytes)
 // corner reads that are 8 here, all at fixed offsets from one LDS address; and
 // a wavefront on its own needs no barrier.  The uniform 944,492-element canyon
 // takes 10.5 us a step in FP32C (4.3 TB/s of those 48 B) against 16.0 with
-// tiles only, and 11.3 against 17.2 in FP64.  Parts of cells count where much
+// tiles of 256 only, and 11.3 against 17.2 in FP64.  Parts of cells count where much
 // of a mesh lies along sides, source layers and refinement fronts: whole cells
 // only leave 10 % of a basin's nodes to small tiles that take as long as the
 // rest, parts of cells 3 % (2.47M-element sweep, FP32C: 24.2 us a step against
@@ -727,9 +727,9 @@ __device__ __forceinline__ void patch_step(const DevView& V, int t, const void* 
 // bound by the wavefronts in flight: a tile's share of registers, LDS and
 // instructions (descriptors, 12 corner reads, three barriers a step) allows
 // one or two tiles per compute unit, in several rounds.  Patches need a third
-// less of each: the 141,000-element basin takes 5.06 us a step in FP32C at 256
-// nodes per tile and 3 steps per launch against 7.63 with tiles only (FP64
-// 5.05 against 7.94), 3.86 at its best shape against 5.2.
+// less of each: the 141,000-element basin takes 3.43 us a step in FP32C at 256
+// nodes per tile and 3 steps per launch against 6.86 with tiles only (FP64
+// 3.55 against 7.34), 3.35 at its best shape against 4.4.
 // ---------------------------------------------------------------------------
 template <class P>
 __device__ __forceinline__ void block_patch_steps(const DevView& V, int t, int k, const void* U0, const void* Um,
@@ -1489,8 +1489,8 @@ static void launch_one(const DevView& V, int grid, size_t lds, hipStream_t st, i
     };
     // several steps per launch: meshes without hanging nodes have a kernel
     // without their phases, their barrier and a quarter of the registers
-    // (40,000-element layer, FP64, 3 steps per launch: 2.95 us a step against
-    // 3.29 with the other); layouts of tiles only, where the slowest tile
+    // (40,000-element layer, FP64, 3 steps per launch: 2.58 us a step against
+    // 2.98 with the other); layouts of tiles only, where the slowest tile
     // bounds the launch, one without the branch to patches and the report of
     // the call's end (canyon quadtree, FP32C: 3.21 against 3.23)
     const Parts parts = V.patches ? Parts::kPatches : call ? Parts::kWhole : Parts::kTiles;
