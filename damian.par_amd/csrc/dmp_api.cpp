@@ -2707,9 +2707,15 @@ void alloc_ring(Runtime& R, int nsteps)
     if (e != hipSuccess)
         throw fail(DMP_ENOMEM, "hipHostMalloc(%zu bytes) failed: %s", slots * row * sizeof(double),
                    hipGetErrorString(e));
-    std::memset(p, 0, slots * row * sizeof(double));
     R.hstage = static_cast<double*>(p);
     R.hstage_cap = slots * row;
+    // (the host's first touch maps each page: by several threads, 4 MiB at a time)
+    constexpr size_t kPart = (size_t(4) << 20) / sizeof(double);
+    const int parts = (int)((R.hstage_cap + kPart - 1) / kPart);
+    parallel_items(parts, std::min(setup_threads(), parts), [&](int i) {
+        const size_t lo = (size_t)i * kPart;
+        std::memset(R.hstage + lo, 0, std::min(kPart, R.hstage_cap - lo) * sizeof(double));
+    });
     void* dp = nullptr;
     HIPCHECK(hipHostGetDevicePointer(&dp, R.hstage, 0));
     R.V.recv_buf = static_cast<double*>(dp);
