@@ -310,8 +310,13 @@ struct Runtime {
     bool whole = false;            // one tile holds the mesh: no rings, up to V.depth steps per launch
     int state_depth = kMaxDepth;   // depth whose state_slot() the state buffers are in
     std::vector<void*> tile_allocs;
-    hipEvent_t ev0 = nullptr, ev1 = nullptr;
-    float last_ms = 0.0f;          // device time of the last run (events on `stream`)
+    // start and end of run calls on `stream`, in turn: a call that fails part
+    // way leaves those of the last complete one
+    struct Span {
+        hipEvent_t start = nullptr, end = nullptr;
+    } spans[2];
+    int last_span = 0;             // of the last complete call
+    float last_ms = 0.0f;          // its device time
     bool ms_pending = false;       // last_ms is still to be read off the events
     // completion word of run calls (report_done), mapped host memory, and the
     // number of the last call that used it
@@ -357,9 +362,11 @@ struct Runtime {
         allocs.clear();
         for (void* p : tile_allocs) (void)hipFree(p);
         tile_allocs.clear();
-        if (ev0) (void)hipEventDestroy(ev0);
-        if (ev1) (void)hipEventDestroy(ev1);
-        ev0 = ev1 = nullptr;
+        for (Span& t : spans) {
+            if (t.start) (void)hipEventDestroy(t.start);
+            if (t.end) (void)hipEventDestroy(t.end);
+            t = Span{};
+        }
         for (hipEvent_t e : free_ev) (void)hipEventDestroy(e);
         free_ev.clear();
         if (done) (void)hipHostFree(done);
@@ -2202,8 +2209,10 @@ void build_runtime(Runtime& R, const std::vector<Instance*>& insts)
     R.device = insts[0]->device;
     HIPCHECK(hipSetDevice(R.device));
     HIPCHECK(hipStreamCreateWithFlags(&R.stream, hipStreamNonBlocking));
-    HIPCHECK(hipEventCreate(&R.ev0));
-    HIPCHECK(hipEventCreate(&R.ev1));
+    for (Runtime::Span& t : R.spans) {
+        HIPCHECK(hipEventCreate(&t.start));
+        HIPCHECK(hipEventCreate(&t.end));
+    }
     HIPCHECK(scratch_address(R.device, &R.scratch));
     PhaseTimer pt_pack("pack");
     int NA = 0, NV = 0, NE = 0, NM = 0, NS = 0, NT = 0, NDE = 0, NR = 0, NSE = 0, NF = 0;
@@ -2837,7 +2846,8 @@ int run_steps(Runtime& R, int n, double* out)
     };
     auto last_sample = [&](int t0, int k) { return rec ? (long)(t0 + k - 1) / I : 0L; };
 
-    HIPCHECK(hipEventRecord(R.ev0, R.stream));
+    const Runtime::Span& span = R.spans[1 - R.last_span];
+    HIPCHECK(hipEventRecord(span.start, R.stream));
     int done = 0;
     if (G > 0 && n >= G) {
         if (R.graph_steps != G || R.graph_k != K || !R.gexec) capture_graph(R, G, K);
@@ -2876,12 +2886,13 @@ int run_steps(Runtime& R, int n, double* out)
         HIPCHECK(launch_recv(V, R.precision, s + n, call, R.stream));
         after(q_hi + 1);
     }
-    HIPCHECK(hipEventRecord(R.ev1, R.stream));
+    HIPCHECK(hipEventRecord(span.end, R.stream));
     while (mhead < marks.size()) retire();   // copies overlap the launches still running
     // a last kernel of one workgroup reports the end itself
-    if (call) wait_done(R, call, R.ev1);
-    else wait_event(R.ev1);
+    if (call) wait_done(R, call, span.end);
+    else wait_event(span.end);
     if (stream_out) copy_out(q_hi + 1);
+    R.last_span = 1 - R.last_span;
     R.ms_pending = true;
     R.step = s + n;
     R.first_run = false;
@@ -2919,7 +2930,8 @@ int run_steps_noalloc(Runtime& R, int n, double* out)
     const int K = V.depth;
     const bool end_sample = rec && (s + n) % I == 0 && (n > 0 || R.first_run);
     bool end_done = false;
-    HIPCHECK(hipEventRecord(R.ev0, R.stream));
+    const Runtime::Span& span = R.spans[1 - R.last_span];
+    HIPCHECK(hipEventRecord(span.start, R.stream));
     for (int done = 0; done < n;) {
         const int k = std::min(K, n - done);
         const int end = end_sample && done + k == n && k < V.depth ? 1 : 0;
@@ -2942,9 +2954,10 @@ int run_steps_noalloc(Runtime& R, int n, double* out)
             q += cnt;
         }
     }
-    HIPCHECK(hipEventRecord(R.ev1, R.stream));
-    HIPCHECK(hipEventSynchronize(R.ev1));
-    HIPCHECK(hipEventElapsedTime(&R.last_ms, R.ev0, R.ev1));
+    HIPCHECK(hipEventRecord(span.end, R.stream));
+    HIPCHECK(hipEventSynchronize(span.end));
+    HIPCHECK(hipEventElapsedTime(&R.last_ms, span.start, span.end));
+    R.last_span = 1 - R.last_span;
     R.ms_pending = false;
     // no kernel writes the samples of receivers in no element; the scratch
     // may hold another call's samples there
@@ -3048,8 +3061,8 @@ void fetch_states(Runtime& R, int q, int nnodes, double* u, double* up, const st
 float run_ms(Runtime& R)
 {
     if (R.ms_pending) {
-        HIPCHECK(hipEventSynchronize(R.ev1));
-        HIPCHECK(hipEventElapsedTime(&R.last_ms, R.ev0, R.ev1));
+        HIPCHECK(hipEventSynchronize(R.spans[R.last_span].end));
+        HIPCHECK(hipEventElapsedTime(&R.last_ms, R.spans[R.last_span].start, R.spans[R.last_span].end));
         R.ms_pending = false;
     }
     return R.last_ms;

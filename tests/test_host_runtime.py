@@ -1,0 +1,72 @@
+"""The library's host code without a device: error paths, launch shapes and
+allocations, under the HIP runtime of host_hip/ (which notes launches and runs
+no kernel)."""
+import os
+import subprocess
+import sys
+from pathlib import Path
+
+import pytest
+
+HERE = Path(__file__).resolve().parent
+PRELUDE = """
+import ctypes, sys
+sys.path.insert(0, {python!r})
+import numpy as np
+from damian_hip import cases, lib
+hh = ctypes.CDLL("libamdhip64.so.7")
+hh.hh_launches.restype = hh.hh_hostmallocs.restype = ctypes.c_char_p
+def launches():
+    return [l.split() for l in hh.hh_launches().decode().splitlines()]
+def fail(name, n=1):
+    hh.hh_fail(name.encode(), n)
+"""
+
+
+@pytest.fixture(scope="session")
+def host_hip(tmp_path_factory):
+    """Runs a script under that runtime; returns its standard output and the
+    layouts that the library says it built (dicts of numbers)."""
+    d = tmp_path_factory.mktemp("host_hip")
+    subprocess.run(["g++", "-std=c++17", "-O1", "-fPIC", "-shared", "-D__HIP_PLATFORM_AMD__", "-I/opt/rocm/include",
+                    HERE / "host_hip" / "host_hip.cpp", f"-Wl,--version-script={HERE / 'host_hip' / 'versions.map'}",
+                    "-Wl,-soname,libamdhip64.so.7", "-o", d / "libamdhip64.so.7"], check=True)
+
+    def run(script):
+        prelude = PRELUDE.format(python=str(HERE.parent / "damian.par_amd" / "python"))
+        r = subprocess.run([sys.executable, "-c", prelude + script], capture_output=True, text=True, timeout=300,
+                           env=dict(os.environ, LD_LIBRARY_PATH=str(d), DMP_LAYOUT_STATS="1"))
+        assert r.returncode == 0, r.stdout[-2000:] + r.stderr[-4000:]
+        layouts = []
+        for line in r.stderr.splitlines():
+            if line.startswith("layout "):
+                layouts.append({k: float(v) for k, v in (w.split("=") for w in line.split() if w.count("=") == 1 and "," not in w)})
+        return r.stdout, layouts
+
+    return run
+
+
+@pytest.mark.parametrize("name", ["f1", "c1"])
+def test_failed_call_leaves_last_run_ms(host_hip, name):
+    """The device time of the last complete call, whether it is asked for before
+    or after a call that fails part way (one tile, many tiles)."""
+    host_hip(f"""
+s = lib.Solver(cases.{name}())
+s.set_tuning(64, 1, 0, 2)
+s.run(10)
+launches()
+s.run(20)
+want = len(launches())
+for asked in (False, True):
+    if asked:
+        assert s.last_run_ms() == want
+    fail("hipLaunchKernel", 4)
+    try:
+        s.run(30)
+        raise SystemExit("not refused")
+    except lib.DmpError as e:
+        assert e.code == -3
+    assert s.last_run_ms() == want, (asked, s.last_run_ms(), want)
+s.run(6)
+assert 0 < s.last_run_ms() < want
+""")
