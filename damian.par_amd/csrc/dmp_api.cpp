@@ -384,6 +384,25 @@ struct Runtime {
         stream = nullptr;
     }
 
+    // Pinned host memory that kernels write.  Coherent (fine-grained) by request:
+    // the host reads samples and the completion word while the stream still
+    // runs, and sees the stores of earlier kernels, from every XCD, because
+    // such memory is not held in the L2s; a release writes back only the L2 of
+    // the XCD that makes it.
+    template <class T> T* pinned(size_t n, T** dev)
+    {
+        void *p = nullptr, *d = nullptr;
+        const hipError_t e = hipHostMalloc(&p, n * sizeof(T), hipHostMallocMapped | hipHostMallocCoherent);
+        if (e != hipSuccess)
+            throw fail(DMP_ENOMEM, "hipHostMalloc(%zu bytes) failed: %s", n * sizeof(T), hipGetErrorString(e));
+        if (hipHostGetDevicePointer(&d, p, 0) != hipSuccess) {
+            (void)hipHostFree(p);
+            throw fail(DMP_EHIP, "no device address of %zu pinned bytes", n * sizeof(T));
+        }
+        *dev = static_cast<T*>(d);
+        return static_cast<T*>(p);
+    }
+
     template <class T> T* dalloc(size_t n)
     {
         if (n == 0) n = 1;
@@ -2548,14 +2567,8 @@ void build_runtime(Runtime& R, const std::vector<Instance*>& insts)
             }
         }
     }
-    {
-        void* p = nullptr;
-        HIPCHECK(hipHostMalloc(&p, sizeof(uint32_t), hipHostMallocMapped));
-        R.done = static_cast<uint32_t*>(p);
-        *R.done = 0;
-        HIPCHECK(hipHostGetDevicePointer(&p, R.done, 0));
-        V.done = static_cast<uint32_t*>(p);
-    }
+    R.done = R.pinned<uint32_t>(1, &V.done);
+    *R.done = 0;
     V.ctrl = R.dalloc<Ctrl>(1);
     HIPCHECK(hipMemset(V.ctrl, 0, sizeof(Ctrl)));
     R.dev_base = 0;
@@ -2600,13 +2613,7 @@ void build_runtime(Runtime& R, const std::vector<Instance*>& insts)
         }
         R.d_node_int = R.upload(node_int);
         R.schunk = (int)std::min<size_t>(kStateChunk, most);
-        void* p = nullptr;
-        const size_t bytes = (size_t)kStateChunks * R.schunk * sizeof(double2);
-        const hipError_t e = hipHostMalloc(&p, bytes, hipHostMallocMapped);
-        if (e != hipSuccess) throw fail(DMP_ENOMEM, "hipHostMalloc(%zu bytes) failed: %s", bytes, hipGetErrorString(e));
-        R.sstage = static_cast<double2*>(p);
-        HIPCHECK(hipHostGetDevicePointer(&p, R.sstage, 0));
-        R.sstage_dev = static_cast<double2*>(p);
+        R.sstage = R.pinned<double2>((size_t)kStateChunks * R.schunk, &R.sstage_dev);
         for (hipEvent_t& ev : R.sev) HIPCHECK(hipEventCreateWithFlags(&ev, hipEventDisableTiming));
     }
     R.d_act_orig = R.upload(act_orig);
@@ -2711,12 +2718,7 @@ void alloc_ring(Runtime& R, int nsteps)
     const size_t want = (size_t)std::max(nsteps, 0) / I + 2;
     const size_t slots = std::max<size_t>(64, std::min(want, kRingBytes / (row * sizeof(double))));
     if (slots > (size_t)INT32_MAX) throw fail(DMP_EINVAL, "receiver ring too large");
-    void* p = nullptr;
-    const hipError_t e = hipHostMalloc(&p, slots * row * sizeof(double), hipHostMallocMapped);
-    if (e != hipSuccess)
-        throw fail(DMP_ENOMEM, "hipHostMalloc(%zu bytes) failed: %s", slots * row * sizeof(double),
-                   hipGetErrorString(e));
-    R.hstage = static_cast<double*>(p);
+    R.hstage = R.pinned<double>(slots * row, &R.V.recv_buf);
     R.hstage_cap = slots * row;
     // (the host's first touch maps each page: by several threads, 4 MiB at a time)
     constexpr size_t kPart = (size_t(4) << 20) / sizeof(double);
@@ -2725,9 +2727,6 @@ void alloc_ring(Runtime& R, int nsteps)
         const size_t lo = (size_t)i * kPart;
         std::memset(R.hstage + lo, 0, std::min(kPart, R.hstage_cap - lo) * sizeof(double));
     });
-    void* dp = nullptr;
-    HIPCHECK(hipHostGetDevicePointer(&dp, R.hstage, 0));
-    R.V.recv_buf = static_cast<double*>(dp);
     R.V.recv_cap = (int)slots;
     R.drop_graph();   // kernels capture the view by value
     prepare_graph(R);

@@ -1262,9 +1262,11 @@ __device__ void tile_steps(const DevView& V, int tile, int t0, int k, int end)
 
 // Tells the host that run call `call` is complete: the last kernel of the
 // call, in one workgroup, once its own stores are out.  What earlier kernels
-// of the call stored (samples in mapped host memory) precedes this kernel in
-// the stream, so that the release at system scope, which is cumulative, orders
-// it before the word too; the host reads the word with acquire.  It sees it
+// of the call stored (samples, from every XCD) was complete before this kernel
+// began, and ring and word are coherent host memory, which no L2 holds: so the
+// samples are in host memory before the word is.  (The release at system scope
+// orders this kernel's own stores; it writes back the L2 of its XCD, no other.)
+// The host reads the word with acquire.  It sees it
 // before an event recorded after the kernel: one-step calls of the 861-node
 // layer 22.0 -> 19.4 us, 20-step calls of the canyon quadtree 83.4 -> 80.0.
 // Every wavefront waits for its own stores, one makes the release: a release

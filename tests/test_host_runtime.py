@@ -70,3 +70,16 @@ for asked in (False, True):
 s.run(6)
 assert 0 < s.last_run_ms() < want
 """)
+
+
+def test_pinned_memory_is_coherent(host_hip):
+    """The host reads the receiver ring and the completion word before the
+    stream is idle, so both ask for coherent memory by name."""
+    out, _ = host_hip("""
+s = lib.Solver(cases.f1())
+print(hh.hh_hostmallocs().decode())
+""")
+    mapped, coherent = 0x2, 0x40000000
+    made = [(int(a), int(b)) for a, b in (l.split() for l in out.splitlines() if l)]
+    assert sorted(n for n, _ in made)[0] == 4 and len(made) == 3
+    assert all(f == mapped | coherent for _, f in made)
