@@ -303,8 +303,6 @@ struct Runtime {
     std::vector<int> inst_na, inst_nrecv;
     PackedHost host;
     int tiles_block = 0, tiles_depth = 0;   // shape the tile arrays were built for
-    bool own_shape = true;         // the shape is dmp_init's, not one that the caller or the autotuner chose
-    bool tiles_own = true;         // own_shape when the tile arrays were built
     bool no_whole = false;         // the mesh does not fit in one tile after all
     bool no_patches = false;       // the tiles between patches do not fit
     bool whole = false;            // one tile holds the mesh: no rings, up to V.depth steps per launch
@@ -1250,13 +1248,15 @@ bool try_tiles(Runtime& R, std::vector<int>& halves, int pass)
     // A mesh that one workgroup holds needs no rings, so a launch of several
     // steps may take any number of them; what they read ahead (forces and free
     // field) shares the LDS.  Where the caller asks for several steps per
-    // launch and tiles that small a mesh fits in, or has left the shape to the
-    // library, such a mesh is one tile: the two-material valley of 358 nodes
+    // launch and tiles that small a mesh fits in, or for dmp_init's own shape
+    // (also where the caller sets what dmp_get_tuning gave), such a mesh is one
+    // tile: the two-material valley of 358 nodes
     // takes 1.79 us a step in FP32C so, 3.2 in two tiles at three steps per
     // launch and 2.3 at eight; the layer of 861 nodes 1.91 against 2.56 and 1.83
     // in FP64, 1.78 against 2.50 and 1.74 in FP32C, in half the launches.
     // Descriptors address no more slots.
-    R.whole = K > 1 && NA <= kMaxSlots && (R.tuning[0] >= NA || R.own_shape) && !R.no_whole;
+    const bool init_shape = R.tuning[0] == R.init_tuning[0] && K == R.init_tuning[3];
+    R.whole = K > 1 && NA <= kMaxSlots && (R.tuning[0] >= NA || init_shape) && !R.no_whole;
     const int B = R.whole ? std::max(NA, 1) : K == 1 && !R.no_patches ? std::min(R.tuning[0], kRestBlock) : R.tuning[0];
     int ntiles = (NA + B - 1) / B;
     const int NR = (int)H.recv.size();
@@ -2035,15 +2035,15 @@ bool try_tiles(Runtime& R, std::vector<int>& halves, int pass)
         ring = (double)ring_gid.size();
         int elem_tiles = 0;
         for (const TileInfo& T : tiles) elem_tiles += T.mat_mode;
-        std::fprintf(stderr, "layout B=%d K=%d tiles=%d threads=%d mean_ent=%.1f ring/core=%.3f lds=%zu "
+        std::fprintf(stderr, "layout B=%d K=%d whole=%d depth=%d tiles=%d threads=%d mean_ent=%.1f ring/core=%.3f lds=%zu "
                      "slots=%d vrows=%d virt=%d force=%d side=%d recv=%d elem_tiles=%d hist=",
-                     B, K, ntiles, V.threads, ent / std::max(ntiles, 1), ring / std::max(NA, 1), lds,
+                     B, K, R.whole, V.depth, ntiles, V.threads, ent / std::max(ntiles, 1), ring / std::max(NA, 1), lds,
                      V.lds_slots, V.lds_vrows, V.lds_virt, V.lds_force, V.lds_side,
                      V.lds_recv, elem_tiles);
         for (int h : hist) std::fprintf(stderr, "%d,", h);
         int with_vrow = 0;
         for (const TileInfo& T : tiles) with_vrow += T.n_vrow > 0;
-        std::fprintf(stderr, " tiles with hanging-node rows %d, patches %d\n", with_vrow, V.patches);
+        std::fprintf(stderr, " tiles with hanging-node rows %d, patches=%d\n", with_vrow, V.patches);
     }
     if (lds > R.lds_limit)
         throw fail(DMP_EUNSUPPORTED, "tiles of %d nodes for %d steps per launch need %zu B of LDS "
@@ -2166,7 +2166,6 @@ bool try_tiles(Runtime& R, std::vector<int>& halves, int pass)
     R.state_depth = K;
     R.tiles_block = R.tuning[0];
     R.tiles_depth = K;
-    R.tiles_own = R.own_shape;
     return true;
 }
 
@@ -2180,7 +2179,7 @@ void prepare_graph(Runtime& R);
 
 void Runtime::apply_tuning()
 {
-    if (tiles_block != tuning[0] || tiles_depth != tuning[3] || tiles_own != own_shape) {
+    if (tiles_block != tuning[0] || tiles_depth != tuning[3]) {
         no_whole = no_patches = false;
         try {
             build_tiles(*this);
@@ -2202,8 +2201,6 @@ void Runtime::apply_tuning()
 void set_tuning(Runtime& R, const int* t)
 {
     int old[4];
-    const bool old_own = R.own_shape;
-    R.own_shape = !t;
     for (int k = 0; k < 4; ++k) {
         old[k] = R.tuning[k];
         R.tuning[k] = t ? t[k] : R.init_tuning[k];
@@ -2211,7 +2208,6 @@ void set_tuning(Runtime& R, const int* t)
     try {
         R.apply_tuning();
     } catch (const Error&) {
-        R.own_shape = old_own;
         for (int k = 0; k < 4; ++k) R.tuning[k] = old[k];
         R.apply_tuning();
         throw;
@@ -2642,8 +2638,8 @@ void build_runtime(Runtime& R, const std::vector<Instance*>& insts)
     const int shapes[][2] = {{256, small ? 3 : 1}, {256, 2}, {128, 3}, {128, 2}, {256, 1}, {128, 1}, {64, 1}};
     bool ok = false;
     for (const auto& sh : shapes) {
-        R.tuning[0] = sh[0];
-        R.tuning[3] = sh[1];
+        R.tuning[0] = R.init_tuning[0] = sh[0];
+        R.tuning[3] = R.init_tuning[3] = sh[1];
         try {
             R.apply_tuning();
             ok = true;
@@ -3134,7 +3130,6 @@ void autotune(Runtime& R, int nsteps, int* out)
         R.step = step0;
     };
     int best[4] = {R.tuning[0], R.tuning[1], R.tuning[2], R.tuning[3]};
-    R.own_shape = false;
     double best_t = 1e300;
     // tile sizes: 64, 128, 256, and those giving one or two tiles per compute
     // unit (small meshes are latency-bound: one tile per CU, no CU twice)

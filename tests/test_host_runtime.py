@@ -40,7 +40,7 @@ def host_hip(tmp_path_factory):
         layouts = []
         for line in r.stderr.splitlines():
             if line.startswith("layout "):
-                layouts.append({k: float(v) for k, v in (w.split("=") for w in line.split() if w.count("=") == 1 and "," not in w)})
+                layouts.append({k: float(v) for k, v in (w.rstrip(",").split("=") for w in line.split() if w.count("=") == 1 and not w.startswith("hist="))})
         return r.stdout, layouts
 
     return run
@@ -83,3 +83,35 @@ print(hh.hh_hostmallocs().decode())
     made = [(int(a), int(b)) for a, b in (l.split() for l in out.splitlines() if l)]
     assert sorted(n for n, _ in made)[0] == 4 and len(made) == 3
     assert all(f == mapped | coherent for _, f in made)
+
+
+@pytest.mark.parametrize("name", ["f1", "f2"])
+def test_shape_that_was_got_can_be_set(host_hip, name):
+    """Setting the shape that dmp_get_tuning gave (a small mesh in one tile), or
+    going back to dmp_init's, gives that layout again; where it is still in
+    place nothing is built."""
+    out, layouts = host_hip(f"""
+s = lib.Solver(cases.{name}())
+t = s.tuning()
+s.set_tuning(*t)
+s.set_tuning(64, 1, 0, 2)
+s.set_tuning(*t)
+lib.lib().dmp_set_tuning(s.h, None)
+s.set_tuning(*t)
+launches()
+s.run(40)
+print(len([l for l in launches() if "step_kernel" in l[0]]))
+""")
+    assert [(l["K"], l["whole"]) for l in layouts] == [(3, 1), (2, 0), (3, 1)]
+    assert layouts[0] == layouts[2] and layouts[0]["depth"] > 8
+    assert int(out) == -(-40 // layouts[0]["depth"])
+
+
+def test_same_shape_of_a_large_mesh_is_not_built_again(host_hip):
+    _, layouts = host_hip("""
+s = lib.Solver(cases.c1())
+s.set_tuning(256, 1, 0, 3)
+s.set_tuning(256, 0, 12, 3)
+lib.lib().dmp_set_tuning(s.h, None)
+""")
+    assert len(layouts) == 1
