@@ -3098,7 +3098,7 @@ void check_tuning(const int* t)
 
 // Runs every candidate shape for nsteps steps from a saved state, once to
 // warm up and twice timed; keeps the shape with the shortest timed run.  The
-// state (both levels, step) is restored.
+// state (both levels, step) is restored, on failure the shape too.
 void autotune(Runtime& R, int nsteps, int* out)
 {
     if (nsteps <= 0) throw fail(DMP_EINVAL, "autotune needs a positive step count");
@@ -3121,7 +3121,6 @@ void autotune(Runtime& R, int nsteps, int* out)
         HIPCHECK(hipMemcpyAsync(save[q], R.V.U[state_slot(step0 - q, R.state_depth)], ub, hipMemcpyDeviceToDevice,
                                 R.stream));
     }
-    const bool fr0 = R.first_run;
     auto restore = [&]() {
         for (int q = 0; q < 2; ++q)
             HIPCHECK(hipMemcpyAsync(R.V.U[state_slot(step0 - q, R.state_depth)], save[q], ub,
@@ -3130,6 +3129,24 @@ void autotune(Runtime& R, int nsteps, int* out)
         R.step = step0;
     };
     int best[4] = {R.tuning[0], R.tuning[1], R.tuning[2], R.tuning[3]};
+    struct Undo {
+        Runtime& R;
+        const std::function<void()> undo;
+        const int tuning[4];
+        const bool first_run;
+        bool done = false;
+        ~Undo()
+        {
+            R.first_run = first_run;
+            if (done) return;
+            std::copy(tuning, tuning + 4, R.tuning);
+            try {
+                R.apply_tuning();
+                undo();
+            } catch (...) {   // the error on its way out says what failed
+            }
+        }
+    } undo{R, restore, {best[0], best[1], best[2], best[3]}, R.first_run};
     double best_t = 1e300;
     // tile sizes: 64, 128, 256, and those giving one or two tiles per compute
     // unit (small meshes are latency-bound: one tile per CU, no CU twice)
@@ -3211,7 +3228,7 @@ void autotune(Runtime& R, int nsteps, int* out)
     for (int k = 0; k < 4; ++k) R.tuning[k] = best[k];
     R.apply_tuning();
     restore();
-    R.first_run = fr0;
+    undo.done = true;
     if (out)
         for (int k = 0; k < 4; ++k) out[k] = best[k];
 }

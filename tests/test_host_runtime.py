@@ -115,3 +115,31 @@ s.set_tuning(256, 0, 12, 3)
 lib.lib().dmp_set_tuning(s.h, None)
 """)
     assert len(layouts) == 1
+
+
+@pytest.mark.parametrize("what,n", [("hipLaunchKernel", 500), ("hipMalloc", 100)])
+def test_failed_autotune_leaves_shape_and_state(host_hip, what, n):
+    """A search that fails part way gives back the shape, the step and the
+    state (a launch that fails; memory that runs out while a layout is built)."""
+    host_hip(f"""
+s = lib.Solver(cases.c1())
+s.set_tuning(100, 0, 12, 2)
+launches()
+s.run(7, record=False)
+want = s.tuning()
+kernels = {{tuple(l) for l in launches() if "step_kernel" in l[0]}}
+fail({what!r}, {n})
+try:
+    s.autotune(20)
+    raise SystemExit("not refused")
+except lib.DmpError as e:
+    assert e.code in (-2, -3), e
+assert s.tuning() == want, s.tuning()
+step = ctypes.c_int()
+lib.lib().dmp_get_step(s.h, ctypes.byref(step))
+assert step.value == 7, step.value
+launches()
+out = s.run(6)
+assert out.shape[0] == 6
+assert {{tuple(l) for l in launches() if "step_kernel" in l[0]}} == kernels
+""")
