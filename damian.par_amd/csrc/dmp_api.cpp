@@ -24,6 +24,7 @@
 #include <memory>
 #include <numeric>
 #include <string>
+#include <system_error>
 #include <thread>
 #include <unordered_map>
 #include <vector>
@@ -509,6 +510,19 @@ int setup_threads()
     return (int)std::max(1u, std::min(hw, 16u));
 }
 
+// Starts threads f(1) .. f(n - 1) (f(0) is the caller's) into pool; returns how
+// many of the n there are, fewer where the system gives no more.
+template <class F> int start_threads(std::vector<std::thread>& pool, int n, F&& f)
+{
+    int started = 1;
+    pool.reserve(std::max(n - 1, 0));
+    try {
+        for (; started < n; ++started) pool.emplace_back(f, started);
+    } catch (const std::system_error&) {
+    }
+    return started;
+}
+
 // f(i) for i in [0, n) on up to nthreads threads taking indices in order;
 // the first exception thrown (lowest index) is rethrown after all threads end.
 template <class F> void parallel_items(int n, int nthreads, F&& f)
@@ -520,7 +534,7 @@ template <class F> void parallel_items(int n, int nthreads, F&& f)
     }
     std::atomic<int> next{0};
     std::vector<std::exception_ptr> errs(n);
-    auto work = [&]() {
+    auto work = [&](int) {
         for (int i = next++; i < n; i = next++) {
             try {
                 f(i);
@@ -530,8 +544,8 @@ template <class F> void parallel_items(int n, int nthreads, F&& f)
         }
     };
     std::vector<std::thread> pool;
-    for (int t = 1; t < nthreads; ++t) pool.emplace_back(work);
-    work();
+    start_threads(pool, nthreads, work);
+    work(0);
     for (auto& t : pool) t.join();
     for (auto& e : errs)
         if (e) std::rethrow_exception(e);
@@ -3038,12 +3052,17 @@ void fetch_states(Runtime& R, int q, int nnodes, double* u, double* up, const st
     };
     int launched = 0;
     for (; launched < std::min(np, kStateChunks); ++launched) launch(launched);
-    for (int w = 1; w < nthr; ++w) pool.t.emplace_back(work, w);
-    move_mass(0);
+    // this thread's shares: the first, and those of threads that did not start
+    const int started = start_threads(pool.t, nthr, work);
+    auto mine = [&](auto&& f) {
+        f(0);
+        for (int w = started; w < nthr; ++w) f(w);
+    };
+    mine(move_mass);
     for (int i = 0; i < np; ++i) {
         wait_event(R.sev[i % kStateChunks]);
         ready.store(i + 1, std::memory_order_release);
-        move(0, i);
+        mine([&](int w) { move(w, i); });
         if (launched < np) {   // the next piece takes this one's chunk
             while (left[i].load(std::memory_order_acquire) > 0) std::this_thread::yield();
             launch(launched++);

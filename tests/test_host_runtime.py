@@ -143,3 +143,29 @@ out = s.run(6)
 assert out.shape[0] == 6
 assert {{tuple(l) for l in launches() if "step_kernel" in l[0]}} == kernels
 """)
+
+
+def test_state_download_without_threads(host_hip):
+    """Host threads only speed a large download up: where none can be started
+    (no address space for a stack) the call still moves every byte."""
+    host_hip("""
+import os, resource
+os.environ["DMP_THREADS"] = "1"
+case = cases.c4_valley(200.0)
+s = lib.Solver(case)
+n = case.mesh.nnodes
+a = [np.full(2 * n, np.nan) for _ in range(3)]
+os.environ["DMP_THREADS"] = "8"
+size = int(open("/proc/self/statm").read().split()[0]) * os.sysconf("SC_PAGE_SIZE")
+resource.setrlimit(resource.RLIMIT_AS, (size + (2 << 20), resource.RLIM_INFINITY))
+import threading
+try:
+    threading.Thread(target=int).start()
+    raise SystemExit("a thread can be started: nothing is tested")
+except RuntimeError:
+    pass
+rc = lib.lib().dmp_get_state(s.h, *[x.ctypes.data_as(ctypes.c_void_p) for x in a])
+resource.setrlimit(resource.RLIMIT_AS, (resource.RLIM_INFINITY, resource.RLIM_INFINITY))
+assert rc == 0, lib.last_error(s.h)
+assert all(np.isfinite(x).all() for x in a)
+""")
