@@ -69,6 +69,14 @@ constexpr double kTuneMinSeconds = 2e-3;
 constexpr int kRestBlock = 64;
 constexpr int kPatchWaves = 4;
 
+// Receivers up to which the receivers-only kernel is one workgroup, which can
+// report the end of the call itself.  Above, one compute unit's dependent loads
+// and host stores take longer than the event costs (calls of 3 steps of a
+// 60,501-node layer, receivers all over it, FP64, one workgroup against 256
+// receivers each: 500 receivers 23.2 and 26.4 us, 800 26.5 and 27.5, 1024 29.0
+// and 28.3, 1800 37.6 and 31.6, 6500 87 and 51).
+constexpr int kRecvOne = 896;
+
 // Steps per launch of a mesh that one workgroup holds whole (build_tiles).
 constexpr int kWholeSteps = 32;
 
@@ -2891,7 +2899,7 @@ int run_steps(Runtime& R, int n, double* out)
     if (end_sample && !end_done) {
         ensure_tables(R, s + n, s + n);
         before(q_hi);
-        call = ++R.calls ? R.calls : ++R.calls;   // never 0
+        if (V.nrecv <= kRecvOne) call = ++R.calls ? R.calls : ++R.calls;   // never 0
         HIPCHECK(launch_recv(V, R.precision, s + n, call, R.stream));
         after(q_hi + 1);
     }

@@ -1329,12 +1329,12 @@ void step_kernel(DevView V, int t0_arg, int use_base, int k, int end, uint32_t c
 
 // Receivers at step j (j % recv_interval == 0) straight from the state level
 // in HBM: the last step of a run call, which no step launch of the call
-// starts from.  One workgroup; call: as report_done, or 0.
+// starts from.  call: as report_done (one workgroup), or 0.
 template <class P>
 __global__ __launch_bounds__(kMaxThreads) void recv_kernel(DevView V, int j, uint32_t call)
 {
     const void* U = V.U[state_slot(j, V.depth)];
-    for (int r = (int)threadIdx.x; r < V.nrecv; r += (int)blockDim.x) {
+    for (int r = (int)(blockIdx.x * blockDim.x + threadIdx.x); r < V.nrecv; r += (int)(gridDim.x * blockDim.x)) {
         const RecvG g = V.rg[r];
         double fx = 0.0, fz = 0.0;
         if (g.found) {
@@ -1523,11 +1523,13 @@ hipError_t launch_step(const DevView& V, int precision, int t0, int use_base, in
 hipError_t launch_recv(const DevView& V, int precision, int j, uint32_t call, hipStream_t st)
 {
     if (V.nrecv <= 0) return hipSuccess;
-    const dim3 block(std::min(kMaxThreads, (V.nrecv + 63) / 64 * 64));
+    // one workgroup where it reports the end of the call, else as many as fill the chip
+    const dim3 block(std::min(call ? kMaxThreads : 256, (V.nrecv + 63) / 64 * 64));
+    const dim3 grid(call ? 1 : (V.nrecv + (int)block.x - 1) / (int)block.x);
     if (precision == 0)
-        hipLaunchKernelGGL(recv_kernel<PF64>, dim3(1), block, 0, st, V, j, call);
+        hipLaunchKernelGGL(recv_kernel<PF64>, grid, block, 0, st, V, j, call);
     else
-        hipLaunchKernelGGL(recv_kernel<PF32C>, dim3(1), block, 0, st, V, j, call);
+        hipLaunchKernelGGL(recv_kernel<PF32C>, grid, block, 0, st, V, j, call);
     return hipGetLastError();
 }
 

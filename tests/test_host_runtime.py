@@ -169,3 +169,23 @@ resource.setrlimit(resource.RLIMIT_AS, (resource.RLIM_INFINITY, resource.RLIM_IN
 assert rc == 0, lib.last_error(s.h)
 assert all(np.isfinite(x).all() for x in a)
 """)
+
+
+@pytest.mark.parametrize("nrecv,groups", [(1, 1), (896, 1), (897, 4), (2000, 8)])
+def test_receivers_only_kernel_grows_with_its_receivers(host_hip, nrecv, groups):
+    out, _ = host_hip(f"""
+import copy
+case = copy.copy(cases.c1())
+case.recv_elem = np.resize(case.recv_elem, {nrecv})
+case.recv_xy = np.resize(case.recv_xy, ({nrecv}, 2))
+case.recv_ff = np.resize(case.recv_ff, {nrecv})
+s = lib.Solver(case)
+s.set_tuning(256, 1, 0, 3)
+for noalloc in (False, True):
+    launches()
+    s.run(3, noalloc=noalloc)
+    print(*[l[1:3] for l in launches() if "recv_kernel" in l[0]])
+""")
+    run, noalloc = [eval(l) for l in out.splitlines()]
+    assert int(run[0]) == groups and int(run[0]) * int(run[1]) >= nrecv
+    assert int(noalloc[0]) * int(noalloc[1]) >= nrecv > (int(noalloc[0]) - 1) * int(noalloc[1])
