@@ -60,14 +60,31 @@ constexpr double kAnchorWeight = 5.0;
 constexpr int kTuneMaxRuns = 15;
 constexpr double kTuneMinSeconds = 2e-3;
 
-// One-step layouts: nodes per tile outside patches (at most), and wavefronts
-// per workgroup.  A workgroup's LDS is what the larger of a tile and four
-// patches needs: tiles of 64 nodes need no more than the patches, so that these
-// fill the compute units (2.47M-element sweep, FP32C, tiles of 32, 64, 128 and
-// 256 nodes: 26.4, 24.2, 30.8 and 28.7 us a step).  One and two wavefronts: 25.5
-// and 25.5 (the uniform canyon 11.1 and 10.6 against 10.8 with four).
+// One-step layouts: nodes per compute unit up to which the mesh is plain tiles.
+// Such a launch is a chain of loads, in which the list of nodes outside patches
+// is one more: graphs of the 40,501-node layer 5.65 us a step in plain tiles of
+// 256, 5.90 with patches (FP32C 5.79, 6.13), the 36,000-node basin 6.76 and 7.01
+// (7.13, 7.35).  They meet at 140,000 to 180,000 nodes (basin of 141,541 7.40
+// and 7.21, without XCD remap 7.70 and 7.95; layer of 180,901 6.39 and 6.24,
+// FP32C 6.36 and 6.42); 349,657 nodes 10.5 and 7.7.
+constexpr int kPlainNodes = 768;
+// Above: nodes per tile outside patches (at most), and wavefronts per workgroup.
+// A workgroup's LDS is what the larger of a tile and four patches needs: tiles
+// of 64 nodes need no more than the patches, so that these fill the compute
+// units (2.47M-element sweep, 3 % of the nodes outside, FP32C, tiles of 32, 64,
+// 128 and 256 nodes: 26.4, 24.2, 30.8 and 28.7 us a step).  One and two
+// wavefronts: 25.5 and 25.5 (the uniform canyon 11.1 and 10.6 against 10.8 with
+// four).
 constexpr int kRestBlock = 64;
 constexpr int kPatchWaves = 4;
+// Where more than one node in kManyRest is outside patches (hanging nodes all
+// over the mesh) the tiles are the work: larger ones read fewer ring nodes, and
+// the workgroup is no wider than they need.  470,000 to 670,000 nodes, shares of 9, 15, 26 and
+// 54 %, FP32C, tiles of 64 in four wavefronts against 128: 10.6 and 10.4,
+// 11.6 and 10.6, 14.9 and 11.5, 19.7 and 15.6 us a step (plain tiles of 256:
+// 21.8, 23.4, 23.6 and 21.4); no patches at all 24.0 and 17.2 (17.8).
+constexpr int kManyRest = 8;
+constexpr int kManyRestBlock = 128;
 
 // Receivers up to which the receivers-only kernel is one workgroup, which can
 // report the end of the call itself.  Above, one compute unit's dependent loads
@@ -1279,7 +1296,7 @@ bool try_tiles(Runtime& R, std::vector<int>& halves, int pass)
     // Descriptors address no more slots.
     const bool init_shape = R.tuning[0] == R.init_tuning[0] && K == R.init_tuning[3];
     R.whole = K > 1 && NA <= kMaxSlots && (R.tuning[0] >= NA || init_shape) && !R.no_whole;
-    const int B = R.whole ? std::max(NA, 1) : K == 1 && !R.no_patches ? std::min(R.tuning[0], kRestBlock) : R.tuning[0];
+    int B = R.whole ? std::max(NA, 1) : R.tuning[0];
     int ntiles = (NA + B - 1) / B;
     const int NR = (int)H.recv.size();
     const int NFF = (int)H.ff.size();
@@ -1297,13 +1314,15 @@ bool try_tiles(Runtime& R, std::vector<int>& halves, int pass)
     int ncu = 0;
     if (hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, R.device) != hipSuccess || ncu < 1)
         ncu = 256;
-    // Uniform parts of the mesh as patches: always at one step per launch; at
+    // Uniform parts of the mesh as patches: at one step per launch in meshes of
+    // more than kPlainNodes per compute unit; at
     // several where there are more tiles than compute units, so that work in
     // flight and not the slowest tile's latency bounds a launch.
     // One step per launch: tiles of B nodes each of the list of nodes outside
     // patches.
     PatchRuns patches;
     PatchCells cells;
+    bool many_rest = false;
     std::vector<int> gen_of(K == 1 ? NA : 0, -1);   // place of a node in that list
     if (K == 1 || (ntiles > ncu && !R.whole)) {
         std::vector<char> taken(NA, 0);
@@ -1311,15 +1330,15 @@ bool try_tiles(Runtime& R, std::vector<int>& halves, int pass)
             const int c = x.c[0];
             if (c >= 0) taken[c < NA ? c : H.vanch[c - NA].x] = 1;
         }
-        if (R.no_patches) {
-            if (K == 1) {
-                cells.rest.resize(NA);
-                std::iota(cells.rest.begin(), cells.rest.end(), 0);
-            }
-        } else if (K == 1) {
-            cells = find_cells(H, NA, taken);
+        if (K > 1) {
+            if (!R.no_patches) patches = find_patches(H, NA, taken, kBlockPatch, K);
+        } else if (R.no_patches || NA <= (long)kPlainNodes * ncu) {
+            cells.rest.resize(NA);
+            std::iota(cells.rest.begin(), cells.rest.end(), 0);
         } else {
-            patches = find_patches(H, NA, taken, kBlockPatch, K);
+            cells = find_cells(H, NA, taken);
+            many_rest = cells.rest.size() * kManyRest > (size_t)NA;
+            if (!cells.patch.empty()) B = std::min(B, many_rest ? kManyRestBlock : kRestBlock);
         }
         for (size_t i = 0; i < cells.rest.size(); ++i) gen_of[cells.rest[i]] = (int)i;
     }
@@ -1980,7 +1999,7 @@ bool try_tiles(Runtime& R, std::vector<int>& halves, int pass)
         V.threads = std::max(V.threads, (w * w + 63) / 64 * 64);
         if (V.threads > kMaxThreads) throw fail(DMP_EUNSUPPORTED, "patches need %d threads (max %d)", V.threads, kMaxThreads);
     }
-    if (K == 1 && V.patches) V.threads = std::max(V.threads, 64 * kPatchWaves);
+    if (K == 1 && V.patches && !many_rest) V.threads = std::max(V.threads, 64 * kPatchWaves);
     const int per_block = K == 1 ? V.threads / 64 : 1;
     V.patch_blocks = (V.patches + per_block - 1) / per_block;
     std::vector<PatchT> patch = std::move(cells.patch);
@@ -2065,7 +2084,7 @@ bool try_tiles(Runtime& R, std::vector<int>& halves, int pass)
         for (int h : hist) std::fprintf(stderr, "%d,", h);
         int with_vrow = 0;
         for (const TileInfo& T : tiles) with_vrow += T.n_vrow > 0;
-        std::fprintf(stderr, " tiles with hanging-node rows %d, patches=%d\n", with_vrow, V.patches);
+        std::fprintf(stderr, " tiles with hanging-node rows %d, patches=%d rest=%d\n", with_vrow, V.patches, K == 1 ? NG : NA - V.patches * kBlockPatchNodes);
     }
     if (lds > R.lds_limit)
         throw fail(DMP_EUNSUPPORTED, "tiles of %d nodes for %d steps per launch need %zu B of LDS "
@@ -2095,7 +2114,7 @@ bool try_tiles(Runtime& R, std::vector<int>& halves, int pass)
     }
     V.block = B;
     V.ngen = NG;
-    V.core_gid = K == 1 ? R.upload_tile(cells.rest) : nullptr;
+    V.core_gid = K == 1 && V.patches ? R.upload_tile(cells.rest) : nullptr;
     V.tiles = R.upload_tile(tiles);
     V.patch = R.upload_tile(patch);
     V.patch_ring = R.upload_tile(patch_ring);

@@ -331,11 +331,11 @@ struct DevView {
     const int* patch_ring;    // per patch the nodes around it: kPatchRing (-1: none there), or the block patch's ring entries
     const int* patch_list;    // kPatchNodes per listed patch
     const void* node_coef;    // per active node: 1 / mfull (plain nodes)
-    // one-step layouts: tiles are `block` nodes each of a list of the nodes
-    // outside patches; what a tile loads is at a fixed stride per tile, so that
+    // one-step layouts: tiles are `block` nodes each, with patches of a list of
+    // the nodes outside them (core_gid); what a tile loads is at a fixed stride per tile, so that
     // no load waits for the tile record to know its address
     const int* core_gid;
-    int block, ngen;          // nodes per tile, nodes in the list
+    int block, ngen;          // nodes per tile, nodes that tiles have
     int ring_cap;
     const int* recv_ff;       // lds_recv per tile: free-field point of its receivers, or -1
     uint32_t* done;           // mapped host word: number of the last run call whose work is complete

@@ -793,8 +793,8 @@ __device__ __forceinline__ void block_patch_steps(const DevView& V, int t, int k
 
 // ONE: the layout has depth 1 (one step per launch): two LDS buffers, no
 // rotation, side records read straight into registers.  HANG: the layout has
-// hanging nodes.
-template <class P, bool ONE, bool HANG>
+// hanging nodes.  LISTED: a one-step layout's tiles take their nodes from a list.
+template <class P, bool ONE, bool HANG, bool LISTED>
 __device__ void tile_steps(const DevView& V, int tile, int t0, int k, int end)
 {
     using R = typename P::real;
@@ -884,7 +884,7 @@ __device__ void tile_steps(const DevView& V, int tile, int t0, int k, int end)
         node_t cu{}, cp{};
         uint4 d0{};
         if (e < cnt) {
-            gid = V.core_gid[n0 + e];
+            if (LISTED) gid = V.core_gid[n0 + e];
             d0 = V.core_desc[n0 + e];
             cf = P::coef(V.core_coef, n0 + e);
         }
@@ -1323,7 +1323,7 @@ void step_kernel(DevView V, int t0_arg, int use_base, int k, int end, uint32_t c
     }
     const int tile = V.xcd_remap ? (b & 7) * V.tiles_per_xcd + (b >> 3) : b;
     if (tile >= V.node_tiles) return;   // whole block exits together
-    tile_steps<P, ONE, HANG>(V, tile, t0, k, end);
+    tile_steps<P, ONE, HANG, ONE && PARTS == Parts::kPatches>(V, tile, t0, k, end);
     if (PARTS == Parts::kWhole) report_done(V, call);
 }
 
@@ -1493,10 +1493,12 @@ static void launch_one(const DevView& V, int grid, size_t lds, hipStream_t st, i
     // without their phases, their barrier and a quarter of the registers
     // (40,000-element layer, FP64, 3 steps per launch: 2.58 us a step against
     // 2.98 with the other); layouts of tiles only, where the slowest tile
-    // bounds the launch, one without the branch to patches and the report of
-    // the call's end (canyon quadtree, FP32C: 3.21 against 3.23)
+    // bounds the launch, one without the branch to patches, the list of nodes
+    // between them and the report of the call's end (canyon quadtree, FP32C:
+    // 3.21 against 3.23; 40,000-element layer, 5.72 and 5.57 at one step per launch)
     const Parts parts = V.patches ? Parts::kPatches : call ? Parts::kWhole : Parts::kTiles;
-    if (V.depth == 1) go(step_kernel<P, true, true, Parts::kPatches>);
+    if (V.depth == 1 && parts == Parts::kPatches) go(step_kernel<P, true, true, Parts::kPatches>);
+    else if (V.depth == 1) go(step_kernel<P, true, true, Parts::kTiles>);
     else if (V.nv > 0 && parts == Parts::kPatches) go(step_kernel<P, false, true, Parts::kPatches>);
     else if (V.nv > 0 && parts == Parts::kWhole) go(step_kernel<P, false, true, Parts::kWhole>);
     else if (V.nv > 0) go(step_kernel<P, false, true, Parts::kTiles>);
@@ -1549,13 +1551,15 @@ hipError_t launch_state(int precision, const void* U, const int* node_int, const
 // budget (the most any layout may then need).
 hipError_t configure_kernels(size_t* max_lds)
 {
-    const void* fns[] = {reinterpret_cast<const void*>(step_kernel<PF64, true, true, Parts::kPatches>),
+    const void* fns[] = {reinterpret_cast<const void*>(step_kernel<PF64, true, true, Parts::kTiles>),
+                         reinterpret_cast<const void*>(step_kernel<PF64, true, true, Parts::kPatches>),
                          reinterpret_cast<const void*>(step_kernel<PF64, false, true, Parts::kTiles>),
                          reinterpret_cast<const void*>(step_kernel<PF64, false, true, Parts::kPatches>),
                          reinterpret_cast<const void*>(step_kernel<PF64, false, true, Parts::kWhole>),
                          reinterpret_cast<const void*>(step_kernel<PF64, false, false, Parts::kTiles>),
                          reinterpret_cast<const void*>(step_kernel<PF64, false, false, Parts::kPatches>),
                          reinterpret_cast<const void*>(step_kernel<PF64, false, false, Parts::kWhole>),
+                         reinterpret_cast<const void*>(step_kernel<PF32C, true, true, Parts::kTiles>),
                          reinterpret_cast<const void*>(step_kernel<PF32C, true, true, Parts::kPatches>),
                          reinterpret_cast<const void*>(step_kernel<PF32C, false, true, Parts::kTiles>),
                          reinterpret_cast<const void*>(step_kernel<PF32C, false, true, Parts::kPatches>),

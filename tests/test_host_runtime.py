@@ -16,6 +16,21 @@ import numpy as np
 from damian_hip import cases, lib
 hh = ctypes.CDLL("libamdhip64.so.7")
 hh.hh_launches.restype = hh.hh_hostmallocs.restype = ctypes.c_char_p
+def layer(nx, nz):
+    w, h = 5.0 * nx, 5.0 * nz
+    t = cases.problem_text(w, h, 0.4, 0.002, 0.1, 10, 2.5, [("p", 1000, "s", 500, 2000)], "WAVESV",
+                           [0.6 * w, 0.6 * h, 0.5 * w, 0, 1, 0.2, 0.2, 1.0, 5.0])
+    return cases.S.case_from_problem_text(t, sheet=(-3.3, w - 10.0, 19.1), name="layer")
+def fronts(nx, nz, part, seed=7):
+    # 10 m cells, halved everywhere but in the first `part` of the width, there at random
+    w, h = 10.0 * nx, 10.0 * nz
+    t = cases.problem_text(w, h, 1.0, 0.002, 0.2, 10, 5.0, [("p", 1000, "s", 500, 2000)], "WAVESV",
+                           [0.6 * w, 0.6 * h, 0.5 * w, 0, 1, 0.3, 0.0, 1.0, 3.0])
+    mdl = cases.S.build_model(cases.S.parse_problem(t))
+    rng = np.random.default_rng(seed)
+    m = cases.S.quadtree_mesh(mdl.totcols - 1, mdl.totrows - 1, mdl.blength, 2,
+                              lambda x, z, s: (x >= part * w) | (rng.random(len(x)) < 0.5))
+    return cases.S.finish_case(mdl, m, sheet=(-3.3, w - 10.0, 19.1), name="fronts")
 def launches():
     return [l.split() for l in hh.hh_launches().decode().splitlines()]
 def fail(name, n=1):
@@ -189,3 +204,43 @@ for noalloc in (False, True):
     run, noalloc = [eval(l) for l in out.splitlines()]
     assert int(run[0]) == groups and int(run[0]) * int(run[1]) >= nrecv
     assert int(noalloc[0]) * int(noalloc[1]) >= nrecv > (int(noalloc[0]) - 1) * int(noalloc[1])
+
+
+# 256 compute units: patches above 196,608 nodes
+@pytest.mark.parametrize("case,tuning,want", [
+    ("layer(443, 440)", (256, 1, 0, 1), dict(B=256, threads=256, patches=0)),       # 195,804 nodes
+    ("layer(443, 440)", (64, 1, 0, 1), dict(B=64, threads=64, patches=0)),
+    ("layer(450, 440)", (256, 1, 0, 1), dict(B=64, threads=256, patches=3134)),     # 198,891
+    ("layer(450, 440)", (32, 1, 0, 1), dict(B=32, threads=256, patches=3134)),
+    ("fronts(400, 200, 0.5)", (256, 1, 0, 1), dict(B=128, threads=256)),            # hanging nodes in half of it
+    ("fronts(400, 200, 0.5)", (64, 1, 0, 1), dict(B=64, threads=128)),
+    ("fronts(400, 200, 0.05)", (512, 1, 0, 1), dict(B=64, threads=256)),            # in a twentieth
+    ("cases.c2()", (512, 1, 0, 1), dict(B=512, patches=0)),
+])
+def test_one_step_layouts(host_hip, case, tuning, want):
+    _, layouts = host_hip(f"""
+s = lib.Solver({case})
+s.set_tuning(300, 1, 0, 2)
+s.set_tuning(*{tuning})
+""")
+    got = layouts[-1]
+    assert got["K"] == 1
+    assert {k: got[k] for k in want} == want
+    if "patches" not in want:
+        assert got["patches"] > 100
+
+
+def test_one_step_shapes_that_do_not_fit(host_hip):
+    """Tiles of a small mesh are as large as asked for, and refused where they
+    do not fit, leaving the shape before in place."""
+    host_hip("""
+s = lib.Solver(cases.c2())
+t = s.tuning()
+try:
+    s.set_tuning(800, 1, 0, 1)
+    raise SystemExit("not refused")
+except lib.DmpError as e:
+    assert e.code == -4
+assert s.tuning() == t
+s.run(9)
+""")
