@@ -97,12 +97,25 @@ constexpr int kRecvOne = 896;
 // Steps per launch of a mesh that one workgroup holds whole (build_tiles).
 constexpr int kWholeSteps = 32;
 
-// Several steps per launch: lanes of a workgroup of which a compute unit's
-// registers hold two (16 wavefronts of 128), and what share of the tiles may be
+// Several steps per launch: wavefronts that a compute unit's registers hold
+// (of 128 each), lanes of a workgroup of which it holds two, and what share of the tiles may be
 // halved to stay below, how often.
-constexpr int kPairThreads = 512;
+constexpr int kCuWaves = 16;
+constexpr int kPairThreads = 64 * kCuWaves / 2;
 constexpr int kWideShare = 4;
 constexpr int kHalvings = 3;
+
+// Block patches make every workgroup of a layout as wide as they are (384 lanes
+// at two steps per launch), so that fewer small tiles are in flight.  Where they
+// hold less than kPatchShare of the nodes, or among tiles of up to kPatchSmall,
+// plain tiles are taken if the chip would need more than a tenth of a further
+// round of the workgroups with patches, or kPatchRounds times as many.  Of 532 layouts (22,000 to 589,000
+// nodes, hanging nodes in 0 to 100 % of the mesh, tiles of 64 to 256, 2 to 4
+// steps) patches so take 0.44 to 1.12 of the plain tiles' time; always, up to 1.45
+// (canyon quadtree, 11 % of the nodes in patches, 64 per tile, 2 steps: 748
+// against 573 us for 120 steps).
+constexpr double kPatchShare = 0.6, kPatchRounds = 1.45;
+constexpr int kPatchSmall = 64;
 
 // State downloads: nodes per chunk (2 MiB) and chunks of pinned staging, and
 // the bytes to write that are worth one more host thread (starting one takes
@@ -331,6 +344,8 @@ struct Runtime {
     int tiles_block = 0, tiles_depth = 0;   // shape the tile arrays were built for
     bool no_whole = false;         // the mesh does not fit in one tile after all
     bool no_patches = false;       // the tiles between patches do not fit
+    bool measuring = false;        // building plain tiles for their rounds only
+    double plain_rounds = -1;      // rounds of workgroups that the chip needs with plain tiles; negative: not asked
     bool whole = false;            // one tile holds the mesh: no rings, up to V.depth steps per launch
     int state_depth = kMaxDepth;   // depth whose state_slot() the state buffers are in
     std::vector<void*> tile_allocs;
@@ -1272,8 +1287,12 @@ PatchRuns find_patches(const PackedHost& H, int NA, const std::vector<char>& tak
 }
 
 // build_tiles with the tiles that hold the nodes `halves` ended before them.
-// False, with more such nodes: to be built again (at most kHalvings times).
-bool try_tiles(Runtime& R, std::vector<int>& halves, int pass)
+// kHalve, with more such nodes: to be built again (at most kHalvings times);
+// kMeasure: whether patches pay depends on the rounds of plain tiles, kMeasured:
+// those are known; kPlain: to be built without patches.
+enum class Built { kDone, kHalve, kMeasure, kMeasured, kPlain };
+
+Built try_tiles(Runtime& R, std::vector<int>& halves, int pass)
 {
     PhaseTimer pt("tiles");
     const PackedHost& H = R.host;
@@ -1332,6 +1351,8 @@ bool try_tiles(Runtime& R, std::vector<int>& halves, int pass)
         }
         if (K > 1) {
             if (!R.no_patches) patches = find_patches(H, NA, taken, kBlockPatch, K);
+            const size_t held = patches.start.size() * kBlockPatchNodes;
+            if (held && R.plain_rounds < 0 && (held < kPatchShare * NA || B <= kPatchSmall)) return Built::kMeasure;
         } else if (R.no_patches || NA <= (long)kPlainNodes * ncu) {
             cells.rest.resize(NA);
             std::iota(cells.rest.begin(), cells.rest.end(), 0);
@@ -1720,7 +1741,7 @@ bool try_tiles(Runtime& R, std::vector<int>& halves, int pass)
         if (!wide.empty() && (long)wide.size() * kWideShare <= ntiles) {
             halves.insert(halves.end(), wide.begin(), wide.end());
             std::sort(halves.begin(), halves.end());
-            return false;
+            return Built::kHalve;
         }
     }
     std::vector<TileInfo> tiles;
@@ -1999,6 +2020,17 @@ bool try_tiles(Runtime& R, std::vector<int>& halves, int pass)
         V.threads = std::max(V.threads, (w * w + 63) / 64 * 64);
         if (V.threads > kMaxThreads) throw fail(DMP_EUNSUPPORTED, "patches need %d threads (max %d)", V.threads, kMaxThreads);
     }
+    if (K > 1 && R.plain_rounds >= 0) {
+        const size_t lds = std::max<size_t>(step_lds_bytes(V, R.precision), 1);
+        const size_t held = std::min<size_t>(64 * kCuWaves / V.threads, R.lds_limit / lds);
+        const double rounds = held ? (double)(ntiles + V.patches) / (held * ncu) : HUGE_VAL;
+        if (R.measuring) {
+            R.plain_rounds = rounds;
+            return Built::kMeasured;
+        }
+        if (V.patches && (rounds > std::ceil(R.plain_rounds) + 0.1 || rounds > kPatchRounds * R.plain_rounds))
+            return Built::kPlain;
+    }
     if (K == 1 && V.patches && !many_rest) V.threads = std::max(V.threads, 64 * kPatchWaves);
     const int per_block = K == 1 ? V.threads / 64 : 1;
     V.patch_blocks = (V.patches + per_block - 1) / per_block;
@@ -2207,13 +2239,31 @@ bool try_tiles(Runtime& R, std::vector<int>& halves, int pass)
     R.state_depth = K;
     R.tiles_block = R.tuning[0];
     R.tiles_depth = K;
-    return true;
+    return Built::kDone;
 }
 
 void build_tiles(Runtime& R)
 {
     std::vector<int> halves;
-    for (int pass = 0; !try_tiles(R, halves, pass); ++pass) {}
+    const bool may_patch = !R.no_patches;
+    R.measuring = false;
+    R.plain_rounds = -1;
+    for (int pass = 0;; ++pass) {
+        Built b = Built::kMeasured;
+        try {
+            b = try_tiles(R, halves, pass);
+        } catch (const Error& e) {
+            if (!R.measuring || e.code != DMP_EUNSUPPORTED) throw;
+            R.plain_rounds = HUGE_VAL;   // no plain tiles of this shape
+        }
+        if (b == Built::kDone) return;
+        if (b == Built::kHalve) continue;
+        R.measuring = b == Built::kMeasure;
+        if (R.measuring) R.plain_rounds = 0;
+        R.no_patches = !may_patch || b != Built::kMeasured;
+        halves.clear();
+        pass = -1;
+    }
 }
 
 void prepare_graph(Runtime& R);

@@ -134,3 +134,36 @@ def test_patches_of_small_instances(prec):
             for a, x in zip(b.state(q), w[1:]):
                 assert np.array_equal(a, x)
         b.close()
+
+
+# block patches with 2 to 8 rings (test_host_runtime.py holds that they are there)
+BLOCK_SHAPES = ((128, 0, 0, 2), (192, 1, 12, 3), (128, 1, 0, 4), (96, 1, 0, 5), (64, 1, 0, 6), (48, 1, 0, 8))
+
+
+@pytest.mark.parametrize("name", ["layer", "layer_het", "basin"])
+@pytest.mark.parametrize("prec", [0, 1])
+def test_block_patch_layouts(name, prec):
+    from damian_hip import cases, lib
+    import oracle_ctypes as O
+    if name == "basin":
+        case = cases.c4_valley(200.0, "SV", 10.0)
+    else:
+        case = layer(cases, 300, 200, sheet=(-3.3, 1490.0, 19.1))
+        case = cases.perturbed(case, seed=5) if name == "layer_het" else case
+    shapes = []
+    probe = lib.Solver(case, precision=prec)
+    for t in BLOCK_SHAPES:
+        try:
+            probe.set_tuning(*t)
+            shapes.append(t)
+        except lib.DmpError as e:   # hanging nodes widen the rings of deep launches
+            assert name == "basin" and t[3] > 4 and e.code == -4
+    probe.close()
+    assert len(shapes) >= 3
+    n = 300 if name == "basin" else 60   # the pulse is in the box
+    want = same_bits(cases, lib, case, prec, tuple(shapes), n, first=(256, 1, 0, 1))
+    assert np.abs(want[1]).max() > 1e-3
+    if name != "layer":
+        u_o, up_o, _, _ = O.run(case, nsteps=n, recv_interval=1, threads=8)
+        for a, b in ((want[1], u_o), (want[2], up_o)):
+            assert rel_l2(a, b) <= TOL[prec]

@@ -244,3 +244,44 @@ except lib.DmpError as e:
 assert s.tuning() == t
 s.run(9)
 """)
+
+
+# few patches among small tiles, which they would widen; most of the mesh in
+# them; half of it, where plain tiles would need as many rounds or more
+@pytest.mark.parametrize("case,tuning,patched", [
+    ("cases.c2()", (64, 1, 0, 2), False),
+    ("cases.c2()", (64, 1, 0, 3), False),
+    ("cases.c2()", (64, 1, 0, 4), True),
+    ("layer(300, 200)", (64, 1, 0, 2), False),
+    ("layer(300, 200)", (128, 1, 0, 2), True),
+    ("layer(300, 200)", (48, 1, 0, 8), True),
+    ("fronts(200, 100, 0.4)", (64, 1, 0, 2), False),
+    ("fronts(200, 100, 0.4)", (64, 1, 0, 3), True),
+])
+def test_block_patches_where_they_pay(host_hip, case, tuning, patched):
+    _, layouts = host_hip(f"""
+s = lib.Solver({case})
+s.set_tuning(300, 1, 0, 1)
+s.set_tuning(*{tuning})
+""")
+    assert (layouts[-1]["B"], layouts[-1]["K"]) == (tuning[0], tuning[3])
+    assert (layouts[-1]["patches"] > 0) == patched
+
+
+# the shapes of test_gpu_layouts.py
+@pytest.mark.parametrize("case", ["layer(300, 200)", "cases.c4_valley(200.0, 'SV', 10.0)"])
+def test_block_patch_shapes_of_the_gpu_tests(host_hip, case):
+    from test_gpu_layouts import BLOCK_SHAPES
+    _, layouts = host_hip(f"""
+s = lib.Solver({case})
+s.set_tuning(300, 1, 0, 1)
+for t in {BLOCK_SHAPES}:
+    try:
+        s.set_tuning(*t)
+    except lib.DmpError as e:
+        assert e.code == -4 and t[3] > 4
+        s.set_tuning(300, 1, 0, 1)
+""")
+    built = {(l["B"], l["K"]): l for l in layouts if l["K"] > 1}
+    assert {k for _, k in built} >= {2, 3, 4}
+    assert all(built[b, k]["patches"] > 0 for b, k in built if (b, k) in {(t[0], t[3]) for t in BLOCK_SHAPES})
