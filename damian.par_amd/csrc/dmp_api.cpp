@@ -23,6 +23,7 @@
 #include <functional>
 #include <memory>
 #include <numeric>
+#include <set>
 #include <string>
 #include <system_error>
 #include <thread>
@@ -344,6 +345,7 @@ struct Runtime {
     int tiles_block = 0, tiles_depth = 0;   // shape the tile arrays were built for
     bool no_whole = false;         // the mesh does not fit in one tile after all
     bool no_patches = false;       // the tiles between patches do not fit
+    int one_block = kMaxBlock;     // at one step per launch: nodes per tile at most (fewer between patches)
     bool measuring = false;        // building plain tiles for their rounds only
     double plain_rounds = -1;      // rounds of workgroups that the chip needs with plain tiles; negative: not asked
     bool whole = false;            // one tile holds the mesh: no rings, up to V.depth steps per launch
@@ -1286,6 +1288,22 @@ PatchRuns find_patches(const PackedHost& H, int NA, const std::vector<char>& tak
     return out;
 }
 
+// A mesh that one workgroup holds needs no rings, so a launch of several
+// steps may take any number of them; what they read ahead (forces and free
+// field) shares the LDS.  Where the caller asks for several steps per
+// launch and tiles that small a mesh fits in, or for dmp_init's own shape
+// (also where the caller sets what dmp_get_tuning gave), such a mesh is one
+// tile: the two-material valley of 358 nodes
+// takes 1.79 us a step in FP32C so, 3.2 in two tiles at three steps per
+// launch and 2.3 at eight; the layer of 861 nodes 1.91 against 2.56 and 1.83
+// in FP64, 1.78 against 2.50 and 1.74 in FP32C, in half the launches.
+// Descriptors address no more slots.
+bool may_be_whole(const Runtime& R, int block, int depth)
+{
+    const bool init_shape = block == R.init_tuning[0] && depth == R.init_tuning[3];
+    return depth > 1 && R.V.na <= kMaxSlots && (block >= R.V.na || init_shape);
+}
+
 // build_tiles with the tiles that hold the nodes `halves` ended before them.
 // kHalve, with more such nodes: to be built again (at most kHalvings times);
 // kMeasure: whether patches pay depends on the rounds of plain tiles, kMeasured:
@@ -1303,18 +1321,7 @@ Built try_tiles(Runtime& R, std::vector<int>& halves, int pass)
     R.tiles_depth = 0;
     const int NA = V.na, NV = V.nv;
     const int K = R.tuning[3];
-    // A mesh that one workgroup holds needs no rings, so a launch of several
-    // steps may take any number of them; what they read ahead (forces and free
-    // field) shares the LDS.  Where the caller asks for several steps per
-    // launch and tiles that small a mesh fits in, or for dmp_init's own shape
-    // (also where the caller sets what dmp_get_tuning gave), such a mesh is one
-    // tile: the two-material valley of 358 nodes
-    // takes 1.79 us a step in FP32C so, 3.2 in two tiles at three steps per
-    // launch and 2.3 at eight; the layer of 861 nodes 1.91 against 2.56 and 1.83
-    // in FP64, 1.78 against 2.50 and 1.74 in FP32C, in half the launches.
-    // Descriptors address no more slots.
-    const bool init_shape = R.tuning[0] == R.init_tuning[0] && K == R.init_tuning[3];
-    R.whole = K > 1 && NA <= kMaxSlots && (R.tuning[0] >= NA || init_shape) && !R.no_whole;
+    R.whole = may_be_whole(R, R.tuning[0], K) && !R.no_whole;
     int B = R.whole ? std::max(NA, 1) : R.tuning[0];
     int ntiles = (NA + B - 1) / B;
     const int NR = (int)H.recv.size();
@@ -1349,6 +1356,7 @@ Built try_tiles(Runtime& R, std::vector<int>& halves, int pass)
             const int c = x.c[0];
             if (c >= 0) taken[c < NA ? c : H.vanch[c - NA].x] = 1;
         }
+        if (K == 1) R.one_block = kMaxBlock;
         if (K > 1) {
             if (!R.no_patches) patches = find_patches(H, NA, taken, kBlockPatch, K);
             const size_t held = patches.start.size() * kBlockPatchNodes;
@@ -1359,7 +1367,8 @@ Built try_tiles(Runtime& R, std::vector<int>& halves, int pass)
         } else {
             cells = find_cells(H, NA, taken);
             many_rest = cells.rest.size() * kManyRest > (size_t)NA;
-            if (!cells.patch.empty()) B = std::min(B, many_rest ? kManyRestBlock : kRestBlock);
+            if (!cells.patch.empty()) R.one_block = many_rest ? kManyRestBlock : kRestBlock;
+            B = std::min(B, R.one_block);
         }
         for (size_t i = 0; i < cells.rest.size(); ++i) gen_of[cells.rest[i]] = (int)i;
     }
@@ -3276,21 +3285,36 @@ void autotune(Runtime& R, int nsteps, int* out)
         if (R.V.na > 6 * 256 * ncu) cand_depth = {1, 2};
         else if (R.V.na > 2 * 256 * ncu) cand_depth = {1, 2, 3, 4};
     }
+    // Shapes that give a layout already timed are left out: larger tiles than
+    // there are between patches, and any that hold the mesh in one tile.
+    std::set<std::array<int, 2>> timed;
+    bool whole = false;
+    auto layout_of = [&](int b, int K) {
+        if (K == 1) return std::array<int, 2>{std::min(b, R.one_block), 1};
+        return whole && may_be_whole(R, b, K) ? std::array<int, 2>{0, 0} : std::array<int, 2>{b, K};
+    };
     for (int b : cand_block)
         for (int K : cand_depth) {
+            if (timed.count(layout_of(b, K))) continue;
+            const int shape[4] = {b, 0, 0, K};
+            std::copy(shape, shape + 4, R.tuning);
+            try {
+                R.apply_tuning();
+            } catch (const Error& e) {
+                if (e.code != DMP_EUNSUPPORTED) throw;
+                continue;   // shape the layout cannot use
+            }
+            whole |= R.whole;
+            if (!timed.insert(layout_of(b, K)).second) continue;
+            const bool one_group = R.V.node_tiles + R.V.patch_blocks <= 1;
             const int cand_graph[2] = {0, std::max(K, (std::min(nsteps, 60) / K) * K)};
             for (int x = 0; x <= 1; ++x)
                 for (int g : cand_graph) {
-                    R.tuning[0] = b;
                     R.tuning[1] = x;
                     R.tuning[2] = g;
-                    R.tuning[3] = K;
-                    try {
-                        R.apply_tuning();
-                    } catch (const Error& e) {
-                        if (e.code != DMP_EUNSUPPORTED) throw;
-                        continue;   // shape the layout cannot use
-                    }
+                    // (the launches of another variant)
+                    if ((x && one_group) || (g && graph_length(R) == 0)) continue;
+                    R.apply_tuning();
                     // a warm-up, then timed runs from the saved state until
                     // there are two and 2 ms of them (at most 15: short
                     // calls vary by a few percent from run to run, more than

@@ -160,6 +160,20 @@ assert {{tuple(l) for l in launches() if "step_kernel" in l[0]}} == kernels
 """)
 
 
+# one tile for many shapes; tiles between patches, which are no larger than 64
+# or 128 nodes; neither
+@pytest.mark.parametrize("case", ["cases.f1()", "cases.f2()", "layer(450, 440)", "fronts(400, 200, 0.5)", "cases.c1()"])
+def test_autotune_builds_no_layout_twice(host_hip, case):
+    _, layouts = host_hip(f"""
+s = lib.Solver({case})
+s.set_tuning(33, 1, 0, 2)
+s.autotune(4)
+""")
+    searched = [tuple(sorted((k, v) for k, v in l.items() if k != "K" or not l["whole"])) for l in layouts[2:]]
+    assert len(searched) > 8
+    assert len(set(searched[:-1])) == len(searched) - 1   # the last is the one found, built again
+
+
 def test_state_download_without_threads(host_hip):
     """Host threads only speed a large download up: where none can be started
     (no address space for a stack) the call still moves every byte."""
