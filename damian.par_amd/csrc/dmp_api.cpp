@@ -2877,6 +2877,7 @@ hipEvent_t take_event(Runtime& R)
 int run_steps(Runtime& R, int n, double* out)
 {
     if (n < 0) throw fail(DMP_EINVAL, "negative step count");
+    if (!R.tiles_block) R.apply_tuning();   // the last shape asked for and the one before could not be built
     DevView& V = R.V;
     const int s = R.step;
     const int I = V.recv_interval;
@@ -3004,6 +3005,7 @@ int run_steps(Runtime& R, int n, double* out)
 int run_steps_noalloc(Runtime& R, int n, double* out)
 {
     if (n < 0) throw fail(DMP_EINVAL, "negative step count");
+    if (!R.tiles_block) throw fail(DMP_ESTATE, "no launch shape is in place: the last one could not be built");
     DevView V = R.V;   // the view with the scratch in place of the ring
     const int s = R.step;
     const int I = V.recv_interval;

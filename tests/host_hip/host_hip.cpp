@@ -1,7 +1,8 @@
 // A HIP runtime without a device, for tests of the library's host code: device
 // memory is host memory, kernels are noted and not run, every event is complete
 // when it is recorded and events lie 1 ms apart for each kernel between them.
-// hh_fail(name, n) makes the n-th call from now of that function fail.
+// hh_fail(name, n, times) makes the n-th call from now of that function fail, and
+// as many in all as `times` says.
 #include <hip/hip_runtime.h>
 
 #include <cstdlib>
@@ -13,15 +14,15 @@ namespace {
 
 std::map<const void*, std::string> names;   // kernels by the address they are launched by
 std::string launches, hostmallocs;
-std::map<std::string, int> failing;
+std::map<std::string, std::pair<int, int>> failing;   // calls until the first that fails, calls that fail
 float clock_ms = 0;
 int allocs = 0;
 
 hipError_t status(const char* name)
 {
     auto f = failing.find(name);
-    if (f == failing.end() || --f->second > 0) return hipSuccess;
-    failing.erase(f);
+    if (f == failing.end() || --f->second.first > 0) return hipSuccess;
+    if (--f->second.second <= 0) failing.erase(f);
     return hipErrorUnknown;
 }
 
@@ -45,7 +46,7 @@ const char* hh_launches()
 }
 // "bytes flags" of each hipHostMalloc
 const char* hh_hostmallocs() { return hostmallocs.c_str(); }
-void hh_fail(const char* name, int n) { failing[name] = n; }
+void hh_fail(const char* name, int n, int times) { failing[name] = {n, times}; }
 int hh_allocs() { return allocs; }
 
 void** __hipRegisterFatBinary(const void*)

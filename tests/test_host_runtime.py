@@ -33,8 +33,8 @@ def fronts(nx, nz, part, seed=7):
     return cases.S.finish_case(mdl, m, sheet=(-3.3, w - 10.0, 19.1), name="fronts")
 def launches():
     return [l.split() for l in hh.hh_launches().decode().splitlines()]
-def fail(name, n=1):
-    hh.hh_fail(name.encode(), n)
+def fail(name, n=1, times=1):
+    hh.hh_fail(name.encode(), n, times)
 """
 
 
@@ -158,6 +158,35 @@ out = s.run(6)
 assert out.shape[0] == 6
 assert {{tuple(l) for l in launches() if "step_kernel" in l[0]}} == kernels
 """)
+
+
+def test_no_launch_without_a_layout(host_hip):
+    """Memory that runs out while a shape is built, and again while the one
+    before is, leaves no layout: a run call builds it or fails, and launches
+    nothing until it is there."""
+    _, layouts = host_hip("""
+s = lib.Solver(cases.c1())
+s.set_tuning(128, 1, 0, 3)
+want = s.tuning()
+def refused(call, code):
+    launches()
+    try:
+        call()
+        raise SystemExit("not refused")
+    except lib.DmpError as e:
+        assert e.code == code, e
+    assert not launches()
+fail("hipMalloc", 5, 1000)
+refused(lambda: s.set_tuning(64, 1, 0, 2), -2)
+assert s.tuning() == want
+refused(lambda: s.run(6), -2)
+fail("hipMalloc", 10**9)
+refused(lambda: s.run(6, noalloc=True), -5)
+assert s.run(6).shape[0] == 7
+assert s.run(6, noalloc=True).shape[0] == 6
+s.close()
+""")
+    assert (layouts[-1]["B"], layouts[-1]["K"]) == (128, 3)
 
 
 # one tile for many shapes; tiles between patches, which are no larger than 64
