@@ -2117,9 +2117,9 @@ Built try_tiles(Runtime& R, std::vector<int>& halves, int pass)
         ring = (double)ring_gid.size();
         int elem_tiles = 0;
         for (const TileInfo& T : tiles) elem_tiles += T.mat_mode;
-        std::fprintf(stderr, "layout B=%d K=%d whole=%d depth=%d tiles=%d threads=%d mean_ent=%.1f ring/core=%.3f lds=%zu "
+        std::fprintf(stderr, "layout B=%d K=%d whole=%d depth=%d tiles=%d halved=%zu threads=%d mean_ent=%.1f ring/core=%.3f lds=%zu "
                      "slots=%d vrows=%d virt=%d force=%d side=%d recv=%d elem_tiles=%d hist=",
-                     B, K, R.whole, V.depth, ntiles, V.threads, ent / std::max(ntiles, 1), ring / std::max(NA, 1), lds,
+                     B, K, R.whole, V.depth, ntiles, halves.size(), V.threads, ent / std::max(ntiles, 1), ring / std::max(NA, 1), lds,
                      V.lds_slots, V.lds_vrows, V.lds_virt, V.lds_force, V.lds_side,
                      V.lds_recv, elem_tiles);
         for (int h : hist) std::fprintf(stderr, "%d,", h);

@@ -328,3 +328,23 @@ for t in {BLOCK_SHAPES}:
     built = {(l["B"], l["K"]): l for l in layouts if l["K"] > 1}
     assert {k for _, k in built} >= {2, 3, 4}
     assert all(built[b, k]["patches"] > 0 for b, k in built if (b, k) in {(t[0], t[3]) for t in BLOCK_SHAPES})
+
+
+# the shapes that test_gpu_patches.py::test_halved_tiles does not leave out
+@pytest.mark.parametrize("case,built,halved", [
+    ("cases.c4_valley(200.0, 'SV', 10.0)", [256, 200, 170, 140], [256, 200, 170]),
+    ("cases.c2()", [256, 170, 140], [170]),
+])
+def test_halved_tiles_of_the_gpu_tests(host_hip, case, built, halved):
+    out, layouts = host_hip(f"""
+s = lib.Solver({case})
+for t in ((256, 1, 0, 3), (200, 1, 0, 4), (170, 0, 12, 4), (140, 1, 0, 4)):
+    s.set_tuning(300, 1, 0, 1)
+    try:
+        s.set_tuning(*t)
+        print(t[0])
+    except lib.DmpError as e:
+        assert e.code == -4
+""")
+    assert [int(b) for b in out.split()] == built
+    assert sorted({int(l["B"]) for l in layouts if l["K"] > 1 and l["halved"]}, reverse=True) == halved
