@@ -162,8 +162,16 @@ def measure(lib, case, warmup, steps, tuning, label, accuracy_steps=None):
                      "device_ms_per_step": dev_ms / steps,
                      "bytes_per_step": B,
                      "achieved_GBs": achieved, "frac": achieved / HBM_PEAK_GBS}
+        # bytes_per_step is a model: patches move less than it charges, and so
+        # do launches of several steps
+        moved = measured_traffic(label, name, tuning)
+        traffic = "traffic not measured at this shape"
+        if moved is not None:
+            rate = moved / tuning[3] / per_launch_s / 1e9
+            out[name].update(traffic_per_step=moved / tuning[3], traffic_GBs=rate, traffic_frac=rate / HBM_PEAK_GBS)
+            traffic = f"measured traffic {rate:.0f} GB/s"
         print(f"# {label} {name}: {out[name]['element_steps_per_s']:.3e} element-steps/s, "
-              f"{out[name]['device_ms_per_step'] * 1e3:.2f} us/step, {achieved:.0f} GB/s",
+              f"{out[name]['device_ms_per_step'] * 1e3:.2f} us/step, algorithmic {achieved:.0f} GB/s, {traffic}",
               file=sys.stderr, flush=True)
     if accuracy_steps is None:
         out["accuracy_fp32c_vs_fp64"] = accuracy(recs["fp32c"], recs["fp64"], case.dt)
