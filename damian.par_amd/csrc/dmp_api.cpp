@@ -80,10 +80,10 @@ constexpr int kRestBlock = 64;
 constexpr int kPatchWaves = 4;
 // Where more than one node in kManyRest is outside patches (hanging nodes all
 // over the mesh) the tiles are the work: larger ones read fewer ring nodes, and
-// the workgroup is no wider than they need.  470,000 to 670,000 nodes, shares of 9, 15, 26 and
-// 54 %, FP32C, tiles of 64 in four wavefronts against 128: 10.6 and 10.4,
-// 11.6 and 10.6, 14.9 and 11.5, 19.7 and 15.6 us a step (plain tiles of 256:
-// 21.8, 23.4, 23.6 and 21.4); no patches at all 24.0 and 17.2 (17.8).
+// the workgroup is no wider than they need.  470,000 to 670,000 nodes, shares
+// of 9, 15, 26 and 54 %, FP32C, tiles of 64 in four wavefronts against 128: 10.6
+// and 10.4, 11.6 and 10.6, 14.9 and 11.5, 19.7 and 15.6 us a step (plain tiles
+// of 256: 21.8, 23.4, 23.6 and 21.4); no patches at all 24.0 and 17.2 (17.8).
 constexpr int kManyRest = 8;
 constexpr int kManyRestBlock = 128;
 
@@ -99,8 +99,8 @@ constexpr int kRecvOne = 896;
 constexpr int kWholeSteps = 32;
 
 // Several steps per launch: wavefronts that a compute unit's registers hold
-// (of 128 each), lanes of a workgroup of which it holds two, and what share of the tiles may be
-// halved to stay below, how often.
+// (of 128 each), lanes of a workgroup of which it holds two, and what share of
+// the tiles may be halved to stay below, how often.
 constexpr int kCuWaves = 16;
 constexpr int kPairThreads = 64 * kCuWaves / 2;
 constexpr int kWideShare = 4;
@@ -110,11 +110,11 @@ constexpr int kHalvings = 3;
 // at two steps per launch), so that fewer small tiles are in flight.  Where they
 // hold less than kPatchShare of the nodes, or among tiles of up to kPatchSmall,
 // plain tiles are taken if the chip would need more than a tenth of a further
-// round of the workgroups with patches, or kPatchRounds times as many.  Of 532 layouts (22,000 to 589,000
-// nodes, hanging nodes in 0 to 100 % of the mesh, tiles of 64 to 256, 2 to 4
-// steps) patches so take 0.44 to 1.12 of the plain tiles' time; always, up to 1.45
-// (canyon quadtree, 11 % of the nodes in patches, 64 per tile, 2 steps: 748
-// against 573 us for 120 steps).
+// round of the workgroups with patches, or kPatchRounds times as many.  Of 532
+// layouts (22,000 to 589,000 nodes, hanging nodes in 0 to 100 % of the mesh,
+// tiles of 64 to 256, 2 to 4 steps) patches so take 0.44 to 1.12 of the plain
+// tiles' time; always, up to 1.45 (canyon quadtree, 11 % of the nodes in
+// patches, 64 per tile, 2 steps: 748 against 573 us for 120 steps).
 constexpr double kPatchShare = 0.6, kPatchRounds = 1.45;
 constexpr int kPatchSmall = 64;
 
@@ -1341,9 +1341,9 @@ Built try_tiles(Runtime& R, std::vector<int>& halves, int pass)
     if (hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, R.device) != hipSuccess || ncu < 1)
         ncu = 256;
     // Uniform parts of the mesh as patches: at one step per launch in meshes of
-    // more than kPlainNodes per compute unit; at
-    // several where there are more tiles than compute units, so that work in
-    // flight and not the slowest tile's latency bounds a launch.
+    // more than kPlainNodes per compute unit; at several where there are more
+    // tiles than compute units, so that work in flight and not the slowest
+    // tile's latency bounds a launch.
     // One step per launch: tiles of B nodes each of the list of nodes outside
     // patches.
     PatchRuns patches;
@@ -2733,7 +2733,11 @@ void build_runtime(Runtime& R, const std::vector<Instance*>& insts)
     HIPCHECK(hipDeviceSynchronize());
     // default shape: several steps per launch where launches dominate (small
     // meshes), one where HBM does (large ones); fewer steps or smaller tiles
-    // where a tile of the default shape does not fit
+    // where a tile of the default shape does not fit.  Between, the best depth
+    // depends on the mesh: six basins of 326,000 nodes together take 8.5 us a
+    // step at one step per launch, 8.6 (FP32C, 128 nodes per tile, 4 steps) to
+    // 14.0 at two to four; single basins of 237,000 and 317,000 nodes are faster
+    // at three and four (autotune below, which finds those)
     const bool small = NA < 200000;
     const int shapes[][2] = {{256, small ? 3 : 1}, {256, 2}, {128, 3}, {128, 2}, {256, 1}, {128, 1}, {64, 1}};
     bool ok = false;

@@ -27,7 +27,7 @@ namespace dmp {
 constexpr int kMinBlock = 32;       // core nodes per tile
 constexpr int kMaxBlock = 1024;
 constexpr int kMaxThreads = 1024;   // threads per workgroup
-constexpr int kMaxDepth = 8;       // steps per launch
+constexpr int kMaxDepth = 8;       // steps per launch, of layouts with rings (one-tile layouts: kWholeSteps)
 // u_j lives in U[j mod n], n = state_slots(depth).  A launch of k <= depth
 // steps from t0 reads u_{t0} and u_{t0-1} (any workgroup, at any time during
 // the launch) and writes u_{t0+k} and, for k > 1, u_{t0+k-1}: distinct buffers
@@ -37,7 +37,9 @@ constexpr int kMaxDepth = 8;       // steps per launch
 // first (2.47M-element sweep, 40 MB a buffer: FP32C 28.7 us a step against 32.2
 // with ten, FP64 33.0 against 35.7).  Deeper layouts share one count, a
 // compile-time modulus in the kernel (choosing it by depth there costs the
-// canyon quadtree 0.7 %).
+// canyon quadtree 0.7 %).  A launch of a one-tile layout takes more steps and so
+// may write the buffers it read: its one workgroup has all of both levels in LDS
+// at its first barrier and stores behind that.
 constexpr int kStateSlots = 10;
 __host__ __device__ constexpr int state_slots(int depth) { return depth == 1 ? 3 : kStateSlots; }
 constexpr bool state_slots_suffice()
@@ -278,7 +280,7 @@ struct DevView {
     int na, nv, ne;
     int nrecv;
     int threads;         // threads per workgroup (one LDS entry each)
-    int depth;           // rings per tile = most steps one launch may take
+    int depth;           // most steps one launch may take: rings per tile, or up to kWholeSteps in one tile
     int node_tiles;
     int xcd_remap;       // 1: consecutive tiles stay on one XCD
     int tiles_per_xcd;

@@ -1271,7 +1271,8 @@ __device__ void tile_steps(const DevView& V, int tile, int t0, int k, int end)
 // layer 22.0 -> 19.4 us, 20-step calls of the canyon quadtree 83.4 -> 80.0.
 // Every wavefront waits for its own stores, one makes the release: a release
 // by each writes the same L2 back once per wavefront (19.9 -> 16.8 us and 73.1
-// -> 71.7).
+// -> 71.7, here of calls one after another through the Python binding, which
+// adds 1 us).
 __device__ __forceinline__ void report_done(const DevView& V, uint32_t call)
 {
     if (!call) return;
@@ -1288,7 +1289,7 @@ enum class Parts { kTiles, kPatches, kWhole };
 // samples the receivers at steps t0 .. t0 + k - 1 (and t0 + k when end is set,
 // which needs k < depth).  The one-step kernel is bandwidth-bound, so it is
 // compiled for as many waves per SIMD as its registers allow without spills
-// (FP32C 7 with 72 VGPRs; FP64 6); the deeper one is latency-bound and keeps
+// (FP32C 7 with 68 VGPRs; FP64 6 with 78); the deeper one is latency-bound and keeps
 // the registers a 1024-thread workgroup leaves (4 waves per SIMD).
 template <class P, bool ONE, bool HANG, Parts PARTS>
 __global__ __launch_bounds__(kMaxThreads) __attribute__((amdgpu_waves_per_eu(ONE ? P::kOneWaves : 4)))
