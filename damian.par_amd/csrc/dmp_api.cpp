@@ -345,6 +345,7 @@ struct Runtime {
     int tiles_block = 0, tiles_depth = 0;   // shape the tile arrays were built for
     bool no_whole = false;         // the mesh does not fit in one tile after all
     bool no_patches = false;       // the tiles between patches do not fit
+    bool small_tiles = false;      // at one step per launch: tiles as large as asked for do not fit
     int one_block = kMaxBlock;     // at one step per launch: nodes per tile at most (fewer between patches)
     bool measuring = false;        // building plain tiles for their rounds only
     double plain_rounds = -1;      // rounds of workgroups that the chip needs with plain tiles; negative: not asked
@@ -1361,13 +1362,13 @@ Built try_tiles(Runtime& R, std::vector<int>& halves, int pass)
             if (!R.no_patches) patches = find_patches(H, NA, taken, kBlockPatch, K);
             const size_t held = patches.start.size() * kBlockPatchNodes;
             if (held && R.plain_rounds < 0 && (held < kPatchShare * NA || B <= kPatchSmall)) return Built::kMeasure;
-        } else if (R.no_patches || NA <= (long)kPlainNodes * ncu) {
+        } else if (R.no_patches || (NA <= (long)kPlainNodes * ncu && !R.small_tiles)) {
             cells.rest.resize(NA);
             std::iota(cells.rest.begin(), cells.rest.end(), 0);
         } else {
             cells = find_cells(H, NA, taken);
             many_rest = cells.rest.size() * kManyRest > (size_t)NA;
-            if (!cells.patch.empty()) R.one_block = many_rest ? kManyRestBlock : kRestBlock;
+            if (!cells.patch.empty() || R.small_tiles) R.one_block = many_rest ? kManyRestBlock : kRestBlock;
             B = std::min(B, R.one_block);
         }
         for (size_t i = 0; i < cells.rest.size(); ++i) gen_of[cells.rest[i]] = (int)i;
@@ -2280,14 +2281,18 @@ void prepare_graph(Runtime& R);
 void Runtime::apply_tuning()
 {
     if (tiles_block != tuning[0] || tiles_depth != tuning[3]) {
-        no_whole = no_patches = false;
-        try {
-            build_tiles(*this);
-        } catch (const Error& e) {
-            // a shape that plain tiles can take is taken
-            if (e.code != DMP_EUNSUPPORTED) throw;
-            no_whole = no_patches = true;
-            build_tiles(*this);
+        // a shape that plain tiles can take is taken, at one step per launch
+        // also one that smaller tiles can
+        const int tries = tuning[3] == 1 ? 3 : 2;
+        for (int i = 0; i < tries; ++i) {
+            no_whole = no_patches = i == 1;
+            small_tiles = i == 2;
+            try {
+                build_tiles(*this);
+                break;
+            } catch (const Error& e) {
+                if (e.code != DMP_EUNSUPPORTED || i + 1 == tries) throw;
+            }
         }
     }
     apply_launch_shape();

@@ -164,9 +164,10 @@ int dmp_export_mesh(void *h, int *eptr, int *eind, bool *ediv, int *hanging, int
  * work, so tiles holding hanging-node anchors are smaller).  Uniform parts of
  * the mesh are cut out first, as patches of 8 x 8 nodes with one step per
  * launch and more than 768 nodes per compute unit (the tiles then hold at most
- * 64 of the nodes between, or 128 where these are more than an eighth) and of
- * 16 x 16 with several and more tiles than compute units.  tuning[1] = XCD-aware tile
- * remap (0/1), tuning[2] = steps per captured hipGraph (0 = eager launches),
+ * 64 of the nodes between, or 128 where these are more than an eighth; also in
+ * smaller meshes where tiles of tuning[0] nodes do not fit) and of 16 x 16 with
+ * several and more tiles than compute units.  tuning[1] = XCD-aware tile remap
+ * (0/1), tuning[2] = steps per captured hipGraph (0 = eager launches),
  * tuning[3] = time steps one launch advances (1..8; each tile then carries that
  * many rings of neighbours in LDS).  dmp_init starts from {256, 1, 60, 3}
  * ({256, 1, 60, 1} above 200,000 nodes), falling back to smaller shapes where

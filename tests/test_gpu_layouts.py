@@ -104,6 +104,15 @@ def test_one_step_layouts(name, prec):
 
 
 @pytest.mark.parametrize("prec", [0, 1])
+def test_one_step_tiles_that_do_not_fit(prec):
+    """Cut into patches and small tiles (of 64 and of 128 nodes) instead."""
+    from damian_hip import cases, lib
+    for case in (cases.c2(), fronts(cases, 60, 40, 1.0)):
+        want = same_bits(cases, lib, case, prec, ((1024, 1, 0, 1), (1024, 0, 12, 1)), 80)
+        assert np.abs(want[1]).max() > 0
+
+
+@pytest.mark.parametrize("prec", [0, 1])
 def test_patches_of_small_instances(prec):
     """A batch with patches (above the line as a whole) of meshes at whose sizes
     the patches' number and rings change: none, one, several in a row, cells cut

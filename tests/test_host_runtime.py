@@ -273,20 +273,20 @@ s.set_tuning(*{tuning})
         assert got["patches"] > 100
 
 
-def test_one_step_shapes_that_do_not_fit(host_hip):
-    """Tiles of a small mesh are as large as asked for, and refused where they
-    do not fit, leaving the shape before in place."""
-    host_hip("""
-s = lib.Solver(cases.c2())
-t = s.tuning()
-try:
-    s.set_tuning(800, 1, 0, 1)
-    raise SystemExit("not refused")
-except lib.DmpError as e:
-    assert e.code == -4
-assert s.tuning() == t
+# a mesh with uniform parts, one without
+@pytest.mark.parametrize("case", ["cases.c2()", "fronts(60, 40, 1.0)"])
+def test_one_step_tiles_that_do_not_fit(host_hip, case):
+    """Tiles of a small mesh are as large as asked for; where those do not fit,
+    the mesh is cut into patches and small tiles and the shape is taken."""
+    _, layouts = host_hip(f"""
+s = lib.Solver({case})
+s.set_tuning(512, 1, 0, 1)
+s.set_tuning(1024, 1, 0, 1)
+assert s.tuning() == (1024, 1, 0, 1)
 s.run(9)
 """)
+    assert [(l["B"], l["patches"] > 0) for l in layouts[-2:]] == [(512, False), (layouts[-1]["B"], case == "cases.c2()")]
+    assert layouts[-1]["B"] in (64, 128)
 
 
 # few patches among small tiles, which they would widen; most of the mesh in
